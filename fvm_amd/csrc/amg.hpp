@@ -56,6 +56,7 @@ struct Level {
     std::vector<long long> color_nnz;  // host: off-diagonal entries of each colour's rows
     DArr<int> d_color_ptr;             // the same on the device
     DArr<int> sell_off, sell_col;
+    std::vector<int> h_sell_off;       // host copy of sell_off on levels small enough for the packed tail
     int sell_total = 0;                // SELL-64 elements (padding included) = sell_off[nslices]
     DArr<double> sell_val, pdiag;
     DArr<int> pci, pc2f_row, pc2f_col;
@@ -147,7 +148,10 @@ struct fvm_amg {
     fvm::DArr<double> dense_inv;
     // tuning knobs (fvm_amg_set_tuning): rows below which a level runs in the
     // single-workgroup tail of the V-cycle / is coarsened by one workgroup
-    long long tail_max_rows = 40000;
+    // one workgroup beats the launches of a level up to here (ms per solve at 1,500 / 6,000 / 12,000 rows:
+    // 402k rows FP64 40.6 / 37.0 / 38.0, 8M rows mixed 239.7 / 237.1 / 233.3, 32 systems of ~30k rows
+    // 116.2 / 110.5 / 129.7)
+    long long tail_max_rows = 6000;
     int exact_wg_width = 256;          // runs of consecutive dependency levels of at most this many rows
                                        // sweep in one workgroup launch (no result changes)
     int reuse_setup = 0;               // opt-in: a setup of an unchanged matrix keeps the hierarchy
@@ -190,6 +194,11 @@ struct fvm_amg {
     int tail_lds = 1;                  // tail levels that fit sweep from LDS
     int tail_lds_lim = -1;             // LDS bytes per workgroup of the device (-1: not queried)
     std::vector<int> tail_lds_bytes[2];   // LDS bytes per level (FP64 / mixed descriptors)
+    // packed tail: first packed and first resident level, 16-byte words and bytes of the
+    // part in LDS, the image (its table first, its data at tail_o_img)
+    int tail_lp = 0, tail_lr = 0, tail_img16 = 0, tail_res_bytes = 0;
+    size_t tail_o_img = 0;
+    fvm::DArr<unsigned char> tail_img;
     fvm::DArr<unsigned char> tail_desc;
     // live timing of finest-level kernels with HIP events on the handle's stream
     bool ktime = false;

@@ -624,7 +624,8 @@ __global__ void k_dense_apply(int n, const double *inv, const int *perm, const i
 }
 
 // ------------------------------------------------------------------ single-workgroup tail
-// The small levels of a V-cycle in one launch: every step (restriction, a
+// The small levels of a V-cycle in one launch, in its general form (Jacobi, pre-sweeps,
+// levels that k_tail_gs cannot hold): every step (restriction, a
 // colour of a sweep, prolongation) is a loop of the workgroup over the rows of
 // one level, steps separated by workgroup barriers. Same arithmetic per row as
 // the per-level kernels; it only removes the launches.
@@ -820,6 +821,476 @@ k_tail(const TailLv *lv, int l0, int last, int npre, int npost, int jacobi, cons
         }
         __syncthreads();
         tail_sweeps_lds<V, D, X>(L, npost, jacobi, s_tail, lds_cap);
+    }
+}
+
+// ------------------------------------------------------------------ resident tail
+// The tail of a V-cycle without pre-sweeps and with Gauss-Seidel sweeps (the usual
+// cycle), one workgroup. What bounds it is not bandwidth but, per colour step, a chain
+// of dependent accesses and the instructions of a single wavefront (one instruction per
+// four clocks or more). So the tail has its own format, packed once per hierarchy:
+//  - items of up to 64 rows of one colour; a row's entries are padded to groups of four,
+//    so one 16-byte load brings four entries (mixed: a 16-bit column beside the BF16
+//    value in one word; FP64: two loads of values, one of four columns), and the rows'
+//    g-th groups lie side by side. A padding entry is -0 times a word that holds +0,
+//    which leaves every sum unchanged;
+//  - the smallest levels, from the coarsest up while they fit, are resident: copied to
+//    LDS in one round trip, their vectors live there. Larger ones keep x in LDS and
+//    stream their entries;
+//  - each wavefront loads its next item before it computes the present one. The barriers
+//    wait for LDS only, so those loads stay in flight across them;
+//  - levels whose colours have at most 64 rows are swept by one wavefront, without
+//    barriers (its LDS accesses stay in order).
+// The arithmetic per row and its order are those of the launched kernels: same bits.
+// Measured (levels 4,948 ... 2 of a 402,550-row FP64 hierarchy, one V-cycle): 179 us; the
+// general tail kernel below 6,000 rows takes about 940 us, the same levels launched
+// 400 us. A step of a resident level costs 0.4 to 0.8 us, about 130 to 250 instructions
+// of one wavefront plus five LDS round trips.
+constexpr int TAIL_NT = 512;                // eight wavefronts (a barrier of 4 / 8 / 16 costs 11 / 87 / 336 clocks)
+constexpr int TAIL_ROWS_CAP = 16384;        // largest level packed
+constexpr int TAIL_RES_BYTES = 104 * 1024;  // LDS of the item tables and the resident levels
+constexpr int TAIL_Q = 4;                   // groups of four entries loaded ahead
+
+template <class T>
+using GPtr = const T __attribute__((address_space(1))) *;   // a pointer read from memory, known to be global
+template <class T>
+using GMut = T __attribute__((address_space(1))) *;
+
+// a packed level: byte offsets in the image, of which the first bytes (this table too)
+// are copied to LDS: a table read from memory costs every level a round trip
+struct TailTab {
+    int n, ncolor, one_wave, resident;
+    int item, cptr;               // LDS: items (int2), first item of each colour (int)
+    int ent, val, diag;           // entries: uint32 (mixed) / columns uint16 and values (FP64); diagonal
+    int pci, c2r, c2c;            // resident: transfer to the level below, uint16 (pci 0xffff: none)
+    int perm, iperm;              // direct level
+    int b, x;                     // resident: vectors in LDS
+    const int *g_pci, *g_c2r, *g_c2c;   // the same in memory
+    void *g_b, *g_x;
+};
+// item: first row, row count and groups of four entries; first entry
+__device__ __forceinline__ int item_row(int2 t) { return t.x & 0xffff; }
+__device__ __forceinline__ int item_rows(int2 t) { return (t.x >> 16) & 0xff; }
+__device__ __forceinline__ int item_groups(int2 t) { return (int)((unsigned)t.x >> 24); }
+
+// Packs the items (one block of 64 threads per work[] entry {level, item}) and, for
+// item -1, the transfer maps of a resident level or the permutation of the direct one.
+template <class V, class D>
+__global__ void k_tail_pack(const TailLv *lv, const int2 *work, int lp, int last, int direct, unsigned char *img) {
+    const int l = work[blockIdx.x].x, it = work[blockIdx.x].y;
+    const TailLv &L = lv[l];
+    const TailTab T = ((const TailTab *)img)[l - lp];
+    auto put16 = [&](int off, const int *src, int m) {
+        uint16_t *d = (uint16_t *)(img + off);
+        for (int i = threadIdx.x; i < m; i += blockDim.x) d[i] = (uint16_t)src[i];
+    };
+    if (it < 0) {
+        if (l == last && direct) {
+            put16(T.perm, L.perm, L.n);
+            put16(T.iperm, L.iperm, L.n);
+        } else if (l < last) {
+            put16(T.pci, L.pci, L.n);
+            const int nc = lv[l + 1].n;
+            put16(T.c2r, L.c2f_row, nc + 1);
+            put16(T.c2c, L.c2f_col, L.c2f_row[nc]);
+        }
+        return;
+    }
+    const int2 t = ((const int2 *)(img + T.item))[it];
+    const int lane = threadIdx.x;
+    if (lane >= item_rows(t)) return;
+    const int p = item_row(t) + lane, w4 = item_groups(t) * 4;
+    const int s = p >> 6, o = L.soff[s] + (p & 63), w = (L.soff[s + 1] - L.soff[s]) >> 6;
+    const int np = item_rows(t);
+    for (int k = 0; k < w4; k++) {
+        const int c = k < w ? L.scol[o + k * 64] : L.n;   // x[n] holds +0
+        const size_t e = (size_t)t.y + (size_t)((k >> 2) * np + lane) * 4 + (k & 3);
+        const size_t ev = (size_t)t.y + (size_t)((k >> 1) * np + lane) * 2 + (k & 1);
+        if (sizeof(V) == 2) {
+            const unsigned v = k < w ? ((const uint16_t *)L.val)[o + k * 64] : 0x8000u;
+            ((unsigned *)(img + T.ent))[e] = (v << 16) | (unsigned)c;
+        } else {
+            ((uint16_t *)(img + T.ent))[e] = (uint16_t)c;
+            ((double *)(img + T.val))[ev] = k < w ? ((const double *)L.val)[o + k * 64] : -0.0;
+        }
+    }
+    ((D *)(img + T.diag))[p] = ((const D *)L.diag)[p];
+}
+
+// uniform value of a wavefront
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T>
+__device__ __forceinline__ T *uni(T *p) {
+    const unsigned long long u = (unsigned long long)p;
+    const unsigned lo = (unsigned)uni((int)(unsigned)u), hi = (unsigned)uni((int)(unsigned)(u >> 32));
+    return (T *)((unsigned long long)hi << 32 | lo);
+}
+
+// Entry groups (four entries of a row each) of both value types: group g of row ln of an
+// item of np rows whose first group is k.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+template <class V> struct TailGroup;
+template <> struct TailGroup<uint16_t> {
+    using X = float;
+    using E = u32x4;     // {BF16 value, column} x 4
+    using W = u32x4;     // (no separate values)
+    u32x4 q;
+    template <class PE, class PV>
+    __device__ __forceinline__ void load(PE ent, PV, int k, int g, int np, int ln) { q = ent[k + g * np + ln]; }
+    __device__ __forceinline__ void gather(const float *x, float *xv) const {
+        xv[0] = x[q.x & 0xffffu];
+        xv[1] = x[q.y & 0xffffu];
+        xv[2] = x[q.z & 0xffffu];
+        xv[3] = x[q.w & 0xffffu];
+    }
+    __device__ __forceinline__ float add(float acc, const float *xv) const {
+        acc += __uint_as_float(q.x & 0xffff0000u) * xv[0];
+        acc += __uint_as_float(q.y & 0xffff0000u) * xv[1];
+        acc += __uint_as_float(q.z & 0xffff0000u) * xv[2];
+        acc += __uint_as_float(q.w & 0xffff0000u) * xv[3];
+        return acc;
+    }
+};
+template <> struct TailGroup<double> {
+    using X = double;
+    using E = u16x4;     // columns x 4
+    using W = f64x2;     // values
+    u16x4 c;
+    f64x2 v0, v1;
+    template <class PE, class PV>
+    __device__ __forceinline__ void load(PE ent, PV val, int k, int g, int np, int ln) {
+        c = ent[k + g * np + ln];
+        v0 = val[2 * k + 2 * g * np + ln];
+        v1 = val[2 * k + (2 * g + 1) * np + ln];
+    }
+    __device__ __forceinline__ void gather(const double *x, double *xv) const {
+        xv[0] = x[c.x];
+        xv[1] = x[c.y];
+        xv[2] = x[c.z];
+        xv[3] = x[c.w];
+    }
+    __device__ __forceinline__ double add(double acc, const double *xv) const {
+        acc += v0.x * xv[0];
+        acc += v0.y * xv[1];
+        acc += v1.x * xv[2];
+        acc += v1.y * xv[3];
+        return acc;
+    }
+};
+// acc + G groups already loaded
+template <int G, class V, class X>
+__device__ __forceinline__ X tail_add(X acc, const TailGroup<V> *q, const X *x) {
+    X xv[4 * G];
+#pragma unroll
+    for (int g = 0; g < G; g++) q[g].gather(x, xv + 4 * g);
+#pragma unroll
+    for (int g = 0; g < G; g++) acc = q[g].add(acc, xv + 4 * g);
+    return acc;
+}
+// acc + groups g..g + G - 1 from memory
+template <int G, class V, class X, class PE, class PV>
+__device__ __forceinline__ X tail_chunk(X acc, PE ent, PV val, int k, int g, int np, int ln, const X *x) {
+    TailGroup<V> q[G];
+#pragma unroll
+    for (int u = 0; u < G; u++) q[u].load(ent, val, k, g + u, np, ln);
+    return tail_add<G, V, X>(acc, q, x);
+}
+template <class V, class X, class PE, class PV>
+__device__ __forceinline__ X tail_groups(X acc, PE ent, PV val, int k, int g, int ng, int np, int ln, const X *x) {
+    for (; g + 4 <= ng; g += 4) acc = tail_chunk<4, V, X>(acc, ent, val, k, g, np, ln, x);
+    if (ng - g == 3) acc = tail_chunk<3, V, X>(acc, ent, val, k, g, np, ln, x);
+    else if (ng - g == 2) acc = tail_chunk<2, V, X>(acc, ent, val, k, g, np, ln, x);
+    else if (ng - g == 1) acc = tail_chunk<1, V, X>(acc, ent, val, k, g, np, ln, x);
+    return acc;
+}
+
+// ns sweeps of a resident level: every operand in LDS, whose latency (65 clocks) needs no
+// look-ahead; only the next item's descriptor is read ahead
+template <class V, class D, class X>
+__device__ __forceinline__ void tail_sweep_lds(unsigned char *sm, const TailTab *T, X *x, int ns) {
+    using E = typename TailGroup<V>::E;
+    using W = typename TailGroup<V>::W;
+    const int lane = threadIdx.x & 63;
+    const bool one = uni(T->one_wave) != 0;
+    const int wave = uni(threadIdx.x >> 6), nw = one ? 1 : TAIL_NT / 64;
+    const int nc = uni(T->ncolor), per = 2 * nc - 1;   // forward, then back without the last colour again
+    const int2 *item = (const int2 *)(sm + uni(T->item));
+    const int *cptr = (const int *)(sm + uni(T->cptr));
+    const E *ent = (const E *)(sm + uni(T->ent));
+    const W *val = (const W *)(sm + uni(T->val));
+    const D *dg = (const D *)(sm + uni(T->diag));
+    const X *b = (const X *)(sm + uni(T->b));
+    if (!one || wave == 0)
+        for (int st = 0, r = 0; st < ns * per; st++, r = r + 1 < per ? r + 1 : 0) {
+            const int c = r < nc ? r : per - 1 - r;
+            const int end = uni(cptr[c + 1]);
+            for (int i = uni(cptr[c]) + wave; i < end; i += nw) {
+                const int2 u = item[i];
+                const int2 t = {uni(u.x), uni(u.y)};
+                const int np = item_rows(t), ng = item_groups(t);
+                const int ln = min(lane, np - 1);   // lanes past the item repeat its last row
+                const int p = item_row(t) + ln;
+                const D d = dg[p];
+                const X acc = tail_groups<V, X>(b[p], ent, val, t.y >> 2, 0, ng, np, ln, (const X *)x);
+                if (lane < np) x[p] = -acc / (X)d;
+            }
+            if (one) {   // the wavefront's LDS accesses stay in order: no barrier
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            } else {
+                __syncthreads();
+            }
+        }
+    if (one) __syncthreads();
+}
+
+// ns sweeps of a streamed level: item tables and x in LDS, the entries, the diagonal and
+// b from memory, each wavefront one item ahead (two items in registers, in turn)
+template <class V, class D, class X>
+struct TailItem {
+    TailGroup<V> q[TAIL_Q];
+    X b;
+    D d;
+    int p, np, ng, k, ln;   // this lane's row, rows (0: no item), groups, first group, place of the row
+};
+template <class V, class D, class X, class PE, class PV, class PD, class PB>
+__device__ __forceinline__ void tail_sweep_stream(unsigned char *sm, const TailTab *T, PE ent, PV val, PD dg, PB b,
+                                                  X *x, int ns) {
+    const int lane = threadIdx.x & 63;
+    const int wave = uni(threadIdx.x >> 6), nw = TAIL_NT / 64;
+    const int nc = uni(T->ncolor), per = 2 * nc - 1;
+    const int2 *item = (const int2 *)(sm + uni(T->item));
+    const int *cptr = (const int *)(sm + uni(T->cptr));
+    auto load = [&](TailItem<V, D, X> &P, int i, int end) {
+        P.np = 0;
+        if (i >= end) return;
+        const int2 u = item[i];
+        const int2 t = {uni(u.x), uni(u.y)};
+        P.np = item_rows(t);
+        P.ng = item_groups(t);
+        P.ln = min(lane, P.np - 1);
+        P.p = item_row(t) + P.ln;
+        P.k = t.y >> 2;
+#pragma unroll
+        for (int g = 0; g < TAIL_Q; g++)
+            if (g < P.ng) P.q[g].load(ent, val, P.k, g, P.np, P.ln);
+        P.b = b[P.p];
+        P.d = dg[P.p];
+    };
+    auto row = [&](const TailItem<V, D, X> &P) {
+        if (P.np == 0) return;
+        X acc = P.b;
+        if (P.ng >= 4) {
+            acc = tail_add<4, V, X>(acc, P.q, x);
+            if (P.ng > 4) acc = tail_groups<V, X>(acc, ent, val, P.k, 4, P.ng, P.np, P.ln, (const X *)x);
+        } else if (P.ng == 3) {
+            acc = tail_add<3, V, X>(acc, P.q, x);
+        } else if (P.ng == 2) {
+            acc = tail_add<2, V, X>(acc, P.q, x);
+        } else if (P.ng == 1) {
+            acc = tail_add<1, V, X>(acc, P.q, x);
+        }
+        if (lane < P.np) x[P.p] = -acc / (X)P.d;
+    };
+    int st = 0, r = 0;   // step, its place within the sweep
+    int i = uni(cptr[0]) + wave, end = uni(cptr[1]), nbeg = 0, nend = 0;
+    const int nst = ns * per;
+    auto ahead = [&]() {   // the first item and the end of the next step's colour (after the last step: not used)
+        const int rn = r + 1 < per ? r + 1 : 0, cn = rn < nc ? rn : per - 1 - rn;
+        nbeg = uni(cptr[cn]) + wave;
+        nend = uni(cptr[cn + 1]);
+        r = rn;
+    };
+    // the present item is in Q: its successor goes to P; true after the last step
+    auto turn = [&](TailItem<V, D, X> &Q, TailItem<V, D, X> &P) {
+        const bool more = i + nw < end;
+        load(P, more ? i + nw : nbeg, more ? end : nend);
+        row(Q);
+        i += nw;
+        if (!more) {
+            __syncthreads();
+            i = nbeg;
+            end = nend;
+            if (++st == nst) return true;
+            ahead();
+        }
+        return false;
+    };
+    TailItem<V, D, X> A, B;
+    load(A, i, end);
+    ahead();
+    while (!turn(A, B) && !turn(B, A)) {}
+}
+
+// bc[I] = sum of r over the fine rows of I in order, for every I < nc: NB coarse rows per
+// thread at a time, so that the dependent loads (range, rows, values) of all of them and
+// of up to five members are in flight together
+template <int NB, class PR, class PX, class X, class F>
+__device__ __forceinline__ void tail_restrict(int nc, PR row, PR col, PX r, F &&put) {
+    constexpr int M = 5;
+    for (int I0 = threadIdx.x; I0 < nc; I0 += NB * TAIL_NT) {
+        int q0[NB], m[NB], c[NB][M];
+        X v[NB][M];
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int I = min(I0 + u * TAIL_NT, nc - 1);
+            q0[u] = row[I];
+            m[u] = row[I + 1] - q0[u];
+        }
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+#pragma unroll
+            for (int j = 0; j < M; j++) c[u][j] = j < m[u] ? col[q0[u] + j] : -1;
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+#pragma unroll
+            for (int j = 0; j < M; j++) v[u][j] = c[u][j] >= 0 ? r[c[u][j]] : (X)0;
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            X sum = 0;
+#pragma unroll
+            for (int j = 0; j < M; j++)
+                if (j < m[u]) sum += v[u][j];
+            for (int j = M; j < m[u]; j++) sum += r[col[q0[u] + j]];
+            if (I0 + u * TAIL_NT < nc) put(I0 + u * TAIL_NT, sum);
+        }
+    }
+}
+
+// levels l0..last of a V-cycle (l0 holds its b, x is zero); levels >= lr are resident,
+// the coarsest one among them. img16: 16-byte words of the image that go to LDS, its
+// table (from level lp on) first; xoff: LDS offset of a streamed level's x.
+template <class V, class D, class X>
+__global__ void __launch_bounds__(TAIL_NT)
+k_tail_gs(const unsigned char *__restrict__ img, int img16, int lp, int l0, int lr, int last, int npost,
+          const double *__restrict__ inv, int direct, int xoff) {
+    using E = typename TailGroup<V>::E;
+    using W = typename TailGroup<V>::W;
+    extern __shared__ __align__(16) unsigned char sm[];
+    for (int i = threadIdx.x; i < img16; i += TAIL_NT) ((uint4 *)sm)[i] = ((const uint4 *)img)[i];
+    __syncthreads();
+    const TailTab *tab = (const TailTab *)sm - lp;
+    // down: b of each level from the one above (no pre-sweeps: b itself is restricted)
+    for (int l = l0; l < lr; l++) {
+        const GPtr<X> r = (GPtr<X>)(const X *)uni(tab[l].g_b);
+        const GPtr<int> row = (GPtr<int>)uni(tab[l].g_c2r), col = (GPtr<int>)uni(tab[l].g_c2c);
+        const int nc = uni(tab[l + 1].n);
+        if (l + 1 < lr) {
+            GMut<X> bc = (GMut<X>)(X *)uni(tab[l + 1].g_b);
+            tail_restrict<2, GPtr<int>, GPtr<X>, X>(nc, row, col, r, [&](int I, X v) { bc[I] = v; });
+        } else {
+            X *bc = (X *)(sm + uni(tab[l + 1].b));
+            tail_restrict<2, GPtr<int>, GPtr<X>, X>(nc, row, col, r, [&](int I, X v) { bc[I] = v; });
+        }
+        __syncthreads();
+    }
+    const int lt = l0 < lr ? lr : l0;   // first resident level of this tail
+    if (l0 >= lr) {
+        const GPtr<X> b = (GPtr<X>)(const X *)uni(tab[l0].g_b);
+        X *sb = (X *)(sm + uni(tab[l0].b));
+        for (int i = threadIdx.x; i < uni(tab[l0].n); i += TAIL_NT) sb[i] = b[i];
+        __syncthreads();
+    }
+    for (int l = lt; l < last; l++) {
+        X *bc = (X *)(sm + uni(tab[l + 1].b));
+        tail_restrict<1, const uint16_t *, const X *, X>(
+            uni(tab[l + 1].n), (const uint16_t *)(sm + uni(tab[l].c2r)), (const uint16_t *)(sm + uni(tab[l].c2c)),
+            (const X *)(sm + uni(tab[l].b)), [&](int I, X v) { bc[I] = v; });
+        __syncthreads();
+    }
+    // up, resident levels
+    for (int l = last; l >= lt; l--) {
+        const int n = uni(tab[l].n);
+        X *x = (X *)(sm + uni(tab[l].x));
+        if (l == last && direct) {
+            // x = -A^{-1} b, one wavefront per row, the sums in dense_row's order
+            const uint16_t *perm = (const uint16_t *)(sm + uni(tab[l].perm));
+            const uint16_t *iperm = (const uint16_t *)(sm + uni(tab[l].iperm));
+            const X *b = (const X *)(sm + uni(tab[l].b));
+            const int lane = threadIdx.x & 63;
+            constexpr int NR = 8;   // rows whose loads are in flight together
+            const int nw = TAIL_NT / 64;
+            double bj[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) bj[k] = lane + 64 * k < n ? (double)b[iperm[lane + 64 * k]] : 0.0;
+            for (int p0 = threadIdx.x >> 6; p0 < n; p0 += NR * nw) {
+                double a[NR][4], s[NR];
+#pragma unroll
+                for (int u = 0; u < NR; u++) {
+                    const int p = min(p0 + u * nw, n - 1);
+                    const double *ri = inv + (size_t)perm[p] * n;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) a[u][k] = ri[min(lane + 64 * k, n - 1)];
+                }
+#pragma unroll
+                for (int u = 0; u < NR; u++) {
+                    s[u] = 0;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        if (lane + 64 * k < n) s[u] += a[u][k] * bj[k];
+                }
+                for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+                    for (int u = 0; u < NR; u++) s[u] += __shfl_xor(s[u], o, 64);
+#pragma unroll
+                for (int u = 0; u < NR; u++)
+                    if (lane == 0 && p0 + u * nw < n) x[p0 + u * nw] = (X)(-s[u]);
+            }
+            __syncthreads();
+            continue;
+        }
+        if (l == last) {
+            for (int i = threadIdx.x; i <= n; i += TAIL_NT) x[i] = (X)0;
+        } else {
+            const uint16_t *pci = (const uint16_t *)(sm + uni(tab[l].pci));
+            const X *xc = (const X *)(sm + uni(tab[l + 1].x));
+            for (int i = threadIdx.x; i <= n; i += TAIL_NT) {
+                const int I = i < n ? pci[i] : 0xffff;
+                x[i] = I != 0xffff ? (X)0 + xc[I] : (X)0;
+            }
+        }
+        __syncthreads();
+        tail_sweep_lds<V, D, X>(sm, tab + l, x, npost);
+    }
+    if (l0 >= lr) {
+        const X *x = (const X *)(sm + uni(tab[l0].x));
+        GMut<X> gx = (GMut<X>)(X *)uni(tab[l0].g_x);
+        for (int i = threadIdx.x; i < uni(tab[l0].n); i += TAIL_NT) gx[i] = x[i];
+    }
+    // up, streamed levels
+    for (int l = lr - 1; l >= l0; l--) {
+        const TailTab *T = tab + l;
+        const int n = uni(T->n);
+        X *x = (X *)(sm + xoff);
+        const GPtr<int> pci = (GPtr<int>)uni(T->g_pci);
+        const GPtr<X> xg = (GPtr<X>)(const X *)uni(tab[l + 1].g_x);
+        const X *xs = (const X *)(sm + uni(tab[lr].x));
+        const bool below = l + 1 < lr;   // the level below is streamed as well
+        constexpr int NB = 4;
+        for (int i0 = threadIdx.x; i0 <= n; i0 += NB * TAIL_NT) {
+            int I[NB];
+            X v[NB];
+#pragma unroll
+            for (int u = 0; u < NB; u++) I[u] = i0 + u * TAIL_NT < n ? pci[i0 + u * TAIL_NT] : -1;
+#pragma unroll
+            for (int u = 0; u < NB; u++) {
+                v[u] = (X)0;
+                if (I[u] >= 0) v[u] = below ? xg[I[u]] : xs[I[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < NB; u++)
+                if (i0 + u * TAIL_NT <= n) x[i0 + u * TAIL_NT] = (X)0 + v[u];
+        }
+        __syncthreads();
+        tail_sweep_stream<V, D, X>(sm, T, (GPtr<E>)(const E *)(img + uni(T->ent)),
+                                   (GPtr<W>)(const W *)(img + uni(T->val)),
+                                   (GPtr<D>)(const D *)(img + uni(T->diag)), (GPtr<X>)(const X *)uni(T->g_b), x,
+                                   npost);
+        GMut<X> gx = (GMut<X>)(X *)uni(T->g_x);
+        for (int i = threadIdx.x; i < n; i += TAIL_NT) gx[i] = x[i];
+        __syncthreads();
     }
 }
 
@@ -1035,6 +1506,142 @@ void symmetric_scale(Run &R, int l, double *scale_out) {
     k_scale<<<1, 1, 0, s>>>(scratch_scalar(h, 8), scratch_scalar(h, 9), scale_out);
 }
 
+// The image of the tail levels for k_tail_gs (see there) behind the descriptors d:
+// the item tables of every packed level and the resident levels first (the part that
+// goes to LDS), then the entries of the streamed levels.
+void build_tail_image(Run &R, const std::vector<TailLv> &d) {
+    fvm_amg *h = R.h;
+    hipStream_t s = h->stream;
+    const bool direct = R.mixed && R.last == h->direct_level;
+    const int ds = R.mixed ? 4 : 8, xs = R.mixed ? 4 : 8;   // bytes per diagonal / x
+    std::vector<TailTab> tab(d.size());
+    std::vector<std::vector<int2>> items(d.size());
+    std::vector<std::vector<int>> cptr(d.size());
+    std::vector<long long> entries(d.size(), 0);
+    // items of every level that can be packed, from the coarsest up
+    int lp = R.last + 1;
+    for (int l = R.last; l >= 1; l--) {
+        const Level &L = h->lev[l];
+        if (L.n <= 0 || L.n > TAIL_ROWS_CAP || L.h_sell_off.empty()) break;
+        TailTab &T = tab[l];
+        T.n = L.n;
+        T.ncolor = L.ncolor;
+        T.one_wave = 1;
+        bool ok = true;
+        cptr[l].assign(1, 0);
+        for (int c = 0; c < L.ncolor; c++) {
+            const int cb = L.color_ptr[c], ce = L.color_ptr[c + 1];
+            if (ce - cb > 64) T.one_wave = 0;
+            for (int p0 = cb; p0 < ce; p0 += 64) {
+                const int cnt = std::min(64, ce - p0);
+                int w = 0;
+                for (int sl = p0 >> 6; sl <= (p0 + cnt - 1) >> 6; sl++)
+                    w = std::max(w, (L.h_sell_off[sl + 1] - L.h_sell_off[sl]) >> 6);
+                const int ng = (w + 3) / 4;
+                ok = ok && ng <= 255 && entries[l] + 256LL * ng < (1 << 28);
+                items[l].push_back({(int)((unsigned)p0 | (unsigned)cnt << 16 | (unsigned)ng << 24), (int)entries[l]});
+                entries[l] += (long long)cnt * ng * 4;
+            }
+            cptr[l].push_back((int)items[l].size());
+        }
+        if (!ok) break;
+        lp = l;
+    }
+    // resident levels, from the coarsest up while they fit beside every item table
+    long long used = al16((long long)sizeof(TailTab) * (R.last + 1 - lp));
+    for (int l = lp; l <= R.last; l++) used += al16(8LL * items[l].size()) + al16(4LL * cptr[l].size());
+    const int limit = std::min(TAIL_RES_BYTES, h->tail_lds_lim);
+    int lr = R.last + 1;
+    for (int l = R.last; l >= lp; l--) {
+        const bool dl = direct && l == R.last;
+        const long long nc = l < R.last ? d[l + 1].n : 0;
+        long long need = 2LL * al16((long long)xs * (d[l].n + 1));
+        if (dl) need += 2LL * al16(2LL * d[l].n);
+        else need += al16((R.mixed ? 4 : 2) * entries[l]) + (R.mixed ? 0 : al16(8 * entries[l])) + al16((long long)ds * d[l].n);
+        if (l < R.last) need += 2LL * al16(2LL * d[l].n) + al16(2 * (nc + 1));
+        if (used + need > limit) break;
+        used += need;
+        lr = l;
+    }
+    h->tail_lr = lr;
+    h->tail_lp = lp;
+    if (lr > R.last) return;
+    long long img = 0;
+    auto take = [&](long long bytes) {
+        const int o = (int)img;
+        img += al16(bytes);
+        return o;
+    };
+    auto take_matrix = [&](TailTab &T, int l) {
+        T.ent = take((R.mixed ? 4 : 2) * entries[l]);
+        T.val = R.mixed ? T.ent : take(8 * entries[l]);
+        T.diag = take((long long)ds * T.n);
+    };
+    std::vector<int2> work;
+    take((long long)sizeof(TailTab) * (R.last + 1 - lp));
+    for (int l = lp; l <= R.last; l++) {
+        tab[l].g_pci = d[l].pci;
+        tab[l].g_c2r = d[l].c2f_row;
+        tab[l].g_c2c = d[l].c2f_col;
+        tab[l].g_b = d[l].b;
+        tab[l].g_x = d[l].x;
+        tab[l].item = take(8LL * items[l].size());
+        tab[l].cptr = take(4LL * cptr[l].size());
+    }
+    const size_t tables = (size_t)img;
+    for (int l = lr; l <= R.last; l++) {
+        TailTab &T = tab[l];
+        T.resident = 1;
+        work.push_back({l, -1});
+        if (direct && l == R.last) {
+            T.perm = take(2LL * T.n);
+            T.iperm = take(2LL * T.n);
+            continue;
+        }
+        take_matrix(T, l);
+        if (l < R.last) {
+            T.pci = take(2LL * T.n);
+            T.c2r = take(2LL * (d[l + 1].n + 1));
+            T.c2c = take(2LL * T.n);
+        }
+        for (int i = 0; i < (int)items[l].size(); i++) work.push_back({l, i});
+    }
+    h->tail_img16 = (int)(img / 16);
+    long long lds = img;   // the resident vectors follow the image in LDS only
+    for (int l = lr; l <= R.last; l++) {
+        tab[l].b = (int)lds;
+        lds += al16((long long)xs * tab[l].n);
+        tab[l].x = (int)lds;
+        lds += al16((long long)xs * (tab[l].n + 1));
+    }
+    h->tail_res_bytes = (int)lds;
+    for (int l = lp; l < lr; l++) {
+        take_matrix(tab[l], l);
+        for (int i = 0; i < (int)items[l].size(); i++) work.push_back({l, i});
+    }
+    // device: work list, image (its tables uploaded, the rest packed there)
+    const size_t o_img = (sizeof(int2) * work.size() + 255) & ~(size_t)255;
+    std::vector<unsigned char> up(o_img + tables, 0);
+    memcpy(up.data(), work.data(), sizeof(int2) * work.size());
+    memcpy(up.data() + o_img, tab.data() + lp, sizeof(TailTab) * (R.last + 1 - lp));
+    for (int l = lp; l <= R.last; l++) {
+        memcpy(up.data() + o_img + tab[l].item, items[l].data(), 8 * items[l].size());
+        memcpy(up.data() + o_img + tab[l].cptr, cptr[l].data(), 4 * cptr[l].size());
+    }
+    h->tail_img.alloc(o_img + (size_t)img);
+    h->tail_o_img = o_img;
+    FVM_HIP(hipMemcpyAsync(h->tail_img.p, up.data(), up.size(), hipMemcpyHostToDevice, s));
+    const TailLv *dl = (const TailLv *)h->tail_desc.p;
+    const int2 *dw = (const int2 *)h->tail_img.p;
+    auto pack = [&](auto kern) {
+        kern<<<(unsigned)work.size(), 64, 0, s>>>(dl, dw, lp, R.last, direct ? 1 : 0, h->tail_img.p + o_img);
+    };
+    if (R.mixed) pack(k_tail_pack<uint16_t, float>);
+    else pack(k_tail_pack<double, double>);
+    FVM_HIP(hipGetLastError());
+    FVM_HIP(hipStreamSynchronize(s));
+}
+
 // Descriptors of every level for the tail kernel (coloured layout), built once per precision.
 template <class X>
 void build_tail_desc(Run &R) {
@@ -1075,11 +1682,16 @@ void build_tail_desc(Run &R) {
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lim));
             FVM_HIP(hipFuncSetAttribute((const void *)k_tail<double, double, double>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lim));
+            FVM_HIP(hipFuncSetAttribute((const void *)k_tail_gs<uint16_t, float, float>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, lim));
+            FVM_HIP(hipFuncSetAttribute((const void *)k_tail_gs<double, double, double>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, lim));
         }
     }
     h->tail_desc.alloc(sizeof(TailLv) * d.size());
     FVM_HIP(hipMemcpyAsync(h->tail_desc.p, d.data(), sizeof(TailLv) * d.size(), hipMemcpyHostToDevice, h->stream));
     FVM_HIP(hipStreamSynchronize(h->stream));
+    build_tail_image(R, d);
     h->tail_prec = prec;
 }
 
@@ -1133,6 +1745,23 @@ void cycle(Run &R, int type, int l, bool x_zero) {
         const TailLv *d = (const TailLv *)h->tail_desc.p;
         const int direct = (R.mixed && R.last == h->direct_level) ? 1 : 0;
         const int jac = h->prm.smootherType == FVM_JACOBI ? 1 : 0;
+        // the usual cycle: smallest levels resident in LDS, the others with x in LDS
+        if (h->tail_lds && !jac && h->prm.nPreSweeps == 0 && h->prm.nPostSweeps > 0 && h->tail_lr <= R.last &&
+            l >= h->tail_lp) {
+            long long lds = h->tail_res_bytes;
+            if (l < h->tail_lr) lds += al16((R.mixed ? 4LL : 8LL) * (h->lev[l].n + 1));   // the largest streamed level
+            if (lds <= h->tail_lds_lim) {
+                auto launch = [&](auto kern) {
+                    kern<<<1, TAIL_NT, (size_t)lds, s>>>(h->tail_img.p + h->tail_o_img, h->tail_img16, h->tail_lp, l,
+                                                         h->tail_lr, R.last, h->prm.nPostSweeps, h->dense_inv.p,
+                                                         direct, h->tail_res_bytes);
+                };
+                if (R.mixed) launch(k_tail_gs<uint16_t, float, float>);
+                else launch(k_tail_gs<double, double, double>);
+                FVM_HIP(hipGetLastError());
+                return;
+            }
+        }
         // LDS for the largest tail level within the limit set up with the descriptors
         int cap = 0;
         if (h->tail_lds)

@@ -2111,6 +2111,7 @@ void build_hierarchy(fvm_amg *h, int n_self, int n_total, const int *d_row, cons
     h->direct_tried = false;
     h->tail_prec = -1;
     h->tail_desc.release();
+    h->tail_img.release();
     invalidate_cycle_graphs(h);
     h->n_self = n_self;
     h->n_total = n_total;
@@ -2394,7 +2395,15 @@ void prepare_fast_level(fvm_amg *h, Level &L, int l, hipStream_t s, Workspace &w
     k_sell_width<<<grid_for(nslice, BS, 4096), BS, 0, s>>>(n, nslice, L.perm.p, L.row.p, w64.p);
     L.sell_off.alloc((size_t)nslice + 1);
     ws.scan.exclusive(w64.p, L.sell_off.p, nslice + 1, s);
-    const int total = read_scalar(L.sell_off.p + nslice, s);
+    int total;
+    if (n <= 16384) {   // levels that the single-workgroup tail may pack: it needs every slice's width
+        L.h_sell_off.resize((size_t)nslice + 1);
+        FVM_HIP(hipMemcpyAsync(L.h_sell_off.data(), L.sell_off.p, L.sell_off.bytes(), hipMemcpyDeviceToHost, s));
+        FVM_HIP(hipStreamSynchronize(s));
+        total = L.h_sell_off[nslice];
+    } else {
+        total = read_scalar(L.sell_off.p + nslice, s);
+    }
     L.sell_total = total;
     {
         const double wmean = (double)total / (64.0 * nslice);
@@ -2627,6 +2636,7 @@ void build_hierarchy_batched(fvm_amg *h, BatchInfo &B) {
     h->direct_tried = false;
     h->tail_prec = -1;
     h->tail_desc.release();
+    h->tail_img.release();
     invalidate_cycle_graphs(h);
     std::vector<int> off0(K + 1, 0);
     bool any_bnd = false;

@@ -1,0 +1,47 @@
+"""The packed single-workgroup tail of the coloured V-cycle (resident and streamed levels)
+gives the bits of the launched cycle: sizes at the edges of its items (64 rows), of the
+single-wavefront levels and of what stays resident; both precisions, one and two sweeps."""
+import numpy as np
+import pytest
+
+import matgen
+from test_gpu_parity import gpu_amg, ls_from
+
+pytestmark = pytest.mark.gpu
+
+
+def box_rows(n, seed):
+    """A random sparse matrix without structure: non-symmetric pattern, ragged rows."""
+    rng = np.random.default_rng(seed)
+    row, col, off = [0], [], []
+    for i in range(n):
+        c = rng.choice(n, size=min(n - 1, int(rng.integers(0, 24))), replace=False)
+        c = c[c != i]
+        col += list(c)
+        off += list(rng.uniform(0.01, 1.0, len(c)))
+        row.append(len(col))
+    diag = np.array([-1.2 * sum(off[row[i]:row[i + 1]]) - 0.1 for i in range(n)])
+    return dict(n_self=n, n_total=n, row=np.array(row, np.int32), col=np.array(col, np.int32), diag=diag,
+                off=np.array(off), b=rng.uniform(-1, 1, n))
+
+
+CASES = {"chain65": lambda: matgen.chain(65, d=-2.1), "chain130": lambda: matgen.chain(130, d=-2.1),
+         "grid5": lambda: matgen.grid3d(5, seed=1), "grid11": lambda: matgen.grid3d(11, seed=2, contrast=1.5),
+         "grid21": lambda: matgen.grid3d(21, seed=3, contrast=2.0), "grid26": lambda: matgen.grid3d(26, seed=4),
+         "ragged63": lambda: box_rows(63, 5), "ragged700": lambda: box_rows(700, 6),
+         "ragged3000": lambda: box_rows(3000, 7)}
+
+
+@pytest.mark.parametrize("prec,npost", [(0, 1), (1, 1), (0, 2), (1, 2)])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_packed_tail_is_bit_identical(case, prec, npost):
+    m = CASES[case]()
+    res = []
+    for tail in (0, 6000, 1 << 30):
+        a = gpu_amg(gsOrdering=1, precision=prec, nPostSweeps=npost, nMaxIterations=6, relativeTolerance=1e-30)
+        a.set_tuning("tail_max_rows", tail)
+        ls = ls_from(m)
+        a.solve(ls)
+        res.append((ls.delta.copy(), a.history()))
+    for d, h in res[1:]:
+        assert np.array_equal(res[0][0], d) and np.array_equal(res[0][1], h)
