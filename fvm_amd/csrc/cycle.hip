@@ -314,6 +314,245 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
     if (threadIdx.x == 0) atomicAdd(&ctl[1], 1);
 }
 
+// ---------------------------------------------------- reference order in one workgroup
+// A reference-order sweep (both directions) of a level by one workgroup. Spread over the
+// chip (k_csr_gs_flow) a hop from one dependency level to the next costs 2 to 6 us: the
+// new value goes through the memory side of the caches. Inside one workgroup it goes
+// through LDS: 0.35 us a hop for rows of 4 entries, 0.6 us for 10. Items of up to 64 rows of one dependency level are
+// taken by the wavefronts in turn; a wavefront loads its item's rows, entries and old
+// values while the items before it are still running, then waits (an LDS counter of
+// finished items) until every item of the earlier dependency levels is done. Item i waits
+// only for items below it, so every wait ends. New values lie in an LDS ring, by their
+// place in the schedule; a value that the ring has overwritten is read back from memory,
+// where it was stored many items ago by a wavefront of the same CU, whose vector memory
+// operations pass its L1 in order.
+// The price is one CU's throughput (about 20 GB/s of what its L2 does not hold), so b and
+// x are first brought into the order of the schedule: rows of one dependency level side
+// by side, sorted, their neighbours nearly so (44k rows: 510 -> 320 us a sweep). An item
+// takes 0.2 us, a hop across the chip about 2.9 us: past FL_ITEMS items per dependency level, and past FL_ROWS rows, whose entries
+// come from HBM, the whole chip is faster (210,000 rows, 7 items per level: 1.3 ms slower
+// per sweep here). Milliseconds per V-cycle against chip-wide sweeps on every level:
+// 27,000 rows 1.31 / 5.08, 125,000 rows 3.7 / 11.1, 729,000 rows 15.6 / 26.2.
+// One schedule serves both directions: its reverse is a valid order of the backward sweep.
+// Arithmetic and order per row: those of k_csr_gs_flow.
+// Shapes by the level's longest row: two, four or six groups of four entries loaded ahead
+// (each costs registers and LDS words for the entries' old values). An entry past those
+// is read after the wait, which costs the hop a round trip to memory.
+constexpr int FL_ITEMS = 12;        // items per dependency level, on average, up to which one workgroup is used
+constexpr int FL_ROWS = 150000;
+constexpr int FL_OWN_ROWS = 4096;   // up to here the kernel reorders x and b itself (8 rows per thread)
+constexpr int FL_NW = 8;   // wavefronts (twelve were slower: 44k rows, 620 against 510 us a sweep)
+template <class X> constexpr int fl_ring() { return sizeof(X) == 8 ? 4096 : 8192; }
+template <class X, int NW, int Q> constexpr size_t fl_lds() {
+    return sizeof(X) * (size_t)(NW * Q * 4 * 64 + fl_ring<X>() + 1) + 2 * sizeof(int);
+}
+// entry codes: >= 0 the row whose old value is read; FL_NEW | place in the ring (the zero
+// word past its end for padding); FL_NEW | FL_FAR | row for a value no longer in the ring
+constexpr int FL_NEW = (int)0x80000000, FL_FAR = 0x40000000, FL_IDX = 0x3fffffff;
+
+// groups of four of every item (one wavefront each): count takes their place, fill packs
+// the entries: codes at group (eo + g * np + row), values likewise
+template <class V, class X, bool FILL>
+__global__ void __launch_bounds__(64)
+k_flow_pack(int n, int dir, int4 *items, const int *lvl_end, const int *rows, const int *place, const int *row,
+            const int *col, const V *off, const X *diag, int *total, int4 *code, X *val, X *dg) {   // total: groups, longest item
+    constexpr int R = fl_ring<X>();
+    int4 t = items[blockIdx.x];
+    const int np = t.y & 0xff, lane = threadIdx.x;
+    // the backward sweep takes the schedule from its end; place[] is the forward place
+    const int i = lane < np ? rows[dir ? n - 1 - (t.x + lane) : t.x + lane] : -1;
+    const int rb = i >= 0 ? row[i] : 0, len = i >= 0 ? row[i + 1] - rb : 0;
+    if (!FILL) {
+        int m = len;
+        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+        if (lane == 0) {
+            const int ng = max(1, (m + 3) / 4);   // (rows without entries: one group of padding)
+            t.y = np | ng << 8;
+            t.w = atomicAdd(total, np * ng);
+            atomicMax(total + 1, ng);
+            items[blockIdx.x] = t;
+        }
+        return;
+    }
+    if (i < 0) return;
+    dg[t.x + lane] = diag[i];
+    const int ng = t.y >> 8, le = lvl_end[blockIdx.x];
+    for (int k = 0; k < 4 * ng; k++) {
+        int c = FL_NEW | R;   // padding: -0 times the ring's zero word, which leaves the sum unchanged
+        X v = (X)-0.0;
+        if (k < len) {
+            const int j = col[rb + k];
+            v = (X)ldv(off, rb + k);
+            c = place[j];
+            if (dir ? j > i : j < i) {
+                const int q = dir ? n - 1 - c : c;   // its turn in this sweep
+                c = FL_NEW | (le - q <= R ? q & (R - 1) : FL_FAR | c);
+            }
+        }
+        const size_t g = (size_t)t.w + (size_t)(k >> 2) * np + lane;
+        ((int *)(code + g))[k & 3] = c;
+        val[4 * g + (k & 3)] = v;
+    }
+}
+
+__global__ void k_flow_place(int n, const int *rows, int *place) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) place[rows[k]] = k;
+}
+
+template <class X>
+struct FlowDir {
+    const int4 *items;   // first place, rows | groups << 8, items that must be done, first group
+    const int4 *code;
+    const X *val, *dg;
+    int nitem;
+};
+
+// b and x in the order of the schedule, and x back
+template <class X>
+__global__ void k_flow_in(int n, const int *__restrict__ rows, const X *__restrict__ x, const X *__restrict__ b,
+                          X *__restrict__ xp, X *__restrict__ bp) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int i = rows[k];
+        xp[k] = x[i];
+        bp[k] = b[i];
+    }
+}
+template <class X>
+__global__ void k_flow_out(int n, const int *__restrict__ rows, const X *__restrict__ xp, X *__restrict__ x) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) x[rows[k]] = xp[k];
+}
+
+template <class X, int NW, int Q>
+__global__ void __launch_bounds__(64 * NW)
+k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const int *__restrict__ rows, X *x_io,
+             const X *b_in, const uint8_t *__restrict__ mask, int *ctl, int spin_limit) {
+    constexpr int R = fl_ring<X>(), FL_SCR = NW * Q * 4 * 64;
+    extern __shared__ __align__(16) unsigned char s_fl[];
+    X *sm = (X *)s_fl;            // [0, FL_SCR): old values; then the ring and its zero word
+    int *done = (int *)(sm + FL_SCR + R + 1), *stop = done + 1;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int waits = 0;
+    if (x_io)   // a small level: x and b brought into schedule order here, without launches of their own
+        for (int k = threadIdx.x; k < n; k += 64 * NW) {
+            const int i = rows[k];
+            xa[k] = x_io[i];
+            b[k] = b_in[i];
+        }
+    if (threadIdx.x == 0) {
+        sm[FL_SCR + R] = (X)0;
+        *stop = __hip_atomic_load(&ctl[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int dir = 0; dir < 2; dir++) {
+        const FlowDir<X> D = dir ? bwd : fwd;
+        const X *xo = dir ? xb : xa;
+        X *xn = dir ? xa : xb;
+        if (threadIdx.x == 0) *done = 0;
+        __syncthreads();
+        if (*stop) return;
+        int4 tn = wave < D.nitem ? D.items[wave] : int4{0, 0, 0, 0};
+        for (int it = wave; it < D.nitem; it += NW) {
+            const int p0 = __builtin_amdgcn_readfirstlane(tn.x), pk = __builtin_amdgcn_readfirstlane(tn.y);
+            const int need = __builtin_amdgcn_readfirstlane(tn.z), eo = __builtin_amdgcn_readfirstlane(tn.w);
+            const int np = pk & 0xff, ng = pk >> 8;
+            if (it + NW < D.nitem) tn = D.items[it + NW];
+            const int ln = min(lane, np - 1), pos = p0 + ln;
+            const int i = dir ? n - 1 - pos : pos;   // its place in the vectors
+            const X di = D.dg[pos];
+            // groups past the item's last repeat it and are not added: no branches in the loads
+            int a[4 * Q];
+            X v[4 * Q], old[4 * Q];
+#pragma unroll
+            for (int g = 0; g < Q; g++) {
+                const int e = eo + min(g, ng - 1) * np + ln;
+                const int4 c = D.code[e];
+                a[4 * g] = c.x; a[4 * g + 1] = c.y; a[4 * g + 2] = c.z; a[4 * g + 3] = c.w;
+#pragma unroll
+                for (int u = 0; u < 4; u++) v[4 * g + u] = D.val[4 * (size_t)e + u];
+            }
+            const X bi = b[i];
+            const bool keep = mask && !mask[rows[i]];   // row of a system that has stopped cycling
+            X xold = (X)0;
+            if (keep) xold = xo[i];
+            // old values to the scratch words, and the LDS word of each entry
+#pragma unroll
+            for (int u = 0; u < 4 * Q; u++) old[u] = xo[a[u] >= 0 ? a[u] : i];
+            bool far = false;
+            int sc[4 * Q];
+#pragma unroll
+            for (int u = 0; u < 4 * Q; u++) {
+                const int own = (wave * 4 * Q + u) * 64 + lane;
+                sm[own] = old[u];
+                sc[u] = a[u] >= 0 ? own : (a[u] & FL_FAR) ? ~(a[u] & FL_IDX) : FL_SCR + (a[u] & FL_IDX);
+                far = far || sc[u] < 0;
+            }
+            const bool anyfar = __any(far);
+            // every item of the earlier dependency levels done?
+            while (__builtin_amdgcn_readfirstlane(
+                       __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < need) {
+                if (spin_limit > 0) {   // a caller's bound on the waits (0: none)
+                    if (++waits >= spin_limit) {
+                        if (lane == 0) {
+                            atomicOr(&ctl[2], 1);
+                            __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                        break;
+                    }
+                    if (__builtin_amdgcn_readfirstlane(
+                            __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)))
+                        break;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (anyfar) {
+#pragma unroll
+                for (int u = 0; u < 4 * Q; u++)
+                    if (sc[u] < 0) {
+                        const X w = __hip_atomic_load(xn + ~sc[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        sc[u] = (wave * 4 * Q + u) * 64 + lane;
+                        sm[sc[u]] = w;
+                    }
+            }
+            // the reference's arithmetic: b, then the entries in CSR order, over -diag
+            X xv[4 * Q];
+#pragma unroll
+            for (int u = 0; u < 4 * Q; u++) xv[u] = sm[sc[u]];
+            X acc = bi;
+#pragma unroll
+            for (int g = 0; g < Q; g++)
+                if (g < ng) {
+#pragma unroll
+                    for (int u = 4 * g; u < 4 * g + 4; u++) acc += v[u] * xv[u];
+                }
+            for (int g = Q; g < ng; g++) {   // long rows
+                const size_t e = (size_t)eo + g * np + ln;
+                const int4 c4 = D.code[e];
+                const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+                X w[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (c[u] >= 0) w[u] = xo[c[u]];
+                    else if (c[u] & FL_FAR) w[u] = __hip_atomic_load(xn + (c[u] & FL_IDX), __ATOMIC_RELAXED,
+                                                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+                    else w[u] = sm[FL_SCR + (c[u] & FL_IDX)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) acc += D.val[4 * e + u] * w[u];
+            }
+            const X x = keep ? xold : -acc / di;
+            if (lane < np) {
+                sm[FL_SCR + (pos & (R - 1))] = x;
+                __hip_atomic_store(xn + i, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            // LDS operations of a wavefront are performed in order: the values before the count
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            if (lane == 0) __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        __syncthreads();
+    }
+    if (x_io)
+        for (int k = threadIdx.x; k < n; k += 64 * NW) x_io[rows[k]] = xa[k];
+}
+
 // Launch plan of a reference-order sweep from its dependency-level offsets hp
 // (nlev levels): each maximal run of consecutive levels of at most W rows is one
 // single-workgroup launch; every wider level is a launch of its own.
@@ -1401,6 +1640,27 @@ void gs_sweep(Run &R, int l, X *x, const X *b) {
             // b read, x read and written (the neighbours' x are counted once per updated row)
             if (t0) timing_end(R.h, KT_SWEEP, t0, pass_bytes(value_type(R, l), sizeof(X), 3, rows, nnz));
         }
+    } else if (R.h->exact_flow && L.flow_prec == (sizeof(X) == 8 ? 0 : 1)) {
+        fvm_amg *h = R.h;
+        h->flow_used = true;
+        DArr<X> &xa = vx_arr<X>(L);
+        FVM_CHECK(x == xa.p, FVM_E_INVALID, "reference-order sweep on a vector other than the level's own");
+        auto dirp = [&](Level::FlowPack &P) {
+            return FlowDir<X>{(const int4 *)P.items.p, (const int4 *)P.code.p, (const X *)P.val.p, (const X *)P.dg.p,
+                              P.nitem};
+        };
+        const int n = L.n;
+        X *xp = (X *)L.flow_vec.p, *xq = xp + n, *bp = xq + n;
+        const bool own = n <= FL_OWN_ROWS;
+        if (!own) k_flow_in<X><<<grid_for(n, BS), BS, 0, s>>>(n, L.fwd_rows.p, x, b, xp, bp);
+        auto launch = [&](auto kern, int nw, size_t lds) {
+            kern<<<1, 64 * nw, lds, s>>>(n, dirp(L.flow[0]), dirp(L.flow[1]), xp, xq, bp, L.fwd_rows.p,
+                                         own ? x : nullptr, b, l == 0 ? R.mask0 : nullptr, h->flow_ctl.p, h->flow_spin_limit);
+        };
+        if (L.flow_groups <= 2) launch(k_gs_flow_wg<X, FL_NW, 2>, FL_NW, fl_lds<X, FL_NW, 2>());
+        else if (L.flow_groups <= 4) launch(k_gs_flow_wg<X, FL_NW, 4>, FL_NW, fl_lds<X, FL_NW, 4>());
+        else launch(k_gs_flow_wg<X, FL_NW, 6>, FL_NW, fl_lds<X, FL_NW, 6>());
+        if (!own) k_flow_out<X><<<grid_for(n, BS), BS, 0, s>>>(n, L.fwd_rows.p, xp, x);
     } else if (R.h->exact_flow) {
         fvm_amg *h = R.h;
         FVM_CHECK(h->flow_ctl.p, FVM_E_INVALID, "reference-order sweep before its control words exist");
@@ -1828,6 +2088,108 @@ void cycle(Run &R, int type, int l, bool x_zero) {
     FVM_HIP(hipGetLastError());
 }
 
+// Packs of the one-workgroup sweep (k_gs_flow_wg) for every level it is used on, built
+// once per hierarchy and precision.
+template <class X>
+void prepare_flow_packs(Run &R) {
+    fvm_amg *h = R.h;
+    hipStream_t s = h->stream;
+    const int prec = sizeof(X) == 8 ? 0 : 1;
+    constexpr int RING = fl_ring<X>();
+    struct Job { int l, dir; std::vector<int4> items; std::vector<int> lend; DArr<int> d_lend; };
+    std::vector<Job> jobs;
+    std::vector<DArr<int>> place(h->lev.size());
+    for (int l = 0; l < (int)h->lev.size(); l++) {
+        Level &L = h->lev[l];
+        if (L.flow_prec == prec) continue;
+        L.flow_prec = -1;
+        // a value leaves the ring well after it was stored: more items later than there are wavefronts
+        if (L.n == 0 || L.n > FL_ROWS || std::max(L.fwd_maxw, L.bwd_maxw) + 64 * (FL_NW + 1) > RING) continue;
+        long long nitem = 0;
+        for (int k = 0; k < L.fwd_nlev; k++) nitem += (L.h_fwd_ptr[k + 1] - L.h_fwd_ptr[k] + 63) / 64;
+        if (nitem > (long long)FL_ITEMS * L.fwd_nlev) continue;
+        for (int dir = 0; dir < 2; dir++) {
+            jobs.emplace_back();
+            Job &J = jobs.back();
+            J.l = l;
+            J.dir = dir;
+            const std::vector<int> &hp = dir ? L.h_bwd_ptr : L.h_fwd_ptr;
+            for (size_t k = 0; k + 1 < hp.size(); k++) {
+                const int need = (int)J.items.size();
+                for (int p = hp[k]; p < hp[k + 1]; p += 64) {
+                    J.items.push_back({p, std::min(64, hp[k + 1] - p), need, 0});
+                    J.lend.push_back(hp[k + 1]);
+                }
+            }
+        }
+    }
+    if (jobs.empty()) return;
+    // the device's LDS for the kernel, granted once (outside any capture)
+    FVM_HIP(hipFuncSetAttribute((const void *)k_gs_flow_wg<X, FL_NW, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)fl_lds<X, FL_NW, 2>()));
+    FVM_HIP(hipFuncSetAttribute((const void *)k_gs_flow_wg<X, FL_NW, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)fl_lds<X, FL_NW, 4>()));
+    FVM_HIP(hipFuncSetAttribute((const void *)k_gs_flow_wg<X, FL_NW, 6>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)fl_lds<X, FL_NW, 6>()));
+    DArr<int> total(2 * jobs.size());
+    FVM_HIP(hipMemsetAsync(total.p, 0, total.bytes(), s));
+    auto launch = [&](Job &J, int k, bool fill) {
+        Level &L = h->lev[J.l];
+        Level::FlowPack &P = L.flow[J.dir];
+        const int *rows = L.fwd_rows.p;
+        auto go = [&](const auto *off, const X *diag) {
+            using V = std::remove_const_t<std::remove_pointer_t<decltype(off)>>;
+            if (fill)
+                k_flow_pack<V, X, true><<<P.nitem, 64, 0, s>>>(L.n, J.dir, (int4 *)P.items.p, J.d_lend.p, rows, place[J.l].p, L.row.p,
+                                                               L.col.p, off, diag, total.p + 2 * k, (int4 *)P.code.p,
+                                                               (X *)P.val.p, (X *)P.dg.p);
+            else
+                k_flow_pack<V, X, false><<<P.nitem, 64, 0, s>>>(L.n, J.dir, (int4 *)P.items.p, nullptr, rows, nullptr, L.row.p,
+                                                                L.col.p, off, diag, total.p + 2 * k, nullptr, nullptr,
+                                                                nullptr);
+        };
+        if constexpr (sizeof(X) == 8) {
+            go((const double *)L.off.p, L.diag.p);
+        } else {
+            if (J.l == 0) go((const float *)L.off32.p, L.diag32.p);
+            else go((const uint16_t *)L.off16.p, L.diag32.p);
+        }
+        FVM_HIP(hipGetLastError());
+    };
+    for (size_t k = 0; k < jobs.size(); k++) {
+        Job &J = jobs[k];
+        Level &L = h->lev[J.l];
+        Level::FlowPack &P = L.flow[J.dir];
+        P.nitem = (int)J.items.size();
+        P.items.alloc(4 * J.items.size());
+        J.d_lend.alloc(J.lend.size());
+        if (J.dir == 0) {
+            place[J.l].alloc(L.n);
+            L.flow_vec.alloc(3 * sizeof(X) * (size_t)L.n);
+            k_flow_place<<<grid_for(L.n, BS, 4096), BS, 0, s>>>(L.n, L.fwd_rows.p, place[J.l].p);
+        }
+        FVM_HIP(hipMemcpyAsync(P.items.p, J.items.data(), sizeof(int4) * J.items.size(), hipMemcpyHostToDevice, s));
+        FVM_HIP(hipMemcpyAsync(J.d_lend.p, J.lend.data(), sizeof(int) * J.lend.size(), hipMemcpyHostToDevice, s));
+        launch(J, (int)k, false);
+    }
+    std::vector<int> ht(2 * jobs.size());
+    FVM_HIP(hipMemcpyAsync(ht.data(), total.p, total.bytes(), hipMemcpyDeviceToHost, s));
+    FVM_HIP(hipStreamSynchronize(s));
+    for (size_t k = 0; k < jobs.size(); k++) {
+        Job &J = jobs[k];
+        Level::FlowPack &P = h->lev[J.l].flow[J.dir];
+        const size_t g = std::max(ht[2 * k], 1);
+        Level &L = h->lev[J.l];
+        L.flow_groups = J.dir ? std::max(L.flow_groups, ht[2 * k + 1]) : ht[2 * k + 1];
+        P.code.alloc(4 * g);
+        P.val.alloc(4 * sizeof(X) * g);
+        P.dg.alloc(sizeof(X) * (size_t)h->lev[J.l].n);
+        launch(J, (int)k, true);
+    }
+    FVM_HIP(hipStreamSynchronize(s));
+    for (Job &J : jobs) h->lev[J.l].flow_prec = prec;
+}
+
 Run make_run(fvm_amg *h) {
     FVM_CHECK(h->ready, FVM_E_NOT_SETUP, "solve/smooth called before setup");
     Run R;
@@ -1848,6 +2210,10 @@ Run make_run(fvm_amg *h) {
     if (R.mixed) {
         prepare_mixed(h, R.fast);
         if (h->direct_level < 0 && !h->direct_tried) prepare_direct(h);
+    }
+    if (!R.fast && h->exact_flow && h->prm.smootherType == FVM_GAUSS_SEIDEL) {
+        if (R.mixed) prepare_flow_packs<float>(R);
+        else prepare_flow_packs<double>(R);
     }
     R.last = (int)h->lev.size() - 1;
     if (R.mixed && h->direct_level >= 0) R.last = h->direct_level;

@@ -1293,6 +1293,28 @@ __global__ void k_sched_round(int lvl, int dir, const int *row, const int *col, 
     }
 }
 
+// dependency level of every row (place k of the schedule lies in the level l with
+// ptr[l] <= k < ptr[l + 1]), and the rows in ascending order
+__global__ void k_sched_level(int n, int nlev, const int *ptr, const int *rows, int *lev, int *idx) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        int lo = 0, hi = nlev;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (ptr[mid] <= k) lo = mid;
+            else hi = mid;
+        }
+        lev[rows[k]] = lo;
+        idx[k] = k;
+    }
+}
+
+__global__ void k_sched_reverse(int n, int nlev, const int *rows, const int *ptr, int *brows, int *bptr) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < max(n, nlev + 1); k += gridDim.x * blockDim.x) {
+        if (k < n) brows[k] = rows[n - 1 - k];
+        if (k <= nlev) bptr[k] = n - ptr[nlev - k];
+    }
+}
+
 __global__ void k_set_ptr01(int *ptr, const int *tail) {
     ptr[0] = 0;
     ptr[1] = *tail;
@@ -2229,11 +2251,10 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
     const int n = L.n;
     if (n == 0) { L.sched_ready = true; return; }
     ensure_transpose(h, L);
-    for (int dir = 0; dir < 2; dir++) {
+    std::vector<int> &hp = L.h_fwd_ptr;
+    {
         DArr<int> indeg(n), ctr(2);
-        DArr<int> &rows = dir ? L.bwd_rows : L.fwd_rows;
-        DArr<int> &ptr = dir ? L.bwd_ptr : L.fwd_ptr;
-        rows.alloc(n);
+        DArr<int> rows(n), ptr;
         const int batch = 32;
         ptr.alloc((size_t)n + batch + 4);
         FVM_HIP(hipMemsetAsync(ctr.p, 0, ctr.bytes(), s));
@@ -2241,8 +2262,7 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
         unsigned *done_blocks = (unsigned *)(ctr.p + 1);
         const int *rT = L.sym ? nullptr : L.rowT.p;
         const int *cT = L.sym ? nullptr : L.colT.p;
-        k_sched_init<<<grid_for(n, BS, 4096), BS, 0, s>>>(n, dir, L.row.p, L.col.p, rT, cT, indeg.p,
-                                                          rows.p, tail);
+        k_sched_init<<<grid_for(n, BS, 4096), BS, 0, s>>>(n, 0, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, tail);
         k_set_ptr01<<<1, 1, 0, s>>>(ptr.p, tail);
         FVM_HIP(hipGetLastError());
         int lvl = 0;
@@ -2250,8 +2270,8 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
         for (;;) {
             for (int k = 0; k < batch; k++, lvl++) {
                 FVM_CHECK((size_t)lvl + 2 < ptr.n, FVM_E_NUMERIC, "GS schedule overflow");
-                k_sched_round<<<g, BS, 0, s>>>(lvl, dir, L.row.p, L.col.p, rT, cT, indeg.p, rows.p,
-                                               ptr.p, tail, done_blocks);
+                k_sched_round<<<g, BS, 0, s>>>(lvl, 0, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, ptr.p, tail,
+                                               done_blocks);
             }
             FVM_HIP(hipGetLastError());
             if (read_scalar(tail, s) >= n) break;
@@ -2263,14 +2283,38 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
                 ptr = std::move(np);
             }
         }
-        std::vector<int> hp(lvl + 2);
+        hp.resize(lvl + 2);
         FVM_HIP(hipMemcpyAsync(hp.data(), ptr.p, sizeof(int) * (lvl + 2), hipMemcpyDeviceToHost, s));
         FVM_HIP(hipStreamSynchronize(s));
         int nl = 0, maxw = 0;
         while (nl + 1 < (int)hp.size() && hp[nl] < n) { maxw = std::max(maxw, hp[nl + 1] - hp[nl]); nl++; }
         hp.resize(nl + 1);
-        if (dir) { L.bwd_nlev = nl; L.bwd_maxw = maxw; L.h_bwd_ptr = hp; }
-        else { L.fwd_nlev = nl; L.fwd_maxw = maxw; L.h_fwd_ptr = hp; }
+        L.fwd_nlev = L.bwd_nlev = nl;
+        L.fwd_maxw = L.bwd_maxw = maxw;
+        // rows ascending inside each dependency level (the rounds append them in any order)
+        DArr<int> key(n), key_out(n), idx(n);
+        L.fwd_rows.alloc(n);
+        k_sched_level<<<grid_for(n, BS, 4096), BS, 0, s>>>(n, nl, ptr.p, rows.p, key.p, idx.p);
+        int bits = 1;
+        while ((1LL << bits) <= nl) bits++;
+        size_t bytes = 0;
+        FVM_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, key.p, key_out.p, idx.p, L.fwd_rows.p, n, 0, bits, s));
+        h->ws.sort_tmp.ensure(bytes + 16);
+        FVM_HIP(hipcub::DeviceRadixSort::SortPairs(h->ws.sort_tmp.p, bytes, key.p, key_out.p, idx.p, L.fwd_rows.p, n, 0,
+                                                   bits, s));
+        L.fwd_ptr = std::move(ptr);
+    }
+    // backward: the same schedule from its end. A row reads new values of linked rows of
+    // higher index, all of them in later forward levels.
+    {
+        const int nl = L.fwd_nlev;
+        L.h_bwd_ptr.resize(nl + 1);
+        for (int k = 0; k <= nl; k++) L.h_bwd_ptr[k] = n - hp[nl - k];
+        L.bwd_rows.alloc(n);
+        L.bwd_ptr.alloc((size_t)nl + 1);
+        k_sched_reverse<<<grid_for(std::max(n, nl + 1), BS, 4096), BS, 0, s>>>(n, nl, L.fwd_rows.p, L.fwd_ptr.p,
+                                                                              L.bwd_rows.p, L.bwd_ptr.p);
+        FVM_HIP(hipGetLastError());
     }
     L.runs_width = -1;
     L.sched_ready = true;

@@ -45,3 +45,27 @@ def test_packed_tail_is_bit_identical(case, prec, npost):
         res.append((ls.delta.copy(), a.history()))
     for d, h in res[1:]:
         assert np.array_equal(res[0][0], d) and np.array_equal(res[0][1], h)
+
+
+FLOW = {"chain300": lambda: matgen.chain(300, d=-2.1), "grid4": lambda: matgen.grid3d(4, seed=1),
+        "grid17": lambda: matgen.grid3d(17, seed=2, contrast=1.5), "grid24": lambda: matgen.grid3d(24, seed=3),
+        "ragged63": lambda: box_rows(63, 5), "ragged700": lambda: box_rows(700, 6),
+        "ragged3000": lambda: box_rows(3000, 7),
+        # one dependency level of more than 64 rows, rows without entries, a deep chain behind
+        "empty500": lambda: dict(matgen.chain(500), row=np.zeros(501, np.int32), col=np.zeros(0, np.int32),
+                                 off=np.zeros(0))}
+
+
+@pytest.mark.parametrize("prec,npost", [(0, 1), (1, 1), (0, 2)])
+@pytest.mark.parametrize("case", sorted(FLOW))
+def test_one_workgroup_reference_sweep_is_bit_identical(case, prec, npost):
+    """Reference-order sweeps by one workgroup against the level-by-level launches."""
+    m = FLOW[case]()
+    res = []
+    for flow in (0, 1):
+        a = gpu_amg(gsOrdering=0, precision=prec, nPostSweeps=npost, nMaxIterations=6, relativeTolerance=1e-30)
+        a.set_tuning("exact_flow", flow)
+        ls = ls_from(m)
+        a.solve(ls)
+        res.append((ls.delta.copy(), a.history()))
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
