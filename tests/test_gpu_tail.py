@@ -69,3 +69,26 @@ def test_one_workgroup_reference_sweep_is_bit_identical(case, prec, npost):
         a.solve(ls)
         res.append((ls.delta.copy(), a.history()))
     assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 127, 255, 256])
+def test_direct_level_inverse_at_panel_edges(n):
+    """The blocked inverse of the direct level, at the edges of its panels and at its limit."""
+    rng = np.random.default_rng(n)
+    m = matgen.chain(2 * n)
+    m["off"] = rng.uniform(0.2, 2.0, len(m["off"]))
+    sums = np.add.reduceat(m["off"], m["row"][:-1])
+    m["diag"] = -sums * rng.uniform(0.7, 1.5, 2 * n)          # not dominant everywhere: rows are pivoted
+    a = gpu_amg(gsOrdering=1, precision=1)
+    a.setup(ls_from(m))
+    d = a.direct_level(with_inverse=True)
+    assert d["level"] == 1 and d["n"] <= 256
+    L = a.level(1)
+    A = np.diag(L["diag"])
+    for i in range(d["n"]):
+        for p in range(L["row"][i], L["row"][i + 1]):
+            A[i, L["col"][p]] += L["off"][p]
+    ref = np.linalg.inv(A)
+    # backward error of elimination: n eps cond, and the growth of a few
+    bound = 20 * d["n"] * 2.3e-16 * np.linalg.cond(A)
+    assert np.abs(d["inv"] - ref).max() <= bound * np.abs(ref).max()
