@@ -2673,13 +2673,29 @@ __global__ void k_batch_mark(int n, int K, const int *off, const uint8_t *stoppe
         if (stopped[find_sys(off, K, i)]) bnd[i] = 1;
 }
 
+// smallest and largest group of every system. The rows of a wavefront mostly share their
+// system: it then takes one atomic, and none when the bounds already hold (an atomic per
+// row on K words took 1.26 ms for 800k rows of 32 systems, 12 times a setup)
 __global__ void k_batch_group_range(int n, int K, const int *off, const int *ci, int *gmin, int *gmax) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int I = ci[i];
-        if (I < 0) continue;
-        const int k = find_sys(off, K, i);
-        atomicMin(&gmin[k], I);
-        atomicMax(&gmax[k], I);
+    for (int i0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63; i0 < n; i0 += gridDim.x * blockDim.x) {
+        const int i = i0 + (threadIdx.x & 63);
+        const int I = i < n ? ci[i] : -1;
+        const int ka = find_sys(off, K, i0), kb = find_sys(off, K, min(i0 + 63, n - 1));
+        if (ka == kb) {
+            int lo = I < 0 ? INT_MAX : I, hi = I;
+            for (int o = 32; o > 0; o >>= 1) {
+                lo = min(lo, __shfl_xor(lo, o, 64));
+                hi = max(hi, __shfl_xor(hi, o, 64));
+            }
+            if ((threadIdx.x & 63) == 0 && hi >= 0) {
+                if (lo < gmin[ka]) atomicMin(&gmin[ka], lo);
+                if (hi > gmax[ka]) atomicMax(&gmax[ka], hi);
+            }
+        } else if (I >= 0) {
+            const int k = find_sys(off, K, i);
+            atomicMin(&gmin[k], I);
+            atomicMax(&gmax[k], I);
+        }
     }
 }
 
