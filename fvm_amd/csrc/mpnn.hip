@@ -88,11 +88,13 @@ __global__ void __launch_bounds__(BSZ) k_mp_logd_partial(int n, const double *di
     if (threadIdx.x == 0) { part[2 * blockIdx.x] = s; part[2 * blockIdx.x + 1] = s2; }
 }
 
-__global__ void k_mp_logd(int n, int nb, const double *diag, const double *part, float *l) {
+__global__ void __launch_bounds__(BSZ) k_mp_logd(int n, int nb, const double *diag, const double *part, float *l) {
     __shared__ double mean, sd;
+    double s = 0, s2 = 0;
+    for (int b = threadIdx.x; b < nb; b += BSZ) { s += part[2 * b]; s2 += part[2 * b + 1]; }
+    s = bsum<BSZ>(s);
+    s2 = bsum<BSZ>(s2);
     if (threadIdx.x == 0) {
-        double s = 0, s2 = 0;
-        for (int b = 0; b < nb; b++) { s += part[2 * b]; s2 += part[2 * b + 1]; }
         mean = s / n;
         double var = s2 / n - mean * mean;
         sd = sqrt(var > 0 ? var : 0.0) + 1e-12;
@@ -103,31 +105,31 @@ __global__ void k_mp_logd(int n, int nb, const double *diag, const double *part,
 }
 
 // ------------------------------------------------------------------ forward
-__global__ void __launch_bounds__(BSZ) k_mp_u(int n, const double *r, const double *diag, float *u, double *part) {
+// partial sums of u^2, u = -r / d
+__global__ void __launch_bounds__(BSZ) k_mp_u(int n, const double *r, const double *diag, double *part) {
     double s = 0;
     for (int i = blockIdx.x * BSZ + threadIdx.x; i < n; i += gridDim.x * BSZ) {
         const double ui = -r[i] / diag[i];
-        u[i] = (float)ui;
         s += ui * ui;
     }
     s = bsum<BSZ>(s);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ void k_mp_scale(int n, int nb, const double *part, double *s_out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0;
-        for (int b = 0; b < nb; b++) s += part[b];
-        *s_out = sqrt(s / (n > 0 ? n : 1)) + 1e-300;
-    }
+// one block: the partial sums side by side (one thread adding 1,024 of them took 51 us)
+__device__ double mp_total(int nb, const double *part) {
+    double s = 0;
+    for (int b = threadIdx.x; b < nb; b += BSZ) s += part[b];
+    return bsum<BSZ>(s);
+}
+__global__ void __launch_bounds__(BSZ) k_mp_scale(int n, int nb, const double *part, double *s_out) {
+    const double s = mp_total(nb, part);
+    if (threadIdx.x == 0) *s_out = sqrt(s / (n > 0 ? n : 1)) + 1e-300;
 }
 
-__global__ void k_mp_sum(int nb, const double *part, double *out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0;
-        for (int b = 0; b < nb; b++) s += part[b];
-        *out = s;
-    }
+__global__ void __launch_bounds__(BSZ) k_mp_sum2(int nb, const double *part, double *out) {
+    const double s0 = mp_total(nb, part), s1 = mp_total(nb, part + nb);
+    if (threadIdx.x == 0) { out[0] = s0; out[1] = s1; }
 }
 
 __global__ void k_mp_v(int n, const double *r, const double *diag, const double *s, float *v) {
@@ -136,133 +138,254 @@ __global__ void k_mp_v(int n, const double *r, const double *diag, const double 
         v[i] = (float)((-r[i] / diag[i]) * inv);
 }
 
-__global__ void k_mp_h0(int n, const int *row, const int *col, const float *c, const float *v, const float *l,
-                        uint16_t *h0) {
+// The input features that are not zero, packed: h0 = {v, C v, l, 0} in bf16 (8 bytes).
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// two values to bf16, nearest even: one v_cvt_pk_bf16_f32 (14 instructions as integers)
+__device__ __forceinline__ unsigned pack2(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+__global__ void k_mp_h0(int n, const int *__restrict__ row, const int *__restrict__ col, const float *__restrict__ c,
+                        const float *__restrict__ v, const float *__restrict__ l, uint2 *__restrict__ h0) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int rb = row[i], re = row[i + 1];
         float a = 0.f;
-        for (int p = row[i]; p < row[i + 1]; p++) a += c[p] * v[col[p]];
-        uint16_t *o = h0 + (size_t)i * MF0;
-        o[0] = f2bf(v[i]);
-        o[1] = f2bf(a);
-        o[2] = f2bf(l[i]);
-        for (int f = 3; f < MF0; f++) o[f] = 0;
+        for (int p = rb; p < re; p += 8) {   // eight entries in flight, added in order
+            int j[8];
+            float w[8], x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                j[u] = p + u < re ? col[p + u] : -1;
+                w[u] = p + u < re ? c[p + u] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = j[u] >= 0 ? v[j[u]] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (p + u < re) a = fmaf(w[u], x[u], a);
+        }
+        h0[i] = make_uint2(pack2(v[i], a), pack2(l[i], 0.f));
     }
 }
 
-// One layer for 64 nodes per workgroup (16 per wavefront):
-//   a_i = sum_p c_p h_col(p)   (FP32 sums, stored bf16 for the backward pass)
-//   h'_i = relu([h_i | a_i] W^T + b), W row o = [Ws(o,:) | Wn(o,:)] (bf16)
-// The 16 x 2FIN tile [h | a] of a wavefront is staged in LDS; the products run as
-// v_mfma_f32_16x16x32_bf16 over K = 2FIN in steps of 32, four 16-wide output blocks.
-// Operand layout of that instruction (lane l): A row l%16, k = 8(l/16)..+8;
-// B column l%16, same k; D rows 4(l/16)..+4, column l%16.
-template <int FIN>
-__global__ void __launch_bounds__(BSZ) k_mp_layer(int n, const int *row, const int *col, const float *c,
-                                                  const uint16_t *H, const uint16_t *W, const float *bias,
-                                                  uint16_t *Aout, uint16_t *Hn) {
-    constexpr int K2 = 2 * FIN;
-    constexpr int LDR = K2 + 8;   // padded LDS row (elements), keeps 16-byte alignment
-    constexpr int FQ = FIN / 4;   // features per lane in the gather (4 lanes per node)
-    __shared__ __attribute__((aligned(16))) uint16_t X[4][16 * LDR];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int node0 = (blockIdx.x * 4 + wave) * 16;
-    uint16_t *Xw = X[wave];
-    {
-        const int nl = lane >> 2, q = lane & 3;
-        const int i = node0 + nl;
-        float acc[FQ];
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float lo16(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float hi16(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+__device__ __forceinline__ void add8(float *acc, float w, u32x4 q) {
 #pragma unroll
-        for (int j = 0; j < FQ; j++) acc[j] = 0.f;
-        if (i < n) {
-            const uint16_t *hi = H + (size_t)i * FIN + q * FQ;
+    for (int k = 0; k < 4; k++) {
+        acc[2 * k] = fmaf(w, lo16(q[k]), acc[2 * k]);
+        acc[2 * k + 1] = fmaf(w, hi16(q[k]), acc[2 * k + 1]);
+    }
+}
+__device__ __forceinline__ u32x4 pack8(const float *a) {
+    u32x4 q;
 #pragma unroll
-            for (int j = 0; j < FQ; j++) Xw[nl * LDR + q * FQ + j] = hi[j];
-            for (int p = row[i]; p < row[i + 1]; p++) {
-                const float cp = c[p];
-                const uint16_t *hj = H + (size_t)col[p] * FIN + q * FQ;
-#pragma unroll
-                for (int j = 0; j < FQ; j++) acc[j] += cp * bf2f(hj[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < FQ; j++) {
-                const uint16_t a = f2bf(acc[j]);
-                Xw[nl * LDR + FIN + q * FQ + j] = a;
-                if (Aout) Aout[(size_t)i * FIN + q * FQ + j] = a;   // kept for the backward pass
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < FQ; j++) {
-                Xw[nl * LDR + q * FQ + j] = 0;
-                Xw[nl * LDR + FIN + q * FQ + j] = 0;
-            }
-        }
+    for (int k = 0; k < 4; k++) q[k] = pack2(a[2 * k], a[2 * k + 1]);
+    return q;
+}
+__device__ __forceinline__ bf16x8 frag(u32x4 q) { return __builtin_bit_cast(bf16x8, q); }
+
+// Tiles of 16 nodes, one per wavefront and step. Blocks are handed to the 8 XCDs in turn,
+// so block b works on eighth b % 8 of the tiles, and its blocks walk through that eighth
+// side by side: the nodes of a step are consecutive and the neighbours they gather stay in
+// that XCD's L2. At most 1,536 blocks (6 per CU stay resident); each loads its weights once.
+__host__ __device__ constexpr int mp_tiles(int n) { return (n + 15) / 16; }
+unsigned mp_grid(int n) { return std::min((unsigned)(mp_tiles(n) + 31) / 32, 192u) * 8u; }
+struct MpTiles {
+    int t, end, step;
+    __device__ explicit MpTiles(int n) {
+        const int T = mp_tiles(n), x = blockIdx.x & 7;
+        t = (int)((long long)T * x / 8) + (blockIdx.x >> 3) * 4 + (threadIdx.x >> 6);
+        end = (int)((long long)T * (x + 1) / 8);
+        step = (gridDim.x >> 3) * 4;
+    }
+};
+
+// One layer:  a_i = sum_p c_p h_col(p)  (FP32 sums, then bf16; kept for the backward pass)
+//             h'_i = relu([h_i | a_i] W^T + b), W row o = [Ws(o,:) | Wn(o,:)] (bf16)
+// The products run as v_mfma_f32_16x16x32_bf16 with the weights as the first operand (lane l:
+// output l%16, k = 8(l/16)..+8) and the nodes as the second (node l%16, same k), so lane l
+// gathers for node l%16 exactly the features that it feeds to the matrix cores, and ends
+// with four consecutive outputs of its node per output block (rows 4(l/16)..+4). The
+// weights lie in LDS in lane order (16 KB a block), which leaves registers for six
+// wavefronts per SIMD. LAST: the readout e = s (wo . h' + bo) is taken from the registers;
+// h' is stored only for a backward pass. What bounds it: the gathers, 128 bytes per entry.
+// 763,560 nodes (7-point rows): layer 64 -> 64 165 -> 129 us, the last one with its readout
+// 260 -> 120 us (146 and 110 MB from memory, 10 and 7 million L2 accesses), layer 0 68 -> 41 us.
+// Weights in registers over several tiles: 142 us (3 wavefronts per SIMD). Stores and
+// column reads that bypass the caches, or 96 blocks instead of 192 per XCD: slower.
+template <int FIN, bool LAST>
+__global__ void __launch_bounds__(BSZ, 6)
+k_mp_layer(int n, const int *__restrict__ row, const int *__restrict__ col, const float *__restrict__ c,
+           const void *__restrict__ Hv, const uint16_t *__restrict__ W, const float *__restrict__ bias, void *Aout,
+           uint16_t *Hn, const float *__restrict__ wo, const double *__restrict__ sc, double *e, int accumulate,
+           int *bad) {
+    constexpr int K2 = 2 * FIN, NK = K2 / 32;
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+    __shared__ u32x4 ws[4 * NK * 64];
+    __shared__ f32x4 bs[16], wos[16];
+    for (int t = threadIdx.x; t < 4 * NK * 64; t += BSZ) {
+        const int l = t & 63, ob = (t >> 6) / NK, kk = (t >> 6) % NK;
+        ws[t] = *reinterpret_cast<const u32x4 *>(W + (size_t)(ob * 16 + (l & 15)) * K2 + kk * 32 + (l >> 4) * 8);
+    }
+    if (threadIdx.x < MH) {
+        ((float *)bs)[threadIdx.x] = bias[threadIdx.x];
+        if (LAST) ((float *)wos)[threadIdx.x] = wo[threadIdx.x];
     }
     __syncthreads();
-    f32x4 d[4];
+    for (MpTiles T(n); T.t < T.end; T.t += T.step) {
+        asm volatile("" ::: "memory");   // the weights are read from LDS in each step, not kept in registers
+        const int node0 = T.t * 16;
+        const int i = node0 + r16, ic = min(i, n - 1);
+        const int rb = row[ic], re = row[ic + 1];
+        bf16x8 x[NK];
+        if constexpr (FIN == MF0) {
+            // three features: k 0..7 (lanes q = 0) hold h, k 16..23 (q = 2) hold a; the four
+            // lanes of a node share its entries
+            const uint2 *H = (const uint2 *)Hv;
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+            for (int p = rb + q; p < re; p += 8) {
+                const bool two = p + 4 < re;
+                const int j0 = col[p], j1 = two ? col[p + 4] : j0;
+                const float w0 = c[p], w1 = two ? c[p + 4] : 0.f;
+                const uint2 h0 = H[j0], h1 = H[j1];
+                a0 = fmaf(w0, lo16(h0.x), a0);
+                a1 = fmaf(w0, hi16(h0.x), a1);
+                a2 = fmaf(w0, lo16(h0.y), a2);
+                if (two) {
+                    a0 = fmaf(w1, lo16(h1.x), a0);
+                    a1 = fmaf(w1, hi16(h1.x), a1);
+                    a2 = fmaf(w1, lo16(h1.y), a2);
+                }
+            }
+            for (int o = 16; o < 64; o <<= 1) {
+                a0 += __shfl_xor(a0, o, 64);
+                a1 += __shfl_xor(a1, o, 64);
+                a2 += __shfl_xor(a2, o, 64);
+            }
+            const uint2 hi = H[ic], ai = make_uint2(pack2(a0, a1), pack2(a2, 0.f));
+            if (Aout && q == 2 && i < n) ((uint2 *)Aout)[i] = ai;
+            const u32x4 z = {q == 0 ? hi.x : q == 2 ? ai.x : 0u, q == 0 ? hi.y : q == 2 ? ai.y : 0u, 0u, 0u};
+            x[0] = frag(z);
+        } else {
+            const u32x4 *H = (const u32x4 *)Hv;   // eight features; node i holds 8 i .. 8 i + 7
+            float a[16];
 #pragma unroll
-    for (int ob = 0; ob < 4; ob++) d[ob] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const int r16 = lane & 15, kq = (lane >> 4) * 8;
+            for (int k = 0; k < 16; k++) a[k] = 0.f;
+            for (int p = rb; p < re; p += 4) {   // four entries in flight, added in order
+                int j[4];
+                float wt[4];
+                u32x4 g[4][2];
 #pragma unroll
-    for (int kk = 0; kk < K2; kk += 32) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(Xw + r16 * LDR + kk + kq);
+                for (int u = 0; u < 4; u++) {
+                    j[u] = p + u < re ? col[p + u] : ic;
+                    wt[u] = p + u < re ? c[p + u] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    g[u][0] = H[(size_t)j[u] * 8 + q];
+                    g[u][1] = H[(size_t)j[u] * 8 + 4 + q];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (p + u < re) {
+                        add8(a, wt[u], g[u][0]);
+                        add8(a + 8, wt[u], g[u][1]);
+                    }
+            }
+            const u32x4 b0 = pack8(a), b1 = pack8(a + 8);
+            if (Aout && i < n) {
+                ((u32x4 *)Aout)[(size_t)i * 8 + q] = b0;
+                ((u32x4 *)Aout)[(size_t)i * 8 + 4 + q] = b1;
+            }
+            x[0] = frag(H[(size_t)ic * 8 + q]);
+            x[1] = frag(H[(size_t)ic * 8 + 4 + q]);
+            x[2] = frag(b0);
+            x[3] = frag(b1);
+        }
+        float y = 0.f;
 #pragma unroll
         for (int ob = 0; ob < 4; ob++) {
-            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(W + (size_t)(ob * 16 + r16) * K2 + kk + kq);
-            d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, d[ob], 0, 0, 0);
-        }
-    }
+            f32x4 d = bs[ob * 4 + q];
 #pragma unroll
-    for (int ob = 0; ob < 4; ob++) {
-        const int o = ob * 16 + r16;
-        const float bo = bias[o];
+            for (int kk = 0; kk < NK; kk++)
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(ws[(ob * NK + kk) * 64 + lane]), x[kk], d, 0, 0, 0);
+            float h[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int node = node0 + (lane >> 4) * 4 + t;
-            if (node < n) {
-                const float z = d[ob][t] + bo;
-                Hn[(size_t)node * MH + o] = f2bf(z > 0.f ? z : 0.f);
+            for (int t = 0; t < 4; t++) h[t] = d[t] > 0.f ? d[t] : 0.f;
+            const uint2 st = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+            if (Hn && i < n) *reinterpret_cast<uint2 *>(Hn + (size_t)i * MH + ob * 16 + 4 * q) = st;
+            if (LAST) {
+                const f32x4 wr = wos[ob * 4 + q];
+                y += wr[0] * lo16(st.x) + wr[1] * hi16(st.x) + wr[2] * lo16(st.y) + wr[3] * hi16(st.y);
             }
         }
-    }
-}
-
-// e = s (wo . h3 + bo); accumulate: e += that
-__global__ void k_mp_readout(int n, const uint16_t *h3, const float *wo, const float *bo, const double *s,
-                             double *e, int accumulate, int *bad) {
-    __shared__ float w[MH];
-    if (threadIdx.x < MH) w[threadIdx.x] = wo[threadIdx.x];
-    __syncthreads();
-    const double sc = *s;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float y = bo[0];
-        const uint16_t *hi = h3 + (size_t)i * MH;
-        for (int o = 0; o < MH; o++) y += w[o] * bf2f(hi[o]);
-        const double ei = sc * (double)y;
-        if (!isfinite(ei)) atomicOr(bad, 1);
-        e[i] = accumulate ? e[i] + ei : ei;
+        if (LAST) {
+            y += __shfl_xor(y, 16, 64);
+            y += __shfl_xor(y, 32, 64);
+            if (q == 0 && i < n) {
+                const double ei = *sc * (double)(y + wo[MH]);
+                if (!isfinite(ei)) atomicOr(bad, 1);
+                e[i] = accumulate ? e[i] + ei : ei;
+            }
+        }
     }
 }
 
 // ------------------------------------------------------------------ loss and backward
-// y = add + alpha A x (add may be null)
+// y = A x
 __global__ void k_mp_spmv(int n, const int *row, const int *col, const double *off, const double *diag,
-                          const double *x, const double *add, double alpha, double *y) {
+                          const double *x, double *y) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         double s = diag[i] * x[i];
         for (int p = row[i]; p < row[i + 1]; p++) s += off[p] * x[col[p]];
-        y[i] = add ? add[i] + alpha * s : alpha * s;
+        y[i] = s;
     }
 }
 
-__global__ void k_mp_sub(int n, const double *a, const double *b, double *y) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) y[i] = a[i] - b[i];
+// The loss against a known correction et, in one pass: t = e - et, At = -A t and the partial
+// sums of et^T (-A et) (part[b]) and t^T (-A t) (part[nb + b])
+__global__ void __launch_bounds__(BSZ) k_mp_loss_pair(int n, const int *__restrict__ row, const int *__restrict__ col,
+                                                      const double *__restrict__ off, const double *__restrict__ diag,
+                                                      const double *__restrict__ e, const double *__restrict__ et,
+                                                      double *__restrict__ At, double *__restrict__ part) {
+    double den = 0, num = 0;
+    for (int i = blockIdx.x * BSZ + threadIdx.x; i < n; i += gridDim.x * BSZ) {
+        const double xi = et[i], ti = e[i] - xi, d = diag[i];
+        double s = d * ti, x = d * xi;
+        for (int p = row[i]; p < row[i + 1]; p++) {
+            const int j = col[p];
+            const double w = off[p], xj = et[j];
+            s += w * (e[j] - xj);
+            x += w * xj;
+        }
+        At[i] = -s;
+        den += xi * -x;
+        num += ti * -s;
+    }
+    den = bsum<BSZ>(den);
+    num = bsum<BSZ>(num);
+    if (threadIdx.x == 0) { part[blockIdx.x] = den; part[gridDim.x + blockIdx.x] = num; }
 }
 
-__global__ void __launch_bounds__(BSZ) k_mp_dot_partial(int n, const double *a, const double *b, double *part) {
-    double s = 0;
-    for (int i = blockIdx.x * BSZ + threadIdx.x; i < n; i += gridDim.x * BSZ) s += a[i] * b[i];
-    s = bsum<BSZ>(s);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+// The residual loss: t = r + A e and the partial sums of r^2 and t^2
+__global__ void __launch_bounds__(BSZ) k_mp_loss_res(int n, const int *__restrict__ row, const int *__restrict__ col,
+                                                     const double *__restrict__ off, const double *__restrict__ diag,
+                                                     const double *__restrict__ e, const double *__restrict__ r,
+                                                     double *__restrict__ t, double *__restrict__ part) {
+    double den = 0, num = 0;
+    for (int i = blockIdx.x * BSZ + threadIdx.x; i < n; i += gridDim.x * BSZ) {
+        double s = diag[i] * e[i];
+        for (int p = row[i]; p < row[i + 1]; p++) s += off[p] * e[col[p]];
+        const double ri = r[i], ti = ri + s;
+        t[i] = ti;
+        den += ri * ri;
+        num += ti * ti;
+    }
+    den = bsum<BSZ>(den);
+    num = bsum<BSZ>(num);
+    if (threadIdx.x == 0) { part[blockIdx.x] = den; part[gridDim.x + blockIdx.x] = num; }
 }
 
 // dy_i = s * 2 (A t)_i / ||r||^2
@@ -271,120 +394,252 @@ __global__ void k_mp_dy(int n, const double *At, const double *s, const double *
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dy[i] = (float)(f * At[i]);
 }
 
-// dH3[i][o] = dy_i wo[o]; partial sums of dy_i h3[i][o] and dy_i per block of 256 nodes
-__global__ void __launch_bounds__(BSZ) k_mp_out_bwd(int n, const float *dy, const uint16_t *h3, const float *wo,
-                                                    float *dH, float *part) {
-    __shared__ float acc[4][MH + 1];
-    const int o = threadIdx.x & 63, g = threadIdx.x >> 6;
-    float s = 0.f, sb = 0.f;
-    const float w = wo[o];
-    for (int k = g; k < BSZ; k += 4) {
-        const int i = blockIdx.x * BSZ + k;
-        if (i >= n) break;
-        const float d = dy[i];
-        dH[(size_t)i * MH + o] = d * w;
-        s += d * bf2f(h3[(size_t)i * MH + o]);
-        sb += d;
-    }
-    acc[g][o] = s;
-    if (o == 0) acc[g][MH] = sb;
-    __syncthreads();
-    if (g == 0) {
-        part[(size_t)blockIdx.x * (MH + 1) + o] = acc[0][o] + acc[1][o] + acc[2][o] + acc[3][o];
-        if (o == 0) part[(size_t)blockIdx.x * (MH + 1) + MH] = acc[0][MH] + acc[1][MH] + acc[2][MH] + acc[3][MH];
-    }
-}
-
-// Weight gradients of layer k over a block of 64 nodes (delta = dH' * [h' > 0]):
-// part[blk][o][f] = sum_i delta[i][o] x_i[f] with x_i = [h_i | a_i], part[blk][64*2FIN + o] = sum_i delta[i][o]
-template <int FIN>
-__global__ void __launch_bounds__(BSZ) k_mp_wgrad(int n, const float *dH, const uint16_t *Hn, const uint16_t *H,
-                                                  const uint16_t *A, float *part) {
-    constexpr int K2 = 2 * FIN;
-    constexpr int NB = 64;
-    __shared__ float D[NB][MH + 1];
-    __shared__ float Xs[NB][K2 + 1];
-    const int i0 = blockIdx.x * NB;
-    for (int t = threadIdx.x; t < NB * MH; t += BSZ) {
-        const int k = t / MH, o = t % MH, i = i0 + k;
-        float d = 0.f;
-        if (i < n) d = bf2f(Hn[(size_t)i * MH + o]) > 0.f ? dH[(size_t)i * MH + o] : 0.f;
-        D[k][o] = d;
-    }
-    for (int t = threadIdx.x; t < NB * K2; t += BSZ) {
-        const int k = t / K2, f = t % K2, i = i0 + k;
-        float x = 0.f;
-        if (i < n) x = f < FIN ? bf2f(H[(size_t)i * FIN + f]) : bf2f(A[(size_t)i * FIN + f - FIN]);
-        Xs[k][f] = x;
+// Backward through layer k (k > 0), with delta_k+1 = dL/dh_k+1 * [h_k+1 > 0]:
+//   g_i = sum over entries q of row i of ct_q delta_k+1(col q)
+//   delta_k(i) = (delta_k+1(i) Ws + g_i Wn) * [h_k(i) > 0]
+// (aggregating delta and not delta Wn: one pass, nothing between). All in FP32: the products
+// are v_mfma_f32_16x16x4f32 with the weights' columns as the first operand and the nodes as
+// the second; step 4v + u of lane l is feature 16 v + 4 (l/16) + u of node l%16, so the four
+// lanes of a node read 64 consecutive bytes at a time. The weights lie in LDS as FP32 in
+// lane order (32 KB a block). TOP: delta_3(j) = dy_j wo [h_3(j) > 0] is formed from dy and
+// the bf16 h_3 where it is gathered. What bounds it: the gathers, and at 34,720 nodes its
+// 8 wavefronts per CU.
+// 34,720 nodes: 98 -> 22 us per layer (products per node and feature on the vector units and
+// an aggregation of delta Wn, 390 MB a layer at 763,560 nodes, before).
+template <bool TOP>
+__global__ void __launch_bounds__(BSZ, 4)
+k_mp_bwd(int n, const int *__restrict__ row, const int *__restrict__ col, const float *__restrict__ ct,
+         const float *__restrict__ D, const uint16_t *__restrict__ Hn, const float *__restrict__ wo,
+         const uint16_t *__restrict__ W, const uint16_t *__restrict__ H, float *__restrict__ Dk) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+    __shared__ f32x4 ws[2 * 4 * 4 * 64];   // [part][output block][v][lane], component u
+    for (int t = threadIdx.x; t < 2 * 4 * 4 * 64; t += BSZ) {
+        const int l = t & 63, v = (t >> 6) & 3, fb = (t >> 8) & 3, part = t >> 10;
+        f32x4 w;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            w[u] = bf2f(W[(size_t)(16 * v + 4 * (l >> 4) + u) * (2 * MH) + part * MH + 16 * fb + (l & 15)]);
+        ws[t] = w;
     }
     __syncthreads();
-    float *pb = part + (size_t)blockIdx.x * (MH * K2 + MH);
-    for (int t = threadIdx.x; t < MH * K2; t += BSZ) {
-        const int o = t / K2, f = t % K2;
-        float s = 0.f;
-        for (int k = 0; k < NB; k++) s += D[k][o] * Xs[k][f];
-        pb[t] = s;
-    }
-    for (int o = threadIdx.x; o < MH; o += BSZ) {
-        float s = 0.f;
-        for (int k = 0; k < NB; k++) s += D[k][o];
-        pb[MH * K2 + o] = s;
-    }
-}
-
-// G[i][f] = sum_o delta[i][o] Wn[o][f], P[i][f] = sum_o delta[i][o] Ws[o][f]
-template <int FIN>
-__global__ void k_mp_bwd_gp(int n, const float *dH, const uint16_t *Hn, const uint16_t *W, float *G, float *P) {
-    constexpr int K2 = 2 * FIN;
-    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < (long long)n * FIN;
-         t += (long long)gridDim.x * blockDim.x) {
-        const int i = (int)(t / FIN), f = (int)(t % FIN);
-        float g = 0.f, pv = 0.f;
-        for (int o = 0; o < MH; o++) {
-            const float d = bf2f(Hn[(size_t)i * MH + o]) > 0.f ? dH[(size_t)i * MH + o] : 0.f;
-            pv += d * bf2f(W[(size_t)o * K2 + f]);
-            g += d * bf2f(W[(size_t)o * K2 + FIN + f]);
+    for (MpTiles T(n); T.t < T.end; T.t += T.step) {
+        asm volatile("" ::: "memory");   // the weights are read from LDS in each step, not kept in registers
+        const int i = T.t * 16 + r16, ic = min(i, n - 1);
+        const int rb = row[ic], re = row[ic + 1];
+        f32x4 x[2][4];
+        // features of node j as multiples of wt (TOP: without the factor wo)
+        auto gather = [&](f32x4 *acc, int j, float wt) {
+            if constexpr (TOP) {
+                const uint2 *h = (const uint2 *)(Hn + (size_t)j * MH) + q;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const uint2 hv = h[4 * v];
+                    acc[v][0] += lo16(hv.x) > 0.f ? wt : 0.f;
+                    acc[v][1] += hi16(hv.x) > 0.f ? wt : 0.f;
+                    acc[v][2] += lo16(hv.y) > 0.f ? wt : 0.f;
+                    acc[v][3] += hi16(hv.y) > 0.f ? wt : 0.f;
+                }
+            } else {
+                const f32x4 *d = (const f32x4 *)(D + (size_t)j * MH) + q;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const f32x4 dv = d[4 * v];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) acc[v][u] = fmaf(wt, dv[u], acc[v][u]);
+                }
+            }
+        };
+#pragma unroll
+        for (int v = 0; v < 4; v++) x[0][v] = x[1][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+        gather(x[0], ic, TOP ? D[ic] : 1.f);
+        for (int p = rb; p < re; p += 2) {
+            const bool two = p + 1 < re;
+            const int j0 = col[p], j1 = two ? col[p + 1] : j0;
+            float w0 = ct[p], w1 = two ? ct[p + 1] : 0.f;
+            if (TOP) {
+                w0 *= D[j0];
+                w1 *= D[j1];
+            }
+            gather(x[1], j0, w0);
+            if (two) gather(x[1], j1, w1);
         }
-        G[t] = g;
-        P[t] = pv;
+        if constexpr (TOP) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const float w = wo[16 * v + 4 * q + u];
+                    x[0][v][u] *= w;
+                    x[1][v][u] *= w;
+                }
+        }
+        f32x4 d[4];
+#pragma unroll
+        for (int fb = 0; fb < 4; fb++) d[fb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int part = 0; part < 2; part++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int fb = 0; fb < 4; fb++) {   // four independent sums in turn
+                    const f32x4 w = ws[((part * 4 + fb) * 4 + v) * 64 + lane];
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+                        d[fb] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u], x[part][v][u], d[fb], 0, 0, 0);
+                }
+        if (i < n) {
+#pragma unroll
+            for (int fb = 0; fb < 4; fb++) {
+                const uint2 h = *reinterpret_cast<const uint2 *>(H + (size_t)i * MH + 16 * fb + 4 * q);
+                f32x4 o;
+                o[0] = lo16(h.x) > 0.f ? d[fb][0] : 0.f;
+                o[1] = hi16(h.x) > 0.f ? d[fb][1] : 0.f;
+                o[2] = lo16(h.y) > 0.f ? d[fb][2] : 0.f;
+                o[3] = hi16(h.y) > 0.f ? d[fb][3] : 0.f;
+                *reinterpret_cast<f32x4 *>(Dk + (size_t)i * MH + 16 * fb + 4 * q) = o;
+            }
+        }
     }
 }
 
-// dH_k[i][f] = P[i][f] + sum over entries q of row i of ct[q] G[col q][f]
-template <int FIN>
-__global__ void k_mp_bwd_agg(int n, const int *row, const int *col, const float *ct, const float *G,
-                             const float *P, float *dH) {
-    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < (long long)n * FIN;
-         t += (long long)gridDim.x * blockDim.x) {
-        const int i = (int)(t / FIN), f = (int)(t % FIN);
-        float s = P[t];
-        for (int q = row[i]; q < row[i + 1]; q++) s += ct[q] * G[(size_t)col[q] * FIN + f];
-        dH[t] = s;
+// Weight gradients of all layers and of the readout, one launch: blockIdx.y = layer,
+// blockIdx.x = a run of consecutive nodes, whose sums go to part[blockIdx.x].
+//   dW_k[o][f] = sum_i delta_k+1(i)[o] x_i[f], x_i = [h_k(i) | a_k(i)];  db_k[o] = sum_i delta_k+1(i)[o]
+//   dwo[o] = sum_i dy_i h_3(i)[o];  dbo = sum_i dy_i
+// FP32 v_mfma_f32_16x16x4f32, four nodes per step (node l/16 of lane l). Row r of the output
+// tile of wavefront w is o = 4 r + w, column r of tile fb is feature 4 r + fb of h (fb < 4) or
+// of a, so that each lane reads 16 bytes of delta and 8 bytes each of h and a, whole rows
+// across 16 lanes. A run's sums stay in registers and are written as they lie there.
+// What bounds it: the matrix cores' FP32 rate.
+// 34,720 nodes, three layers and readout: 147 us -> 33 us, and their reduction 422 -> 7 us
+// (543 partial blocks of 33 KB per layer, added by one thread per value, before). Both the
+// runs' sums (n / 256 terms) and their total in FP64 are shorter chains than 64 + n / 64.
+constexpr int WG_W = 4 * 8 * 4 * 64, WG_W0 = 4 * 1 * 4 * 64;   // values of a layer, of layer 0
+constexpr int WG_L = WG_W + MH;
+constexpr int WG_O0 = 2 * WG_L, WG_OWO = WG_O0 + WG_W0 + MH, WG_S = WG_OWO + MH + 1;
+constexpr int WG_MAX = 256;     // runs per layer: 3 x 256 blocks, 18 MB of partial sums
+unsigned mp_runs(int n) { return (unsigned)std::min((n + 127) / 128, WG_MAX); }
+
+template <int K>
+__device__ void mp_wgrad_run(int n, int w, const float *__restrict__ dy, const float *__restrict__ D,
+                             const uint16_t *__restrict__ Hn, const float *__restrict__ wo,
+                             const uint16_t *__restrict__ H, const uint16_t *__restrict__ A, float *__restrict__ pw,
+                             float *__restrict__ pb, float *__restrict__ po) {
+    constexpr bool TOP = K == MLAYERS - 1;
+    constexpr int NF = K == 0 ? 1 : 8;
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+    const int steps = (n + 3) / 4;
+    const int s0 = (int)((long long)steps * blockIdx.x / gridDim.x);
+    const int s1 = (int)((long long)steps * (blockIdx.x + 1) / gridDim.x);
+    f32x4 acc[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float db = 0.f, dwo = 0.f, dbo = 0.f;
+    const float wow = TOP ? wo[4 * r16 + w] : 0.f;
+    for (int s = s0; s < s1; s += 4) {
+        float d[4], hn[4], y[4];
+        uint2 h[4], a[4];
+        uint16_t x0[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {   // clamped loads; a node outside the run gets delta = 0
+            const int i = min(4 * (s + u) + q, n - 1);
+            const bool in = s + u < s1 && 4 * (s + u) + q < n;
+            if constexpr (TOP) {
+                y[u] = in ? dy[i] : 0.f;
+                hn[u] = bf2f(Hn[(size_t)i * MH + 4 * r16 + w]);
+                d[u] = hn[u] > 0.f ? y[u] * wow : 0.f;
+            } else {
+                d[u] = D[(size_t)i * MH + 4 * r16 + w];
+                d[u] = in ? d[u] : 0.f;
+            }
+            if constexpr (K == 0) {
+                x0[u] = (r16 & 4 ? A : H)[(size_t)i * 4 + (r16 & 3)];
+            } else {
+                h[u] = *reinterpret_cast<const uint2 *>(H + (size_t)i * MH + 4 * r16);
+                a[u] = *reinterpret_cast<const uint2 *>(A + (size_t)i * MH + 4 * r16);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            db += d[u];
+            if constexpr (TOP) {
+                dwo = fmaf(y[u], hn[u], dwo);
+                dbo += y[u];
+            }
+            if constexpr (K == 0) {
+                const float x = r16 < 8 ? bf2f(x0[u]) : 0.f;
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[u], x, acc[0], 0, 0, 0);
+            } else {
+                const float x[8] = {lo16(h[u].x), hi16(h[u].x), lo16(h[u].y), hi16(h[u].y),
+                                    lo16(a[u].x), hi16(a[u].x), lo16(a[u].y), hi16(a[u].y)};
+#pragma unroll
+                for (int f = 0; f < 8; f++) acc[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[u], x[f], acc[f], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) pw[((w * NF + f) * 4 + t) * 64 + lane] = acc[f][t];
+    for (int o = 16; o < 64; o <<= 1) {
+        db += __shfl_xor(db, o, 64);
+        if constexpr (TOP) {
+            dwo += __shfl_xor(dwo, o, 64);
+            dbo += __shfl_xor(dbo, o, 64);
+        }
+    }
+    if (q == 0) {
+        pb[4 * r16 + w] = db;
+        if constexpr (TOP) {
+            po[4 * r16 + w] = dwo;
+            if (r16 == 0 && w == 0) po[MH] = dbo;
+        }
     }
 }
 
-// dst[off + j] (+)= sum over blocks of part[blk * stride + j], blocks in order
-__global__ void k_mp_reduce(int nblk, int m, int stride, const float *part, float *dst) {
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < m; j += gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; b++) s += part[(size_t)b * stride + j];
-        dst[j] += s;
-    }
+__global__ void __launch_bounds__(BSZ)
+k_mp_wgrad(int n, const float *dy, const float *D2, const float *D1, const uint16_t *H3, const uint16_t *H2,
+           const uint16_t *H1, const uint16_t *H0, const uint16_t *A2, const uint16_t *A1, const uint16_t *A0,
+           const float *wo, float *part) {
+    const int w = threadIdx.x >> 6;
+    float *p = part + (size_t)blockIdx.x * WG_S;
+    if (blockIdx.y == 0)
+        mp_wgrad_run<2>(n, w, dy, nullptr, H3, wo, H2, A2, p, p + WG_W, p + WG_OWO);
+    else if (blockIdx.y == 1)
+        mp_wgrad_run<1>(n, w, nullptr, D2, nullptr, nullptr, H1, A1, p + WG_L, p + WG_L + WG_W, nullptr);
+    else
+        mp_wgrad_run<0>(n, w, nullptr, D1, nullptr, nullptr, H0, A0, p + WG_O0, p + WG_O0 + WG_W0, nullptr);
 }
 
-// layer gradient block [o][2FIN] + b[o] -> packed Ws (64 x FIN), Wn (64 x FIN), b (64)
-template <int FIN>
-__global__ void k_mp_scatter_wgrad(const float *g, float *grad_layer) {
-    constexpr int K2 = 2 * FIN;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < MH * K2 + MH; t += gridDim.x * blockDim.x) {
-        if (t < MH * K2) {
-            const int o = t / K2, f = t % K2;
-            if (f < FIN) grad_layer[o * FIN + f] += g[t];
-            else grad_layer[MH * FIN + o * FIN + (f - FIN)] += g[t];
+// grad += the runs' sums, added in FP64: 64 values by 4 threads each in a block
+__global__ void __launch_bounds__(BSZ) k_mp_reduce(int nrun, const float *__restrict__ part, float *grad) {
+    __shared__ double sh[4][64];
+    const int g = threadIdx.x >> 6, v = threadIdx.x & 63, j = blockIdx.x * 64 + v;
+    double s = 0;
+    if (j < WG_S) {
+#pragma unroll 8
+        for (int b = g; b < nrun; b += 4) s += part[(size_t)b * WG_S + j];
+    }
+    sh[g][v] = s;
+    __syncthreads();
+    if (g != 0 || j >= WG_S) return;
+    int dst = -1;
+    if (j >= WG_OWO) {
+        dst = WO_OFF + j - WG_OWO;
+    } else {
+        const int k = j < WG_L ? 2 : j < WG_O0 ? 1 : 0;
+        const int jj = j - (k == 2 ? 0 : k == 1 ? WG_L : WG_O0), nw = k ? WG_W : WG_W0;
+        const int fin = k ? MH : MF0, nf = k ? 8 : 1;
+        if (jj >= nw) {
+            dst = layer_off(k) + 2 * MH * fin + jj - nw;
         } else {
-            grad_layer[2 * MH * FIN + (t - MH * K2)] += g[t];
+            const int lane = jj & 63, t = (jj >> 6) & 3, fb = (jj >> 8) % nf, w = (jj >> 8) / nf;
+            const int o = 4 * (4 * (lane >> 4) + t) + w, r = lane & 15;
+            if (k) dst = layer_off(k) + (fb < 4 ? 0 : MH * MH) + o * MH + 4 * r + (fb & 3);
+            else if (r < 8) dst = layer_off(0) + (r < 4 ? 0 : MH * MF0) + o * MF0 + (r & 3);
         }
     }
+    if (dst >= 0) grad[dst] += (float)((sh[0][v] + sh[1][v]) + (sh[2][v] + sh[3][v]));
 }
 
 __global__ void k_mp_adam(int np, float *theta, float *grad, float *m, float *v, float lr, float b1, float b2,
@@ -447,9 +702,10 @@ struct fvm_mpnn {
     const double *off = nullptr, *diag = nullptr;
     DArr<float> c, ct, l;
     // activations and work
+    // layer inputs and aggregates; those of layer 0 hold its four packed features per node
     DArr<uint16_t> H[fvm::MLAYERS + 1], A[fvm::MLAYERS];
-    DArr<float> v, dy, dH, dH2, G, P, part;
-    DArr<double> s, rr, e, t, At, dpart, tmp_a, tmp_b;
+    DArr<float> v, dy, D1, D2, part;
+    DArr<double> s, rr, e, t, At, dpart, tmp_b;
     DArr<int> flag;
 };
 
@@ -469,9 +725,9 @@ struct MpScope {
 void mp_alloc_acts(fvm_mpnn *m) {
     const size_t n = std::max(m->n, 1);
     const size_t nb = (n + BSZ - 1) / BSZ;
-    m->H[0].ensure(n * MF0);
+    m->H[0].ensure(n * 4);
     for (int k = 1; k <= MLAYERS; k++) m->H[k].ensure(n * MH);
-    m->A[0].ensure(n * MF0);
+    m->A[0].ensure(n * 4);
     for (int k = 1; k < MLAYERS; k++) m->A[k].ensure(n * MH);
     m->v.ensure(n);
     m->s.ensure(4);
@@ -487,24 +743,24 @@ void mp_forward(fvm_mpnn *m, const double *r, double *e_out, int accumulate, boo
     const int n = m->n;
     mp_alloc_acts(m);
     const unsigned nb = grid_for(n, BSZ, 1024);
-    k_mp_u<<<nb, BSZ, 0, st>>>(n, r, m->diag, m->v.p, m->dpart.p);
-    k_mp_scale<<<1, 64, 0, st>>>(n, (int)nb, m->dpart.p, m->s.p);
+    k_mp_u<<<nb, BSZ, 0, st>>>(n, r, m->diag, m->dpart.p);
+    k_mp_scale<<<1, BSZ, 0, st>>>(n, (int)nb, m->dpart.p, m->s.p);
     k_mp_v<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, r, m->diag, m->s.p, m->v.p);
-    k_mp_h0<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->v.p, m->l.p, m->H[0].p);
-    const unsigned gl = (unsigned)((n + 63) / 64);
+    k_mp_h0<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->v.p, m->l.p, (uint2 *)m->H[0].p);
+    FVM_HIP(hipMemsetAsync(m->flag.p, 0, sizeof(int), st));
+    const unsigned gl = mp_grid(n);
     for (int k = 0; k < MLAYERS; k++) {
         const float *bias = m->theta.p + layer_off(k) + 2 * MH * fin_of(k);
-        uint16_t *aout = keep ? m->A[k].p : nullptr;
-        if (k == 0)
-            k_mp_layer<MF0><<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->H[0].p, m->wbf[0].p, bias, aout,
-                                               m->H[1].p);
-        else
-            k_mp_layer<MH><<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->H[k].p, m->wbf[k].p, bias, aout,
-                                              m->H[k + 1].p);
+        const bool last = k == MLAYERS - 1;
+        auto launch = [&](auto kern) {
+            kern<<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->H[k].p, m->wbf[k].p, bias,
+                                     keep ? m->A[k].p : nullptr, (!last || keep) ? m->H[k + 1].p : nullptr,
+                                     m->theta.p + WO_OFF, m->s.p, e_out, accumulate, m->flag.p);
+        };
+        if (k == 0) launch(k_mp_layer<MF0, false>);
+        else if (!last) launch(k_mp_layer<MH, false>);
+        else launch(k_mp_layer<MH, true>);
     }
-    FVM_HIP(hipMemsetAsync(m->flag.p, 0, sizeof(int), st));
-    k_mp_readout<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, m->H[MLAYERS].p, m->theta.p + WO_OFF,
-                                                   m->theta.p + WO_OFF + MH, m->s.p, e_out, accumulate, m->flag.p);
     FVM_HIP(hipGetLastError());
 }
 
@@ -516,59 +772,30 @@ double mp_loss_grad(fvm_mpnn *m, const double *r, const double *et) {
     mp_alloc_acts(m);
     const size_t nn = std::max(n, 1);
     m->e.ensure(nn); m->t.ensure(nn); m->At.ensure(nn);
-    m->dy.ensure(nn); m->dH.ensure(nn * MH); m->dH2.ensure(nn * MH);
-    m->G.ensure(nn * MH); m->P.ensure(nn * MH);
+    const unsigned runs = mp_runs(n);
+    m->dy.ensure(nn); m->D1.ensure(nn * MH); m->D2.ensure(nn * MH);
+    m->part.ensure((size_t)runs * WG_S);
     mp_forward(m, r, m->e.p, 0, true);
     const unsigned gs = grid_for(n, BSZ);
     const unsigned nb = grid_for(n, BSZ, 1024);
     // rr[0] = denominator, rr[1] = numerator; At = d(numerator)/de / 2
-    if (!et) {
-        // t = r + A e ; At = A t (A symmetric)
-        k_mp_spmv<<<gs, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->e.p, r, 1.0, m->t.p);
-        k_mp_spmv<<<gs, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->t.p, nullptr, 1.0, m->At.p);
-        k_mp_dot_partial<<<nb, BSZ, 0, st>>>(n, r, r, m->dpart.p);
-        k_mp_dot_partial<<<nb, BSZ, 0, st>>>(n, m->t.p, m->t.p, m->dpart.p + nb);
+    if (!et) {   // t = r + A e ; At = A t (A symmetric)
+        k_mp_loss_res<<<nb, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->e.p, r, m->t.p, m->dpart.p);
+        k_mp_spmv<<<gs, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->t.p, m->At.p);
     } else {
-        // t = e - et ; At = -A t ; den = et^T (-A et) (the -A et product goes to e, no longer needed)
-        k_mp_sub<<<gs, BSZ, 0, st>>>(n, m->e.p, et, m->t.p);
-        k_mp_spmv<<<gs, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->t.p, nullptr, -1.0, m->At.p);
-        k_mp_spmv<<<gs, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, et, nullptr, -1.0, m->e.p);
-        k_mp_dot_partial<<<nb, BSZ, 0, st>>>(n, et, m->e.p, m->dpart.p);
-        k_mp_dot_partial<<<nb, BSZ, 0, st>>>(n, m->t.p, m->At.p, m->dpart.p + nb);
+        k_mp_loss_pair<<<nb, BSZ, 0, st>>>(n, m->row, m->col, m->off, m->diag, m->e.p, et, m->At.p, m->dpart.p);
     }
-    k_mp_sum<<<1, 64, 0, st>>>((int)nb, m->dpart.p, m->rr.p);
-    k_mp_sum<<<1, 64, 0, st>>>((int)nb, m->dpart.p + nb, m->rr.p + 1);
+    k_mp_sum2<<<1, BSZ, 0, st>>>((int)nb, m->dpart.p, m->rr.p);
     k_mp_dy<<<gs, BSZ, 0, st>>>(n, m->At.p, m->s.p, m->rr.p, m->dy.p);
-    // readout backward
-    const unsigned nbo = (unsigned)((nn + BSZ - 1) / BSZ);
-    m->part.ensure((size_t)nbo * (MH + 1));
-    k_mp_out_bwd<<<nbo, BSZ, 0, st>>>(n, m->dy.p, m->H[MLAYERS].p, m->theta.p + WO_OFF, m->dH.p, m->part.p);
-    k_mp_reduce<<<1, 128, 0, st>>>((int)nbo, MH + 1, MH + 1, m->part.p, m->grad.p + WO_OFF);
-    // layers
-    float *dHk = m->dH.p, *dHo = m->dH2.p;
-    const unsigned nbw = (unsigned)((nn + 63) / 64);
-    for (int k = MLAYERS - 1; k >= 0; k--) {
-        const int fin = fin_of(k);
-        const size_t blk = (size_t)MH * 2 * fin + MH;
-        m->part.ensure((size_t)nbw * blk);
-        m->tmp_a.ensure((blk + 1) / 2 + 1);
-        float *gsum = (float *)m->tmp_a.p;
-        FVM_HIP(hipMemsetAsync(gsum, 0, blk * sizeof(float), st));
-        if (fin == MF0)
-            k_mp_wgrad<MF0><<<nbw, BSZ, 0, st>>>(n, dHk, m->H[k + 1].p, m->H[k].p, m->A[k].p, m->part.p);
-        else
-            k_mp_wgrad<MH><<<nbw, BSZ, 0, st>>>(n, dHk, m->H[k + 1].p, m->H[k].p, m->A[k].p, m->part.p);
-        k_mp_reduce<<<grid_for((long long)blk, BSZ), BSZ, 0, st>>>((int)nbw, (int)blk, (int)blk, m->part.p, gsum);
-        float *gl = m->grad.p + layer_off(k);
-        if (fin == MF0) k_mp_scatter_wgrad<MF0><<<grid_for((long long)blk, BSZ), BSZ, 0, st>>>(gsum, gl);
-        else k_mp_scatter_wgrad<MH><<<grid_for((long long)blk, BSZ), BSZ, 0, st>>>(gsum, gl);
-        if (k > 0) {   // gradient of the layer input (fin = 64 here)
-            const unsigned gg = grid_for((long long)n * MH, BSZ);
-            k_mp_bwd_gp<MH><<<gg, BSZ, 0, st>>>(n, dHk, m->H[k + 1].p, m->wbf[k].p, m->G.p, m->P.p);
-            k_mp_bwd_agg<MH><<<gg, BSZ, 0, st>>>(n, m->row, m->col, m->ct.p, m->G.p, m->P.p, dHo);
-            std::swap(dHk, dHo);
-        }
-    }
+    const float *wo = m->theta.p + WO_OFF;
+    const unsigned gl = mp_grid(n);
+    k_mp_bwd<true><<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->ct.p, m->dy.p, m->H[3].p, wo, m->wbf[2].p, m->H[2].p,
+                                       m->D2.p);
+    k_mp_bwd<false><<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->ct.p, m->D2.p, nullptr, nullptr, m->wbf[1].p, m->H[1].p,
+                                        m->D1.p);
+    k_mp_wgrad<<<dim3(runs, MLAYERS), BSZ, 0, st>>>(n, m->dy.p, m->D2.p, m->D1.p, m->H[3].p, m->H[2].p, m->H[1].p,
+                                                    m->H[0].p, m->A[2].p, m->A[1].p, m->A[0].p, wo, m->part.p);
+    k_mp_reduce<<<(WG_S + 63) / 64, BSZ, 0, st>>>((int)runs, m->part.p, m->grad.p);
     FVM_HIP(hipGetLastError());
     m->grad_count++;
     double h_rr[2];

@@ -113,6 +113,93 @@ def test_energy_gradient_matches_restatement():
     assert np.linalg.norm(g - gr) / np.linalg.norm(gr) < 5e-2
 
 
+def _ring(n, rng):
+    """A ring with a chord per node: symmetric weights, diagonally dominant."""
+    i = np.arange(n)
+    a = np.concatenate([i, i])
+    b = np.concatenate([(i + 1) % n, (i + 7) % n])
+    lo, hi = np.minimum(a, b)[a != b], np.maximum(a, b)[a != b]
+    lo, hi = np.unique(np.stack([lo, hi], 1), axis=0).T if len(lo) else (lo, hi)
+    w = 0.5 + rng.random(len(lo))
+    r, c, v = np.concatenate([lo, hi]), np.concatenate([hi, lo]), np.concatenate([w, w])
+    o = np.lexsort((c, r))
+    cnt = np.bincount(r, minlength=n)
+    diag = -(np.bincount(r, weights=v, minlength=n) + 0.1 + rng.random(n))
+    row = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    return dict(n_self=n, row=row, col=c[o].astype(np.int32), off=v[o], diag=diag)
+
+
+def _rounded(theta, G, r, et):
+    """The restatement with the activations rounded to bf16 where the kernels round them; FP64 otherwise.
+    et None: the residual loss. Returns (e, loss, gradient, amplification of an error of e into the loss)."""
+    P = M.unpack(theta)
+    u = -r / G.diag
+    s = np.sqrt(np.mean(u * u)) + 1e-300
+    v = (u / s).astype(np.float32)
+    h = np.zeros((G.n, M.F0))
+    h[:, 0], h[:, 1], h[:, 2] = v, G.agg(v.astype(np.float64)), G.l
+    h = M.bf16_round(h)
+    cache = []
+    for k in range(M.LAYERS):
+        a = M.bf16_round(G.agg(h))
+        hn = M.bf16_round(np.maximum(h @ P["Ws%d" % k].T + a @ P["Wn%d" % k].T + P["b%d" % k], 0.0))
+        cache.append((h, a, hn))
+        h = hn
+    e = s * (h @ P["wo"] + P["bo"][0])
+    if et is None:
+        Ae = G.matvec(e)
+        t, den = r + Ae, r @ r
+        ge, loss, amp = 2.0 * G.matvec(t) / den, t @ t / den, np.linalg.norm(Ae) / np.linalg.norm(t)
+    else:
+        t, den = e - et, -(et @ G.matvec(et))
+        Mt = -G.matvec(t)
+        ge, loss, amp = 2.0 * Mt / den, t @ Mt / den, np.linalg.norm(e) / np.linalg.norm(t)
+    dy = s * ge
+    D = {"wo": h.T @ dy, "bo": np.array([dy.sum()])}
+    dh = np.outer(dy, P["wo"])
+    for k in reversed(range(M.LAYERS)):
+        h, a, hn = cache[k]
+        delta = dh * (hn > 0)
+        D["Ws%d" % k], D["Wn%d" % k], D["b%d" % k] = delta.T @ h, delta.T @ a, delta.sum(0)
+        if k > 0:
+            dh = delta @ P["Ws%d" % k] + G.agg_t(delta @ P["Wn%d" % k])
+    return e, loss, M.pack(D), max(1.0, amp)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 65, 127, 129, 511, 513, 32769, 98321])
+def test_tile_edges(n):
+    """Sizes at the edges of a tile (16 nodes), a block (64), a run of the weight gradients (128; 256 runs
+    from 32,768 nodes on) and of one step of the widest grid (98,304), against the restatement with the
+    kernels' roundings. What is left are FP32 sums of at most 128 terms (1e-5) and the activations that
+    these move over a rounding boundary: fewer than 1 % of them, by one bf16 step (2^-8) each, so less
+    than 2^-8 of a norm even if all lay in one direction; the losses magnify an error of e by amp."""
+    import torch
+    from fvm_amd import LearnedCorrection
+    rng = np.random.default_rng(n)
+    m = _ring(n, rng)
+    G = M.Graph(m["row"], m["col"], m["off"], m["diag"])
+    th = (M.init_params(3) + 0.05 * rng.normal(size=M.n_params())).astype(np.float32)
+    thq = M.quantize(th.astype(np.float64))
+    net = LearnedCorrection(seed=3)
+    net.set_params(th)
+    net.set_graph(*_graph(m))
+    r, et = rng.normal(size=G.n), rng.normal(size=G.n)
+    out = torch.zeros(G.n, dtype=torch.float64, device="cuda:0")
+    net.forward(_dev(r, torch.float64), out)
+    tol = 2.0 ** -8
+    for pair in (None, et):
+        e, Lr, gr, amp = _rounded(thq, G, r, pair)
+        err = np.linalg.norm(out.cpu().numpy() - e) / np.linalg.norm(e)
+        L = net.loss_grad(_dev(r, torch.float64)) if pair is None else \
+            net.loss_grad_pair(_dev(r, torch.float64), _dev(et, torch.float64))
+        g = net.grad(reset=True).astype(np.float64)
+        ge = np.linalg.norm(g - gr) / np.linalg.norm(gr)
+        print("n", n, "e", err, "loss", abs(L - Lr) / Lr, "grad", ge, "amp", amp, flush=True)
+        assert err < tol
+        assert abs(L - Lr) < 2 * tol * amp * Lr
+        assert ge < 2 * tol * amp
+
+
 def test_training_lowers_the_loss():
     import torch
     from fvm_amd import LearnedCorrection
