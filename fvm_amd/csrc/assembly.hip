@@ -355,8 +355,8 @@ __device__ __forceinline__ void unit_step(const double *cc, int c0, int c1, bool
 }
 
 __global__ void k_lsq_coeffs(int n_cells, int nct, int dim, const int *cf_row, const int *cf_col,
-                             const int *fcells, const int *pos01, const int *pos10, const double *cc,
-                             const double *fA, const double *vol, double *gc) {
+                             const int *fcells, const int *slot, const double *cc, const double *fA,
+                             const double *vol, double *gc) {
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nct; c += gridDim.x * blockDim.x) {
         const int qb = cf_row[c], qe = cf_row[c + 1];
         bool degen = false;
@@ -412,28 +412,84 @@ __global__ void k_lsq_coeffs(int n_cells, int nct, int dim, const int *cf_row, c
                 w[1] = (K[1] * u[0] + K[3] * u[1] + K[4] * u[2]) / m;
                 w[2] = (K[2] * u[0] + K[4] * u[1] + K[5] * u[2]) / m;
             }
-            const int p = first ? pos01[f] : pos10[f];
-            for (int a = 0; a < 3; a++) gc[3 * (size_t)p + a] = w[a];
+            for (int a = 0; a < 3; a++) gc[(size_t)(slot[c >> 6] + q - qb) * 192 + 64 * a + (c & 63)] = w[a];
         }
     }
 }
 
+// Row slices of the cell kernels: 64 rows side by side, slot k of a slice holds entry k of
+// its 64 rows (slot[s] = the slices' first slots; a slice has as many slots as its longest
+// row), so that a wavefront reads each slot with consecutive addresses. Per entry: the face
+// with the side in the sign (f if the row is its first cell, ~f otherwise) and the other
+// cell; the gradient coefficients lie in the same order, 3 x 64 per slot. On a conformal
+// mesh entry k of a row is its k-th face, so the CSR position is cf_row + k.
+__global__ void k_slice_len(int nct, const int *cf_row, int *len) {
+    const int s = blockIdx.x * (BS / 64) + (threadIdx.x >> 6), c = 64 * s + (threadIdx.x & 63);
+    if (64 * s >= nct) return;
+    int l = c < nct ? cf_row[c + 1] - cf_row[c] : 0;
+    for (int o = 32; o > 0; o >>= 1) l = max(l, __shfl_xor(l, o, 64));
+    if ((threadIdx.x & 63) == 0) len[s] = l;
+}
+__global__ void k_slice_fill(int nct, const int *cf_row, const int *cf_col, const int *fcells, const int *slot,
+                             int2 *ent) {
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nct; c += gridDim.x * blockDim.x) {
+        int2 *e = ent + (size_t)slot[c >> 6] * 64 + (c & 63);
+        for (int q = cf_row[c], k = 0; q < cf_row[c + 1]; q++, k++) {
+            const int f = cf_col[q], c0 = fcells[2 * f];
+            e[(size_t)k * 64] = c0 == c ? make_int2(f, fcells[2 * f + 1]) : make_int2(~f, c0);
+        }
+    }
+}
+
+// What a face's diffusion takes from the mesh alone (DiffusionDiscretization.h:172-190), four
+// planes of n_faces: |A|^2 / (A . ds) and A - ds |A|^2 / (A . ds), ds between the centroids.
+__global__ void k_face_geo(int nf, const int *fcells, const double *fA, const double *fAm, const double *cc,
+                           double *geo) {
+    for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
+        const int c0 = fcells[2 * f], c1 = fcells[2 * f + 1];
+        const double *A = fA + 3 * (size_t)f;
+        double ds[3];
+        for (int a = 0; a < 3; a++) ds[a] = cc[3 * (size_t)c1 + a] - cc[3 * (size_t)c0 + a];
+        const double metric = fAm[f] * fAm[f] / (A[0] * ds[0] + A[1] * ds[1] + A[2] * ds[2]);
+        geo[f] = metric;
+        for (int a = 0; a < 3; a++) geo[(size_t)(a + 1) * nf + f] = A[a] - ds[a] * metric;
+    }
+}
+
+// Blocks are handed to the 8 XCDs in turn: block b takes a chunk of the b % 8-th eighth, so
+// that neighbouring rows share an L2.
+__device__ __forceinline__ int xcd_block() {
+    const int G = gridDim.x, j = blockIdx.x & 7, q = G >> 3, r = G & 7;
+    return j * q + (j < r ? j : r) + (blockIdx.x >> 3);
+}
+
 // GradientMatrix::getGradient (GradientMatrix.h:55-76) of the self cells, entries in
-// CSR order; a ghost cell then takes its face's cell's gradient (GradientModel.h:500-515)
-__global__ void k_gradient(int n_cells, const int *row, const int *col, const double *gc, const double *x,
-                           double *grad) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n_cells; c += gridDim.x * blockDim.x) {
+// CSR order; a ghost cell then takes its face's cell's gradient (GradientModel.h:500-515).
+// Component a of cell c goes to grad[c per_cell + a per_comp].
+// Bound by the coefficients' 24 bytes per entry. 1,397,760 cells: 66 us (3.9 TB/s),
+// 183 us with the coefficients by CSR row (168 bytes between lanes).
+__global__ void __launch_bounds__(BS) k_gradient(int n_cells, const int *__restrict__ row,
+                                                 const int *__restrict__ slot, const int2 *__restrict__ ent,
+                                                 const double *__restrict__ gc, const double *__restrict__ x,
+                                                 double *__restrict__ grad, int per_cell, int per_comp) {
+    for (int c = xcd_block() * blockDim.x + threadIdx.x; c < n_cells; c += gridDim.x * blockDim.x) {
         double g0 = 0.0, g1 = 0.0, g2 = 0.0;
         const double xc = x[c];
-        for (int nb = row[c]; nb < row[c + 1]; nb++) {
-            const double v = x[col[nb]] - xc;
-            g0 += gc[3 * (size_t)nb] * v;
-            g1 += gc[3 * (size_t)nb + 1] * v;
-            g2 += gc[3 * (size_t)nb + 2] * v;
+        const int len = row[c + 1] - row[c];
+        const size_t s = (size_t)slot[c >> 6];
+        const int2 *e = ent + s * 64 + (c & 63);
+        const double *g = gc + s * 192 + (c & 63);
+#pragma unroll 2
+        for (int k = 0; k < len; k++) {
+            const double v = x[e[(size_t)k * 64].y] - xc;
+            g0 += g[(size_t)k * 192] * v;
+            g1 += g[(size_t)k * 192 + 64] * v;
+            g2 += g[(size_t)k * 192 + 128] * v;
         }
-        grad[3 * c] = g0;
-        grad[3 * c + 1] = g1;
-        grad[3 * c + 2] = g2;
+        double *o = grad + (size_t)c * per_cell;
+        o[0] = g0;
+        o[per_comp] = g1;
+        o[2 * (size_t)per_comp] = g2;
     }
 }
 
@@ -445,143 +501,244 @@ __global__ void k_grad_ghost(int n_cells, int nct, const int *cf_row, const int 
     }
 }
 
-// per face: diffusion coefficient and flux with the secondary (non-orthogonal)
-// term from the volume-weighted face gradient (DiffusionDiscretization.h:172-212)
-__global__ void k_face_diffusion(int nf, const int *fcells, const double *fA, const double *fAm,
-                                 const double *cc, const double *vol, const double *kc,
-                                 const double *x, const double *grad, double *dcoef, double *dflux) {
-    for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
-        const int c0 = fcells[2 * f], c1 = fcells[2 * f + 1];
-        const double vol0 = vol[c0], vol1 = vol[c1];
-        double ds[3];
-        for (int a = 0; a < 3; a++) ds[a] = cc[3 * c1 + a] - cc[3 * c0 + a];
-        double kf;
-        if (vol0 == 0.) kf = kc[c1];
-        else if (vol1 == 0.) kf = kc[c0];
-        else kf = harmonic(kc[c0], kc[c1]);
-        const double *A = fA + 3 * f;
-        const double diffMetric = fAm[f] * fAm[f] / (A[0] * ds[0] + A[1] * ds[1] + A[2] * ds[2]);
-        const double diffCoeff = kf * diffMetric;
-        double sec[3], gradF[3];
-        for (int a = 0; a < 3; a++) sec[a] = kf * (A[a] - ds[a] * diffMetric);
-        for (int a = 0; a < 3; a++) gradF[a] = (grad[3 * c0 + a] * vol0 + grad[3 * c1 + a] * vol1) / (vol0 + vol1);
-        double dsec = 0.0;
-        for (int a = 0; a < 3; a++) dsec += gradF[a] * sec[a];
-        dcoef[f] = diffCoeff;
-        dflux[f] = diffCoeff * (x[c1] - x[c0]) + dsec;
-    }
+// ThermalModel's linearization, one row per thread, from the mesh to the eliminated system. What it computes, in the order of the reference's discretization list
+// (ThermalModel_impl.h:238-265), each sum over the row's faces in ascending order:
+//   diffusion with the secondary (non-orthogonal) term from the volume-weighted face gradient
+//     (DiffusionDiscretization.h:172-212);
+//   convection (ConvectionDiscretization.h:160-185 upwind; :131-147 central, whose face value
+//     is 0.5 (x0 + x0) with the upwind linearization) and the continuity residual;
+//   the source (interior cells);
+//   GenericBCS: Dirichlet adds coeff01 (Tb - x_ghost) to b and drops the coefficient
+//     (GenericBCS.h:77-110), extrapolation folds the ghost's diagonal into the cell (:170-192),
+//     Neumann (:129-150); a specified-temperature face with an outflow convecting flux
+//     extrapolates (ThermalModel_impl.h:306-318);
+//   LinearSystem::initSolve: the marked ghost rows (one neighbour each) are eliminated into
+//     their interior cell, ghosts in ascending order (CRMatrix.h:899-944).
+// The first four are k_thermal_rows, over cells and ghosts; the rest touches only cells with
+// a ghost (k_thermal_bcells) and the ghosts (k_thermal_ghosts). A face's terms are formed by
+// both of its rows, from the same operands in the same order: that costs four divisions per
+// entry and saves the face arrays and the passes that clear rows and look for boundary faces.
+// Values are kept by component and not by cell or face: with 24 bytes between lanes each
+// load touched three times as many cache lines, and the address unit was busy 3/4 of the time.
+// A block's coefficients go through LDS, for whole lines (by row they were written 3.2 times
+// over). Bound by its loads, 80 bytes per entry, 48 of them gathered. 1,397,760
+// cells: 114 us, 236 us with values by cell and face; bcells 24, ghosts 4 us (six passes, 375 us, before).
+struct Thermal {
+    int n_cells, nct, nf, central;
+    const int *cf_row, *fcells, *slot;
+    const int2 *ent;
+    const double *fAm, *geo, *vol, *k, *x, *grad, *F, *cont, *src;
+};
+struct CellValues {
+    double g[3], vol, k, x;
+};
+__device__ __forceinline__ int2 row_entry(const Thermal &T, int c, int k) {
+    return T.ent[(size_t)(T.slot[c >> 6] + k) * 64 + (c & 63)];
 }
-
-// per cell: diffusion sums in face order, then the convection terms of its faces in
-// face order (ConvectionDiscretization.h:160-185 upwind; :131-147 central, whose
-// face value is 0.5 (x0 + x0) with the upwind linearization), the continuity
-// residual, then the source (interior cells) -- the order of the reference's
-// discretization list (ThermalModel_impl.h:238-265)
-__global__ void k_cell_assemble(int n_cells, int nct, const int *cf_row, const int *cf_col,
-                                const int *fcells, const int *pos01, const int *pos10,
-                                const int *row, const double *dcoef, const double *dflux,
-                                const double *F, const double *cont_res, int central, const double *x,
-                                const double *vol, const double *src, double *diag, double *off,
-                                double *b) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nct; c += gridDim.x * blockDim.x) {
-        for (int p = row[c]; p < row[c + 1]; p++) off[p] = 0.0;
-        double d = 0.0, r = 0.0;
-        for (int q = cf_row[c]; q < cf_row[c + 1]; q++) {
-            const int f = cf_col[q];
-            const bool first = (fcells[2 * f] == c);
-            off[first ? pos01[f] : pos10[f]] += dcoef[f];
-            d -= dcoef[f];
-            if (first) r += dflux[f];
-            else r -= dflux[f];
+__device__ __forceinline__ int first_face(const Thermal &T, int c) {
+    const int f = row_entry(T, c, 0).x;
+    return f < 0 ? ~f : f;
+}
+__device__ __forceinline__ void cell_values(const Thermal &T, int c, CellValues &v) {
+    // a ghost cell takes its face's cell's gradient (GradientModel.h:500-515)
+    const int gcell = c < T.n_cells ? c : T.fcells[2 * first_face(T, c)];
+#pragma unroll
+    for (int a = 0; a < 3; a++) v.g[a] = T.grad[(size_t)a * T.n_cells + gcell];
+    v.vol = T.vol[c];
+    v.k = T.k[c];
+    v.x = T.x[c];
+}
+// diffusion coefficient and flux of face f between row c (own) and the other cell; first: the
+// row is the face's first cell. The difference changes its sign exactly, the sums commute.
+__device__ __forceinline__ void face_terms(const Thermal &T, int f, bool first, const CellValues &own,
+                                           const CellValues &oth, double &dcoef, double &dflux) {
+    const double vol0 = first ? own.vol : oth.vol, vol1 = first ? oth.vol : own.vol;
+    const double k0 = first ? own.k : oth.k, k1 = first ? oth.k : own.k;
+    double kf;
+    if (vol0 == 0.) kf = k1;
+    else if (vol1 == 0.) kf = k0;
+    else kf = harmonic(k0, k1);
+    dcoef = kf * T.geo[f];
+    double dsec = 0.0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const double sec = kf * T.geo[(size_t)(a + 1) * T.nf + f];
+        const double gradF = (own.g[a] * own.vol + oth.g[a] * oth.vol) / (vol0 + vol1);
+        dsec += gradF * sec;
+    }
+    dflux = dcoef * (first ? oth.x - own.x : own.x - oth.x) + dsec;
+}
+// a row before the boundary conditions; entry k goes to put(k, value)
+template <class Put>
+__device__ __forceinline__ void thermal_row(const Thermal &T, int c, int len, const CellValues &own, double &d,
+                                            double &r, Put put) {
+    d = 0.0;
+    r = 0.0;
+    const int2 *ent = T.ent + (size_t)T.slot[c >> 6] * 64 + (c & 63);
+    int2 e = len > 0 ? ent[0] : make_int2(0, 0);
+    for (int k = 0; k < len; k++) {
+        const int2 ek = e;
+        if (k + 1 < len) e = ent[(size_t)(k + 1) * 64];   // ahead of the loads that hang on it
+        const bool first = ek.x >= 0;
+        const int f = first ? ek.x : ~ek.x;
+        CellValues oth;
+        cell_values(T, ek.y, oth);
+        double dcoef, dflux;
+        face_terms(T, f, first, own, oth, dcoef, dflux);
+        double o = 0.0;
+        o += dcoef;
+        d -= dcoef;
+        if (first) r += dflux;
+        else r -= dflux;
+        if (T.F) {
+            const double Ff = T.F[f];
+            if (Ff > 0.0 && !first) o += Ff;
+            if (!(Ff > 0.0) && first) o -= Ff;
         }
-        if (F) {
-            for (int q = cf_row[c]; q < cf_row[c + 1]; q++) {
-                const int f = cf_col[q];
-                const int c0 = fcells[2 * f], c1 = fcells[2 * f + 1];
-                const double Ff = F[f];
-                double flux;
-                if (central) flux = 0.5 * Ff * (x[c0] + x[c0]);
-                else flux = Ff > 0.0 ? Ff * x[c0] : Ff * x[c1];
-                if (Ff > 0.0) {
-                    if (c == c0) d -= Ff;
-                    else off[pos10[f]] += Ff;
-                } else {
-                    if (c == c1) d += Ff;
-                    else off[pos01[f]] -= Ff;
-                }
-                if (c == c0) r -= flux;
-                else r += flux;
+        put(k, o);
+    }
+    if (T.F) {
+        for (int k = 0; k < len; k++) {
+            const int2 ek = ent[(size_t)k * 64];
+            const bool first = ek.x >= 0;
+            const double Ff = T.F[first ? ek.x : ~ek.x], xo = T.x[ek.y];
+            const double x0 = first ? own.x : xo, x1 = first ? xo : own.x;
+            double flux;
+            if (T.central) flux = 0.5 * Ff * (x0 + x0);
+            else flux = Ff > 0.0 ? Ff * x0 : Ff * x1;
+            if (Ff > 0.0) {
+                if (first) d -= Ff;
+            } else {
+                if (!first) d += Ff;
             }
-            if (c < n_cells) d += cont_res ? cont_res[c] : 0.0;
+            if (first) r -= flux;
+            else r += flux;
         }
-        if (c < n_cells) r += vol[c] * src[c];
-        diag[c] = d;
-        b[c] = r;
+        if (c < T.n_cells) d += T.cont ? T.cont[c] : 0.0;
     }
+    if (c < T.n_cells) r += T.vol[c] * T.src[c];
 }
-
-// A specified-temperature face with an outflow convecting flux extrapolates
-// (ThermalModel_impl.h:306-318).
 __device__ __forceinline__ bool bc_dirichlet(const Groups &G, int g, const double *F, int f) {
     return G.type[g] == FVM_BC_DIRICHLET && !(F && F[f] > 0.);
 }
+// ghost row j after its boundary condition (d, r: before it): its diagonal, right-hand side
+// and, from o, the coefficient of its first face; returns whether the row is a boundary row
+__device__ __forceinline__ bool ghost_row(const Thermal &T, const Groups &G, int j, double &d, double &r, double &o) {
+    const int f = first_face(T, j), g = group_of(G, f);
+    if (bc_dirichlet(G, g, T.F, f)) {
+        o = 0.0;
+        r = 0.0;
+        d = -1.0;
+        return false;
+    }
+    if (G.type[g] == FVM_BC_DIRICHLET) {
+        d = -1.0;
+        o = 1.0;
+        r = T.x[T.fcells[2 * f]] - T.x[j];
+    } else {
+        const double fluxB = -r;
+        r = G.value[g] * T.fAm[f] - fluxB;
+    }
+    return true;
+}
 
-// GenericBCS, interior side, faces in order: Dirichlet adds coeff01 (Tb - x_ghost)
-// to b[c0] and drops the coefficient (GenericBCS.h:77-100); extrapolation folds
-// the ghost's diagonal into the cell (:170-185). Reads the ghost diagonal before
-// k_bc_ghost resets it.
-__global__ void k_bc_interior(int n_cells, const int *cf_row, const int *cf_col, const int *fcells,
-                             const int *pos01, Groups G, const double *F, const double *x, double *diag,
-                             double *off, double *b) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n_cells; c += gridDim.x * blockDim.x) {
-        for (int q = cf_row[c]; q < cf_row[c + 1]; q++) {
-            const int f = cf_col[q];
-            if (f < G.ptr[1]) continue;
-            const int g = group_of(G, f);
-            const int c1 = fcells[2 * f + 1];
-            if (bc_dirichlet(G, g, F, f)) {
-                const double dX = G.value[g] - x[c1];
-                b[c] += off[pos01[f]] * dX;
-                off[pos01[f]] = 0.0;
-            } else if (G.type[g] == FVM_BC_DIRICHLET) {
-                const double dFdX1 = -diag[c1];
-                const double dx01 = x[c] - x[c1];
-                diag[c] += dFdX1;
-                b[c] += dFdX1 * dx01;
-                off[pos01[f]] = 0.0;
-            }
+constexpr int ROW_LDS = 8 * BS;   // coefficients of a block that go through LDS: 8 per row (7 on hexahedra at most)
+__global__ void __launch_bounds__(BS) k_thermal_rows(Thermal T, double *__restrict__ diag, double *__restrict__ off,
+                                                     double *__restrict__ b, uint8_t *__restrict__ isb) {
+    __shared__ double o_sh[ROW_LDS];
+    for (int c0 = xcd_block() * BS; c0 < T.nct; c0 += gridDim.x * BS) {   // the same for the whole block
+        const int c = c0 + threadIdx.x;
+        const int qb = T.cf_row[c0], nq = T.cf_row[min(c0 + BS, T.nct)] - qb;
+        const bool staged = nq <= ROW_LDS;
+        if (c < T.nct) {
+            const int q0 = T.cf_row[c], len = T.cf_row[c + 1] - q0;
+            CellValues own;
+            cell_values(T, c, own);
+            double d, r;
+            thermal_row(T, c, len, own, d, r, [&](int k, double o) {
+                if (staged) o_sh[q0 - qb + k] = o;
+                else off[q0 + k] = o;
+            });
+            diag[c] = d;
+            b[c] = r;
+            isb[c] = 0;
+        }
+        if (staged) {
+            __syncthreads();
+            for (int q = threadIdx.x; q < nq; q += BS) off[qb + q] = o_sh[q];
+            __syncthreads();
         }
     }
 }
 
-// GenericBCS, ghost side (GenericBCS.h:100-110 Dirichlet, :129-150 Neumann,
-// :187-192 extrapolation)
-__global__ void k_bc_ghost(int n_cells, int nct, const int *cf_row, const int *cf_col, const int *fcells,
-                           const int *pos10, const double *fAm, Groups G, const double *F, const double *x,
-                           double *diag, double *off, double *b, uint8_t *isb) {
-    for (int gc = n_cells + blockIdx.x * blockDim.x + threadIdx.x; gc < nct; gc += gridDim.x * blockDim.x) {
-        const int f = cf_col[cf_row[gc]];
-        const int g = group_of(G, f);
-        isb[gc] = 0;
-        if (bc_dirichlet(G, g, F, f)) {
-            off[pos10[f]] = 0.0;
-            b[gc] = 0.0;
-            diag[gc] = -1.0;
-        } else if (G.type[g] == FVM_BC_DIRICHLET) {
-            diag[gc] = -1.0;
-            off[pos10[f]] = 1.0;
-            b[gc] = x[fcells[2 * f]] - x[gc];
-            isb[gc] = 1;
+// The boundary conditions and the elimination in the cells that have a ghost (as a branch of
+// k_thermal_rows nearly every wavefront would enter it for one or two of its cells). One
+// thread per ghost, which takes the cell whose first ghost it is. The ghost rows stay as they
+// are: k_thermal_ghosts follows.
+__device__ void thermal_bcell(const Thermal &T, const Groups &G, int c, int len, double *diag, double *off, double *b) {
+    const int q0 = T.cf_row[c];
+    double d = diag[c], r = b[c];
+    for (int k = 0; k < len; k++) {
+        const int2 e = row_entry(T, c, k);
+        const int f = e.x < 0 ? ~e.x : e.x;
+        if (f < G.ptr[1]) continue;
+        const int g = group_of(G, f), c1 = e.y;
+        if (G.type[g] != FVM_BC_DIRICHLET) continue;
+        if (bc_dirichlet(G, g, T.F, f)) {
+            const double dX = G.value[g] - T.x[c1];
+            r += off[q0 + k] * dX;
         } else {
-            const double fluxB = -b[gc];
-            b[gc] = G.value[g] * fAm[f] - fluxB;
-            isb[gc] = 1;
+            const double dFdX1 = -diag[c1];
+            const double dx01 = T.x[c] - T.x[c1];
+            d += dFdX1;
+            r += dFdX1 * dx01;
+        }
+        off[q0 + k] = 0.0;
+    }
+    for (int k = 0; k < len; k++) {
+        const int2 e = row_entry(T, c, k);
+        const int j = e.y;
+        if (e.x < 0 || j < T.n_cells) continue;
+        // the ghost's coefficient of this face
+        const int p0 = T.cf_row[j];
+        int p = p0;
+        while (T.ent[(size_t)(T.slot[j >> 6] + p - p0) * 64 + (j & 63)].x != ~e.x) p++;
+        double ajj = diag[j], bj = b[j], ajk = off[p], o = ajk;
+        if (!ghost_row(T, G, j, ajj, bj, o)) continue;
+        if (p == p0) ajk = o;
+        const double aij = off[q0 + k];
+        d -= aij * (ajk / ajj);
+        r -= aij * (bj / ajj);
+        off[q0 + k] = 0.0;
+    }
+    diag[c] = d;
+    b[c] = r;
+}
+
+__global__ void __launch_bounds__(BS) k_thermal_bcells(Thermal T, Groups G, double *diag, double *off, double *b) {
+    for (int j = T.n_cells + blockIdx.x * blockDim.x + threadIdx.x; j < T.nct; j += gridDim.x * blockDim.x) {
+        const int jlen = T.cf_row[j + 1] - T.cf_row[j];
+        for (int kj = 0; kj < jlen; kj++) {
+            const int2 e = row_entry(T, j, kj);   // the ghost is its faces' second cell
+            const int c = e.y, len = T.cf_row[c + 1] - T.cf_row[c];
+            int k = 0;
+            while (row_entry(T, c, k).y < T.n_cells) k++;   // ends at this face at the latest
+            if (row_entry(T, c, k).x == ~e.x) thermal_bcell(T, G, c, len, diag, off, b);
         }
     }
 }
 
-// LinearSystem::initSolve: eliminate the marked ghost rows (one neighbour each)
-// into their interior cell, ghosts in ascending order (CRMatrix.h:899-944).
+__global__ void k_thermal_ghosts(Thermal T, Groups G, double *diag, double *off, double *b, uint8_t *isb) {
+    for (int j = T.n_cells + blockIdx.x * blockDim.x + threadIdx.x; j < T.nct; j += gridDim.x * blockDim.x) {
+        const int p = T.cf_row[j];
+        double d = diag[j], r = b[j], o = off[p];
+        isb[j] = ghost_row(T, G, j, d, r, o);
+        diag[j] = d;
+        b[j] = r;
+        off[p] = o;
+    }
+}
+
 // LinearSystem::postSolve -> CRMatrix::solveBoundary (LinearSystem.cpp:250-252,
 // CRMatrix.h:433-454): every boundary row nr >= n_self takes
 // x[nr] = -(b[nr] + sum off x[col]) / diag[nr], the sum in CSR order.
@@ -610,6 +767,8 @@ __global__ void k_solve_boundary(int n_self, int n_total, const int *row, const 
     }
 }
 
+// LinearSystem::initSolve: eliminate the marked ghost rows (one neighbour each)
+// into their interior cell, ghosts in ascending order (CRMatrix.h:899-944).
 __global__ void k_eliminate(int n_cells, const int *cf_row, const int *cf_col, const int *fcells,
                             const int *pos01, const int *pos10, const uint8_t *isb, double *diag,
                             double *off, double *b) {
@@ -880,7 +1039,10 @@ struct fvm_mesh {
     DArr<int> cf_row, cf_col, cc_row, cc_col, pos01, pos10;
     long long nnz = 0;
     DArr<double> fA, fAm, fc, cc, vol;
-    DArr<double> gcoef;                // least-squares gradient coefficients, 3 per cellCells entry
+    DArr<int> slot;                    // row slices of the cell kernels (k_slice_fill), with lsq
+    DArr<int2> ent;
+    DArr<double> geo;                  // k_face_geo, with lsq
+    DArr<double> gcoef;                // least-squares gradient coefficients, 3 x 64 per slot
 };
 
 struct fvm_system {
@@ -964,22 +1126,40 @@ void mesh_gradient_coeffs(fvm_mesh *m) {
               "the gradient needs a conformal mesh: two cells share at most one face");
     hipStream_t s = m->stream;
     const int nct = m->n_cells + m->n_ghost;
-    m->gcoef.alloc(3 * (size_t)std::max<long long>(m->nnz, 1));
-    k_lsq_coeffs<<<grid_for(nct, BS), BS, 0, s>>>(m->n_cells, nct, m->dim, m->cf_row.p, m->cf_col.p, m->fcells.p,
-                                                  m->pos01.p, m->pos10.p, m->cc.p, m->fA.p, m->vol.p,
-                                                  m->gcoef.p);
+    const int ns = (nct + 63) / 64;
+    Scanner sc;
+    DArr<int> len((size_t)ns + 1);
+    FVM_HIP(hipMemsetAsync(len.p, 0, len.bytes(), s));
+    if (nct) k_slice_len<<<(unsigned)((ns + BS / 64 - 1) / (BS / 64)), BS, 0, s>>>(nct, m->cf_row.p, len.p);
+    m->slot.alloc((size_t)ns + 1);
+    sc.exclusive(len.p, m->slot.p, ns + 1, s);
+    const size_t slots = std::max(read_scalar(m->slot.p + ns, s), 1);
+    m->ent.alloc(64 * slots);
+    m->gcoef.alloc(192 * slots);
+    m->geo.alloc(4 * (size_t)std::max(m->n_faces, 1));
+    if (m->n_faces)
+        k_face_geo<<<grid_for(m->n_faces, BS), BS, 0, s>>>(m->n_faces, m->fcells.p, m->fA.p, m->fAm.p, m->cc.p,
+                                                           m->geo.p);
+    if (nct) {
+        k_slice_fill<<<grid_for(nct, BS), BS, 0, s>>>(nct, m->cf_row.p, m->cf_col.p, m->fcells.p, m->slot.p,
+                                                      m->ent.p);
+        k_lsq_coeffs<<<grid_for(nct, BS), BS, 0, s>>>(m->n_cells, nct, m->dim, m->cf_row.p, m->cf_col.p,
+                                                      m->fcells.p, m->slot.p, m->cc.p, m->fA.p, m->vol.p,
+                                                      m->gcoef.p);
+    }
     FVM_HIP(hipGetLastError());
     FVM_HIP(hipStreamSynchronize(s));
     m->lsq = true;
 }
 
-// GradientModel::compute of a cell field into grad (3 per cell, ghosts included)
-void mesh_gradient(fvm_mesh *m, const double *x, double *grad, hipStream_t s) {
+// GradientModel::compute of a cell field into grad: 3 per cell, ghosts included, or (planes)
+// three planes of n_cells
+void mesh_gradient(fvm_mesh *m, const double *x, double *grad, hipStream_t s, bool planes) {
     const int nct = m->n_cells + m->n_ghost;
     if (m->n_cells)
-        k_gradient<<<grid_for(m->n_cells, BS), BS, 0, s>>>(m->n_cells, m->cc_row.p, m->cc_col.p, m->gcoef.p, x,
-                                                           grad);
-    if (m->n_ghost)
+        k_gradient<<<grid_for(m->n_cells, BS), BS, 0, s>>>(m->n_cells, m->cf_row.p, m->slot.p, m->ent.p, m->gcoef.p,
+                                                           x, grad, planes ? 1 : 3, planes ? m->n_cells : 1);
+    if (!planes && m->n_ghost)
         k_grad_ghost<<<grid_for(m->n_ghost, BS), BS, 0, s>>>(m->n_cells, nct, m->cf_row.p, m->cf_col.p,
                                                              m->fcells.p, grad);
 }
@@ -1002,10 +1182,6 @@ Groups make_groups(const fvm_mesh *m, const int32_t *type, const double *value) 
 
 namespace fvm {
 namespace {
-__global__ void k_fill_u8(int n, uint8_t v, uint8_t *p) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
 // a system with the mesh's cellCells pattern
 void system_alloc(fvm_mesh *m, fvm_system *S) {
     const int nct = m->n_cells + m->n_ghost;
@@ -1023,42 +1199,26 @@ void system_alloc(fvm_mesh *m, fvm_system *S) {
 }
 
 // ThermalModel::linearize + LinearSystem::initSolve into S (pattern already set):
-// gradient of x, diffusion with secondary flux, convection (d_flux may be null),
-// source, boundary conditions, elimination. Scratch: dcoef, dflux (n_faces),
-// grad (3 (n_cells + n_ghost)). Queued on the mesh's stream; no allocation and
-// no host synchronization.
+// gradient of x, then k_thermal_rows (d_flux may be null). Scratch: grad (3 n_cells).
+// Queued on the mesh's stream; no allocation and no host synchronization.
 void assemble_thermal(fvm_mesh *m, fvm_system *S, const double *d_k, const double *d_source, const double *d_x,
-                      const double *d_flux, const double *d_cont, int central, const Groups &G, double *dcoef,
-                      double *dflux, double *grad) {
+                      const double *d_flux, const double *d_cont, int central, const Groups &G, double *grad) {
     hipStream_t s = m->stream;
-    const int nc = m->n_cells, nct = m->n_cells + m->n_ghost, nf = m->n_faces;
-    mesh_gradient(m, d_x, grad, s);
-    if (nf)
-        k_face_diffusion<<<grid_for(nf, 256), 256, 0, s>>>(nf, m->fcells.p, m->fA.p, m->fAm.p, m->cc.p, m->vol.p,
-                                                           d_k, d_x, grad, dcoef, dflux);
-    if (nct)
-        k_cell_assemble<<<grid_for(nct, 256), 256, 0, s>>>(nc, nct, m->cf_row.p, m->cf_col.p, m->fcells.p,
-                                                           m->pos01.p, m->pos10.p, m->cc_row.p, dcoef, dflux,
-                                                           d_flux, d_cont, central, d_x, m->vol.p, d_source,
-                                                           S->diag.p, S->off.p, S->b.p);
-    if (nc)
-        k_bc_interior<<<grid_for(nc, 256), 256, 0, s>>>(nc, m->cf_row.p, m->cf_col.p, m->fcells.p, m->pos01.p, G,
-                                                        d_flux, d_x, S->diag.p, S->off.p, S->b.p);
-    if (nct) k_fill_u8<<<grid_for(nct, 256), 256, 0, s>>>(nct, 0, S->isb.p);
-    if (m->n_ghost)
-        k_bc_ghost<<<grid_for(m->n_ghost, 256), 256, 0, s>>>(nc, nct, m->cf_row.p, m->cf_col.p, m->fcells.p,
-                                                             m->pos10.p, m->fAm.p, G, d_flux, d_x, S->diag.p,
-                                                             S->off.p, S->b.p, S->isb.p);
-    if (nc)
-        k_eliminate<<<grid_for(nc, 256), 256, 0, s>>>(nc, m->cf_row.p, m->cf_col.p, m->fcells.p, m->pos01.p,
-                                                      m->pos10.p, S->isb.p, S->diag.p, S->off.p, S->b.p);
+    const int nct = m->n_cells + m->n_ghost;
+    mesh_gradient(m, d_x, grad, s, true);
+    const Thermal T{m->n_cells, nct,      m->n_faces, central, m->cf_row.p, m->fcells.p, m->slot.p, m->ent.p, m->fAm.p,
+                    m->geo.p,   m->vol.p, d_k,        d_x,     grad,        d_flux,      d_cont,    d_source};
+    if (nct) k_thermal_rows<<<grid_for(nct, BS), BS, 0, s>>>(T, S->diag.p, S->off.p, S->b.p, S->isb.p);
+    if (m->n_ghost) {
+        k_thermal_bcells<<<grid_for(m->n_ghost, BS), BS, 0, s>>>(T, G, S->diag.p, S->off.p, S->b.p);
+        k_thermal_ghosts<<<grid_for(m->n_ghost, BS), BS, 0, s>>>(T, G, S->diag.p, S->off.p, S->b.p, S->isb.p);
+    }
     FVM_HIP(hipGetLastError());
 }
 }  // namespace
 
-// Scratch of the allocation-free re-assembly (fvm_convdiff_reassemble_noalloc):
-// per-face diffusion coefficients and fluxes (2 n_faces) and the cell gradients
-// (3 (n_cells + n_ghost)). One copy per device, held until the process ends.
+// Scratch of the allocation-free re-assembly (fvm_convdiff_reassemble_noalloc): the cell
+// gradients (3 n_cells of the 2 n_faces + 3 (n_cells + n_ghost) that its size limit counts). One copy per device, held until the process ends.
 constexpr size_t NOALLOC_SCRATCH_DOUBLES = (size_t)1 << 22;   // 32 MiB
 static __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 
@@ -1287,6 +1447,7 @@ int fvm_mesh_destroy(fvm_mesh *m) {
         fvm::Dev d(m->device);
         (void)hipStreamSynchronize(m->stream);
         m->nodes.release(); m->fnptr.release(); m->fnodes.release(); m->fcells.release(); m->gcoef.release();
+        m->slot.release(); m->ent.release(); m->geo.release();
         m->cf_row.release(); m->cf_col.release(); m->cc_row.release(); m->cc_col.release();
         m->pos01.release(); m->pos10.release();
         m->fA.release(); m->fAm.release(); m->fc.release(); m->cc.release(); m->vol.release();
@@ -1325,7 +1486,7 @@ int fvm_mesh_gradient(fvm_mesh *m, const double *d_x, double *d_grad) {
     FVM_CHECK(m && d_x && d_grad, FVM_E_INVALID, "null argument");
     fvm::Dev d(m->device);
     fvm::mesh_gradient_coeffs(m);
-    fvm::mesh_gradient(m, d_x, d_grad, m->stream);
+    fvm::mesh_gradient(m, d_x, d_grad, m->stream, false);
     FVM_HIP(hipGetLastError());
     FVM_HIP(hipStreamSynchronize(m->stream));
     return FVM_OK;
@@ -1399,12 +1560,11 @@ int fvm_convdiff_assemble(fvm_mesh *m, const double *d_k, const double *d_source
     fvm::Dev d(m->device);
     fvm::mesh_gradient_coeffs(m);
     const fvm::Groups G = fvm::make_groups(m, bc_type, bc_value);
-    const int nct = m->n_cells + m->n_ghost, nf = m->n_faces;
     fvm_system *S = new fvm_system();
     try {
         fvm::system_alloc(m, S);
-        DArr<double> dcoef(std::max(nf, 1)), dflux(std::max(nf, 1)), grad(3 * (size_t)std::max(nct, 1));
-        fvm::assemble_thermal(m, S, d_k, d_source, d_x, d_flux, d_cont_res, central, G, dcoef.p, dflux.p, grad.p);
+        DArr<double> grad(3 * (size_t)std::max(m->n_cells, 1));
+        fvm::assemble_thermal(m, S, d_k, d_source, d_x, d_flux, d_cont_res, central, G, grad.p);
         FVM_HIP(hipStreamSynchronize(m->stream));
     } catch (...) {
         delete S;
@@ -1438,8 +1598,7 @@ int fvm_convdiff_reassemble_noalloc(fvm_mesh *m, const double *d_k, const double
     fvm::Dev d(m->device);
     double *scr = fvm::scratch_on(m->device);
     const fvm::Groups G = fvm::make_groups(m, bc_type, bc_value);
-    fvm::assemble_thermal(m, S, d_k, d_source, d_x, d_flux, d_cont_res, central, G, scr, scr + nf,
-                          scr + 2 * (size_t)nf);
+    fvm::assemble_thermal(m, S, d_k, d_source, d_x, d_flux, d_cont_res, central, G, scr);
     FVM_HIP(hipStreamSynchronize(m->stream));
     return FVM_OK;
     FVM_API_END

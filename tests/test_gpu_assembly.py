@@ -79,6 +79,56 @@ def test_mesh_from_host_arrays_gives_same_system():
         assert np.array_equal(a[key], b[key]), key
 
 
+def _graph_mesh(n, degree, seed):
+    """Cells joined at random (a chain, ``degree`` chords per cell and a hub), each pair by one face with
+    nodes of its own, and boundary faces in three groups, several on some cells: rows of every length."""
+    rng = np.random.default_rng(seed)
+    pairs = {(i, i + 1) for i in range(n - 1)}
+    for i in range(n):
+        for j in rng.integers(0, n, degree):
+            if i != j:
+                pairs.add((min(i, int(j)), max(i, int(j))))
+    pairs |= {(0, int(j)) for j in rng.integers(1, max(n, 2), min(n // 4, 90)) if 0 < j < n}
+    inner = np.array(sorted(pairs), np.int32).reshape(-1, 2)
+    swap = rng.random(len(inner)) < 0.5
+    inner[swap] = inner[swap][:, ::-1]
+    inner = inner[rng.permutation(len(inner))]
+    nb = n // 3 + 5
+    outer = np.stack([rng.integers(0, n, nb), n + np.arange(nb)], 1)
+    cells = np.concatenate([inner, outer]).astype(np.int32)
+    nf = len(cells)
+    base = rng.normal(size=(nf, 1, 3)) * 5
+    quad = base + rng.normal(size=(nf, 4, 3)) * 0.1 + np.array([[0, 0, 0], [1, 0, 0], [1, 1, 0.2], [0, 1, 0.1]])
+    ni = len(inner)
+    return dict(nodes=quad.reshape(-1), face_nodes=np.arange(4 * nf, dtype=np.int32), face_cells=cells.reshape(-1),
+                n_cells=n, n_ghost=nb, group_ptr=np.array([0, ni, ni + nb // 3, ni + 2 * (nb // 3), nf], np.int32))
+
+
+@pytest.mark.parametrize("n,degree", [(1, 0), (2, 0), (63, 2), (64, 3), (65, 9), (255, 1), (256, 3), (257, 12),
+                                      (1031, 2)])
+def test_row_kernels_on_general_graphs(n, degree):
+    """Slices of 64 rows and blocks of 256 at their edges, rows from one entry to a hub's hundred, blocks
+    with more than the 2,048 coefficients that go through LDS (degree 12): bits of the sequential loops."""
+    import torch
+    from fvm_amd.thermal import Mesh, assemble
+    ref = _graph_mesh(n, degree, n + degree)
+    m = Mesh.from_arrays(ref["nodes"], ref["face_nodes"], ref["face_cells"], ref["n_cells"], ref["n_ghost"],
+                         ref["group_ptr"])
+    rng = np.random.default_rng(n)
+    nt, nf = n + ref["n_ghost"], ref["face_cells"].size // 2
+    dev = lambda a: torch.from_numpy(a).cuda()
+    k, s, x = np.exp(rng.normal(size=nt)), rng.random(nt), rng.normal(size=nt)
+    F, cr = rng.normal(size=nf), rng.normal(size=n)
+    np.testing.assert_array_equal(m.gradient(dev(x)).cpu().numpy(), O.fv_gradient(ref, x))
+    types, values = [0, D, NM, D], [0.0, 1.25, 0.5, -2.0]
+    for flux, cont, central in ((None, None, False), (F, None, False), (F, cr, True)):
+        S = assemble(m, dev(k), dev(s), dev(x), types, values, flux=None if flux is None else dev(flux),
+                     continuity_residual=None if cont is None else dev(cont), central=central).to_host()
+        o = O.fv_thermal(ref, k, s, x, types, values, flux, cont, central)
+        for key in ("row", "col", "diag", "off", "b", "is_boundary"):
+            np.testing.assert_array_equal(S[key], o[key], err_msg=key)
+
+
 def test_amg_on_device_assembled_system_exact():
     import torch
     import fvm_amd
