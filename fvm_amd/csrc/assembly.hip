@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <mutex>
 
 namespace fvm {
@@ -501,7 +502,8 @@ __global__ void k_grad_ghost(int n_cells, int nct, const int *cf_row, const int 
     }
 }
 
-// ThermalModel's linearization, one row per thread, from the mesh to the eliminated system. What it computes, in the order of the reference's discretization list
+// ThermalModel's linearization, one row per thread, from the mesh to the eliminated system.
+// What it computes, in the order of the reference's discretization list
 // (ThermalModel_impl.h:238-265), each sum over the row's faces in ascending order:
 //   diffusion with the secondary (non-orthogonal) term from the volume-weighted face gradient
 //     (DiffusionDiscretization.h:172-212);
@@ -1024,6 +1026,86 @@ __global__ void k_ghost_copy(int n_cells, int nct, const int *cf_row, const int 
 
 using fvm::DArr;
 
+namespace fvm {
+namespace {
+struct Dev {
+    int prev = -1;
+    explicit Dev(int d) {
+        if (hipGetDevice(&prev) != hipSuccess) prev = -1;
+        FVM_HIP(hipSetDevice(d));
+    }
+    ~Dev() { if (prev >= 0) (void)hipSetDevice(prev); }
+};
+
+// What a mesh shares with the systems assembled on it; freed with the last of them.
+//  - the CSR pattern: the systems of a mesh all have the same one and never write it
+//    (a copy each was 73 MB and 310 us at 1,397,760 cells);
+//  - at most one spare block each for a system's values and for an assembly's scratch, so that
+//    a loop that assembles and drops systems does not map and unmap memory every time
+//    (932 -> 232 us per assembly there, copies included; 75 -> 65 us at 9,450 cells).
+// A system's block comes back only when the device has finished with it, as with hipFree;
+// scratch is used on the mesh's stream alone. Both from any thread.
+struct MeshStore {
+    enum Kind { VALUES, SCRATCH };
+    const int device;
+    DArr<int> row, col;
+    explicit MeshStore(int d) : device(d) {}
+    ~MeshStore() {
+        int prev = -1;
+        (void)hipGetDevice(&prev);
+        (void)hipSetDevice(device);
+        row.release();
+        col.release();
+        for (auto &b : spare) if (b.p) (void)hipFree(b.p);
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+    void *take(Kind k, size_t bytes) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (spare[k].p && spare[k].bytes == bytes) {
+                void *p = spare[k].p;
+                spare[k] = Block{};
+                return p;
+            }
+        }
+        void *p = nullptr;
+        const hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess)
+            throw Error(-5, std::string("hipMalloc of ") + std::to_string(bytes) + " bytes failed: " +
+                                hipGetErrorString(e));
+        return p;
+    }
+    // the device is current; ordered: its next user runs on the stream of its last one
+    void put(Kind k, void *p, size_t bytes, bool ordered = false) {
+        if (ordered || hipDeviceSynchronize() == hipSuccess) {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!spare[k].p) {
+                spare[k] = Block{p, bytes};
+                return;
+            }
+        }
+        (void)hipFree(p);
+    }
+
+private:
+    struct Block {
+        void *p = nullptr;
+        size_t bytes = 0;
+    };
+    std::mutex mu;
+    Block spare[2];
+};
+
+// part of a block
+template <class T>
+struct Span {
+    T *p = nullptr;
+    size_t n = 0;
+    size_t bytes() const { return n * sizeof(T); }
+};
+}  // namespace
+}  // namespace fvm
+
 struct fvm_mesh {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -1036,7 +1118,8 @@ struct fvm_mesh {
     long long n_face_nodes = 0;
     // derived
     bool conn = false, metrics = false, lsq = false;
-    DArr<int> cf_row, cf_col, cc_row, cc_col, pos01, pos10;
+    std::shared_ptr<fvm::MeshStore> store;   // the cellCells pattern (row, col), with conn
+    DArr<int> cf_row, cf_col, pos01, pos10;
     long long nnz = 0;
     DArr<double> fA, fAm, fc, cc, vol;
     DArr<int> slot;                    // row slices of the cell kernels (k_slice_fill), with lsq
@@ -1049,22 +1132,38 @@ struct fvm_system {
     int device = 0;
     int n_self = 0, n_total = 0;
     long long nnz = 0;
-    DArr<int> row, col;
-    DArr<double> diag, off, b;
-    DArr<uint8_t> isb;
+    std::shared_ptr<fvm::MeshStore> store;   // row, col
+    void *block = nullptr;                   // diag, off, b, isb
+    size_t block_bytes = 0;
+    fvm::Span<double> diag, off, b;
+    fvm::Span<uint8_t> isb;
+    ~fvm_system() {
+        if (!block) return;
+        int prev = -1;
+        (void)hipGetDevice(&prev);
+        (void)hipSetDevice(device);
+        store->put(fvm::MeshStore::VALUES, block, block_bytes);
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
 };
 
 namespace fvm {
 
 namespace {
-struct Dev {
-    int prev = -1;
-    explicit Dev(int d) {
-        if (hipGetDevice(&prev) != hipSuccess) prev = -1;
-        FVM_HIP(hipSetDevice(d));
-    }
-    ~Dev() { if (prev >= 0) (void)hipSetDevice(prev); }
+// scratch of one assembly on the mesh's stream: n doubles
+struct Scratch {
+    fvm_mesh *m;
+    size_t bytes;
+    double *p;
+    Scratch(fvm_mesh *mesh, size_t n)
+        : m(mesh), bytes(sizeof(double) * std::max<size_t>(n, 1)),
+          p((double *)mesh->store->take(MeshStore::SCRATCH, bytes)) {}
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    ~Scratch() { m->store->put(MeshStore::SCRATCH, p, bytes, true); }
 };
+// the same size for every kind of assembly on a mesh: cell gradients or face fluxes
+size_t scratch_doubles(const fvm_mesh *m) { return std::max(3 * (size_t)m->n_cells, (size_t)m->n_faces); }
 
 void mesh_connectivity(fvm_mesh *m) {
     if (m->conn) return;
@@ -1083,14 +1182,16 @@ void mesh_connectivity(fvm_mesh *m) {
     FVM_HIP(hipMemsetAsync(cnt.p, 0, cnt.bytes(), s));
     k_cc_build<<<grid_for(nct, BS, 4096), BS, 0, s>>>(nct, m->cf_row.p, m->cf_col.p, m->fcells.p, nullptr,
                                                       cnt.p, nullptr, nullptr, nullptr, 0);
-    m->cc_row.alloc((size_t)nct + 1);
-    sc.exclusive(cnt.p, m->cc_row.p, nct + 1, s);
-    m->nnz = read_scalar(m->cc_row.p + nct, s);
-    m->cc_col.alloc(std::max<long long>(m->nnz, 1));
+    m->store = std::make_shared<MeshStore>(m->device);
+    DArr<int> &cc_row = m->store->row, &cc_col = m->store->col;
+    cc_row.alloc((size_t)nct + 1);
+    sc.exclusive(cnt.p, cc_row.p, nct + 1, s);
+    m->nnz = read_scalar(cc_row.p + nct, s);
+    cc_col.alloc(std::max<long long>(m->nnz, 1));
     m->pos01.alloc(std::max(nf, 1));
     m->pos10.alloc(std::max(nf, 1));
     k_cc_build<<<grid_for(nct, BS, 4096), BS, 0, s>>>(nct, m->cf_row.p, m->cf_col.p, m->fcells.p,
-                                                      m->cc_row.p, nullptr, m->cc_col.p, m->pos01.p,
+                                                      cc_row.p, nullptr, cc_col.p, m->pos01.p,
                                                       m->pos10.p, 1);
     FVM_HIP(hipGetLastError());
     FVM_HIP(hipStreamSynchronize(s));
@@ -1182,20 +1283,22 @@ Groups make_groups(const fvm_mesh *m, const int32_t *type, const double *value) 
 
 namespace fvm {
 namespace {
-// a system with the mesh's cellCells pattern
+// a system with the mesh's cellCells pattern, values unset
 void system_alloc(fvm_mesh *m, fvm_system *S) {
-    const int nct = m->n_cells + m->n_ghost;
+    const size_t nct = (size_t)m->n_cells + m->n_ghost, nnz = (size_t)m->nnz;
     S->device = m->device;
     S->n_self = m->n_cells;
-    S->n_total = nct;
+    S->n_total = (int)nct;
     S->nnz = m->nnz;
-    S->row.alloc((size_t)nct + 1);
-    S->col.alloc(std::max<long long>(m->nnz, 1));
-    S->off.alloc(std::max<long long>(m->nnz, 1));
-    S->diag.alloc(std::max(nct, 1)); S->b.alloc(std::max(nct, 1)); S->isb.alloc(std::max(nct, 1));
-    FVM_HIP(hipMemcpyAsync(S->row.p, m->cc_row.p, S->row.bytes(), hipMemcpyDeviceToDevice, m->stream));
-    if (m->nnz)
-        FVM_HIP(hipMemcpyAsync(S->col.p, m->cc_col.p, sizeof(int) * m->nnz, hipMemcpyDeviceToDevice, m->stream));
+    const size_t nd = (std::max<size_t>(nct, 1) + 31) / 32 * 32, no = (std::max<size_t>(nnz, 1) + 31) / 32 * 32;
+    S->block_bytes = sizeof(double) * (2 * nd + no) + nd;
+    S->store = m->store;
+    S->block = m->store->take(MeshStore::VALUES, S->block_bytes);
+    double *p = (double *)S->block;   // 256-byte boundaries
+    S->off = {p, std::max<size_t>(nnz, 1)};
+    S->diag = {p + no, std::max<size_t>(nct, 1)};
+    S->b = {p + no + nd, std::max<size_t>(nct, 1)};
+    S->isb = {(uint8_t *)(p + no + 2 * nd), std::max<size_t>(nct, 1)};
 }
 
 // ThermalModel::linearize + LinearSystem::initSolve into S (pattern already set):
@@ -1218,7 +1321,8 @@ void assemble_thermal(fvm_mesh *m, fvm_system *S, const double *d_k, const doubl
 }  // namespace
 
 // Scratch of the allocation-free re-assembly (fvm_convdiff_reassemble_noalloc): the cell
-// gradients (3 n_cells of the 2 n_faces + 3 (n_cells + n_ghost) that its size limit counts). One copy per device, held until the process ends.
+// gradients (3 n_cells of the 2 n_faces + 3 (n_cells + n_ghost) that its size limit counts).
+// One copy per device, held until the process ends.
 constexpr size_t NOALLOC_SCRATCH_DOUBLES = (size_t)1 << 22;   // 32 MiB
 static __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 
@@ -1254,25 +1358,14 @@ void mesh_device_metrics(fvm_mesh *m, const int **fcells, const double **fA, con
 
 hipStream_t mesh_stream(fvm_mesh *m) { return m->stream; }
 
-// A system with the mesh's cell-cell pattern (row and column arrays copied on the
-// mesh's stream), values unset; the caller owns it (fvm_system_destroy).
+// A system with the mesh's cell-cell pattern (shared with the mesh), values
+// unset; the caller owns it (fvm_system_destroy).
 fvm_system *system_for_mesh(fvm_mesh *m) {
     Dev d(m->device);
     mesh_metrics(m);
-    const int nct = m->n_cells + m->n_ghost;
     fvm_system *S = new fvm_system();
     try {
-        S->device = m->device;
-        S->n_self = m->n_cells;
-        S->n_total = nct;
-        S->nnz = m->nnz;
-        S->row.alloc((size_t)nct + 1);
-        S->col.alloc(std::max<long long>(m->nnz, 1));
-        S->off.alloc(std::max<long long>(m->nnz, 1));
-        S->diag.alloc(std::max(nct, 1)); S->b.alloc(std::max(nct, 1)); S->isb.alloc(std::max(nct, 1));
-        FVM_HIP(hipMemcpyAsync(S->row.p, m->cc_row.p, S->row.bytes(), hipMemcpyDeviceToDevice, m->stream));
-        if (m->nnz)
-            FVM_HIP(hipMemcpyAsync(S->col.p, m->cc_col.p, sizeof(int) * m->nnz, hipMemcpyDeviceToDevice, m->stream));
+        system_alloc(m, S);
     } catch (...) {
         delete S;
         throw;
@@ -1291,7 +1384,7 @@ void kinetic_assemble_into(fvm_mesh *m, const double *c, const double *d_nue, co
     const int nc = m->n_cells, nct = m->n_cells + m->n_ghost, nf = m->n_faces;
     k_face_conv<<<grid_for(nf, 256), 256, 0, s>>>(nf, m->fA.p, c[0], c[1], c[2], F);
     k_cell_kinetic<<<grid_for(nct, 256), 256, 0, s>>>(nc, nct, m->cf_row.p, m->cf_col.p, m->fcells.p, m->pos01.p,
-                                                      m->pos10.p, m->cc_row.p, F, m->vol.p, d_nue, d_feq, d_x,
+                                                      m->pos10.p, m->store->row.p, F, m->vol.p, d_nue, d_feq, d_x,
                                                       S->diag.p, S->off.p, S->b.p);
     FVM_HIP(hipMemsetAsync(S->isb.p, 0, nct, s));
     const int first_bface = m->gptr.size() > 1 ? m->gptr[1] : nf;
@@ -1318,8 +1411,8 @@ void kinetic_assemble_into(fvm_mesh *m, const double *c, const double *d_nue, co
 void system_post_solve_async(const fvm_system *S, double *d_delta, hipStream_t s) {
     const int ng = S->n_total - S->n_self;
     if (ng <= 0) return;
-    k_solve_boundary<false><<<grid_for(ng, 256), 256, 0, s>>>(S->n_self, S->n_total, S->row.p, S->col.p, S->diag.p,
-                                                              S->off.p, S->isb.p, S->b.p, d_delta);
+    k_solve_boundary<false><<<grid_for(ng, 256), 256, 0, s>>>(S->n_self, S->n_total, S->store->row.p, S->store->col.p,
+                                                              S->diag.p, S->off.p, S->isb.p, S->b.p, d_delta);
     FVM_HIP(hipGetLastError());
 }
 }  // namespace fvm
@@ -1448,7 +1541,7 @@ int fvm_mesh_destroy(fvm_mesh *m) {
         (void)hipStreamSynchronize(m->stream);
         m->nodes.release(); m->fnptr.release(); m->fnodes.release(); m->fcells.release(); m->gcoef.release();
         m->slot.release(); m->ent.release(); m->geo.release();
-        m->cf_row.release(); m->cf_col.release(); m->cc_row.release(); m->cc_col.release();
+        m->cf_row.release(); m->cf_col.release(); m->store.reset();
         m->pos01.release(); m->pos10.release();
         m->fA.release(); m->fAm.release(); m->fc.release(); m->cc.release(); m->vol.release();
         (void)hipStreamDestroy(m->stream);
@@ -1563,7 +1656,7 @@ int fvm_convdiff_assemble(fvm_mesh *m, const double *d_k, const double *d_source
     fvm_system *S = new fvm_system();
     try {
         fvm::system_alloc(m, S);
-        DArr<double> grad(3 * (size_t)std::max(m->n_cells, 1));
+        fvm::Scratch grad(m, fvm::scratch_doubles(m));
         fvm::assemble_thermal(m, S, d_k, d_source, d_x, d_flux, d_cont_res, central, G, grad.p);
         FVM_HIP(hipStreamSynchronize(m->stream));
     } catch (...) {
@@ -1615,20 +1708,11 @@ int fvm_phonon_assemble(fvm_mesh *m, const double *vg, double tau, const double 
     const int nc = m->n_cells, nct = m->n_cells + m->n_ghost, nf = m->n_faces;
     fvm_system *S = new fvm_system();
     try {
-        S->device = m->device;
-        S->n_self = nc;
-        S->n_total = nct;
-        S->nnz = m->nnz;
-        S->row.alloc((size_t)nct + 1);
-        S->col.alloc(std::max<long long>(m->nnz, 1));
-        S->off.alloc(std::max<long long>(m->nnz, 1));
-        S->diag.alloc(nct); S->b.alloc(nct); S->isb.alloc(nct);
-        FVM_HIP(hipMemcpyAsync(S->row.p, m->cc_row.p, S->row.bytes(), hipMemcpyDeviceToDevice, s));
-        FVM_HIP(hipMemcpyAsync(S->col.p, m->cc_col.p, sizeof(int) * m->nnz, hipMemcpyDeviceToDevice, s));
-        DArr<double> F(std::max(nf, 1));
+        fvm::system_alloc(m, S);
+        fvm::Scratch F(m, fvm::scratch_doubles(m));
         fvm::k_face_conv<<<fvm::grid_for(nf, 256), 256, 0, s>>>(nf, m->fA.p, vg[0], vg[1], vg[2], F.p);
         fvm::k_cell_phonon<<<fvm::grid_for(nct, 256), 256, 0, s>>>(
-            nc, nct, m->cf_row.p, m->cf_col.p, m->fcells.p, m->pos01.p, m->pos10.p, m->cc_row.p, F.p, m->vol.p,
+            nc, nct, m->cf_row.p, m->cf_col.p, m->fcells.p, m->pos01.p, m->pos10.p, m->store->row.p, F.p, m->vol.p,
             d_e0, d_x, tau, S->diag.p, S->off.p, S->b.p);
         const int first_bface = m->gptr.size() > 1 ? m->gptr[1] : nf;
         fvm::k_bc_phonon_interior<<<fvm::grid_for(nc, 256), 256, 0, s>>>(
@@ -1698,8 +1782,8 @@ int fvm_system_info(const fvm_system *S, int *n_self, int *n_total, long long *n
 int fvm_system_device(const fvm_system *S, const int32_t **row, const int32_t **col, const double **diag,
                       const double **off, const double **b, const uint8_t **is_boundary) {
     if (!S) return FVM_E_INVALID;
-    if (row) *row = S->row.p;
-    if (col) *col = S->col.p;
+    if (row) *row = S->store->row.p;
+    if (col) *col = S->store->col.p;
     if (diag) *diag = S->diag.p;
     if (off) *off = S->off.p;
     if (b) *b = S->b.p;
@@ -1717,14 +1801,16 @@ int fvm_system_post_solve(const fvm_system *S, double *d_delta) {
     DArr<int> flag(1);
     FVM_HIP(hipMemset(flag.p, 0, sizeof(int)));
     const unsigned g = fvm::grid_for(ng, 256);
-    fvm::k_boundary_dep<<<g, 256>>>(S->n_self, S->n_total, S->row.p, S->col.p, S->isb.p, flag.p);
+    fvm::k_boundary_dep<<<g, 256>>>(S->n_self, S->n_total, S->store->row.p, S->store->col.p, S->isb.p, flag.p);
     int dep = 0;
     FVM_HIP(hipMemcpy(&dep, flag.p, sizeof(int), hipMemcpyDeviceToHost));
     if (dep)   // a boundary row reads another one: the reference's ascending row order
-        fvm::k_solve_boundary<true><<<1, 1>>>(S->n_self, S->n_total, S->row.p, S->col.p, S->diag.p, S->off.p,
+        fvm::k_solve_boundary<true><<<1, 1>>>(S->n_self, S->n_total, S->store->row.p, S->store->col.p,
+                                              S->diag.p, S->off.p,
                                               S->isb.p, S->b.p, d_delta);
     else
-        fvm::k_solve_boundary<false><<<g, 256>>>(S->n_self, S->n_total, S->row.p, S->col.p, S->diag.p, S->off.p,
+        fvm::k_solve_boundary<false><<<g, 256>>>(S->n_self, S->n_total, S->store->row.p, S->store->col.p,
+                                              S->diag.p, S->off.p,
                                                  S->isb.p, S->b.p, d_delta);
     FVM_HIP(hipGetLastError());
     FVM_HIP(hipDeviceSynchronize());
@@ -1737,8 +1823,8 @@ int fvm_system_get(const fvm_system *S, int32_t *row, int32_t *col, double *diag
     FVM_API_BEGIN
     FVM_CHECK(S, FVM_E_INVALID, "null system");
     fvm::Dev d(S->device);
-    if (row) FVM_HIP(hipMemcpy(row, S->row.p, S->row.bytes(), hipMemcpyDeviceToHost));
-    if (col && S->nnz) FVM_HIP(hipMemcpy(col, S->col.p, sizeof(int) * S->nnz, hipMemcpyDeviceToHost));
+    if (row) FVM_HIP(hipMemcpy(row, S->store->row.p, S->store->row.bytes(), hipMemcpyDeviceToHost));
+    if (col && S->nnz) FVM_HIP(hipMemcpy(col, S->store->col.p, sizeof(int) * S->nnz, hipMemcpyDeviceToHost));
     if (diag) FVM_HIP(hipMemcpy(diag, S->diag.p, S->diag.bytes(), hipMemcpyDeviceToHost));
     if (off && S->nnz) FVM_HIP(hipMemcpy(off, S->off.p, sizeof(double) * S->nnz, hipMemcpyDeviceToHost));
     if (b) FVM_HIP(hipMemcpy(b, S->b.p, S->b.bytes(), hipMemcpyDeviceToHost));
@@ -1750,10 +1836,7 @@ int fvm_system_get(const fvm_system *S, int32_t *row, int32_t *col, double *diag
 int fvm_system_destroy(fvm_system *S) {
     FVM_API_BEGIN
     if (!S) return FVM_OK;
-    {
-        fvm::Dev d(S->device);
-        S->row.release(); S->col.release(); S->diag.release(); S->off.release(); S->b.release(); S->isb.release();
-    }
+    fvm::Dev d(S->device);
     delete S;
     return FVM_OK;
     FVM_API_END
@@ -1763,7 +1846,8 @@ int fvm_amg_setup_system(fvm_amg *h, const fvm_system *S) {
     FVM_API_BEGIN
     FVM_CHECK(h && S, FVM_E_INVALID, "null argument");
     FVM_CHECK(h->device == S->device, FVM_E_INVALID, "system and solver on different devices");
-    return fvm_amg_setup_device(h, S->n_self, S->n_total, S->row.p, S->col.p, S->diag.p, S->off.p, S->isb.p);
+    return fvm_amg_setup_device(h, S->n_self, S->n_total, S->store->row.p, S->store->col.p, S->diag.p, S->off.p,
+                                S->isb.p);
     FVM_API_END
 }
 

@@ -129,6 +129,29 @@ def test_row_kernels_on_general_graphs(n, degree):
             np.testing.assert_array_equal(S[key], o[key], err_msg=key)
 
 
+@pytest.mark.parametrize("alive", [1, 2, 4])
+def test_systems_of_a_mesh_share_only_the_pattern(alive):
+    """Systems of one mesh that live side by side, are dropped in another order than made (one block of
+    values is kept for the next one) and outlive the mesh: each keeps the values it was assembled with."""
+    from fvm_amd.thermal import Mesh, assemble
+    m = Mesh.hex(6, 0.2, 3)
+    k, s, x = _dev_fields(m, 1.0, 1, 3)
+    live, seen = [], []
+    for i in range(3 * alive):
+        live.append((assemble(m, k * (1.0 + i), s, x, BC_T, BC_V), i))
+        if len(live) > alive:
+            live.pop((7 * i) % len(live))
+        seen.append(live[-1][0].to_host())
+    ref = O.fv_thermal(hexmesh.hex_mesh(6, 0.2, 3), k.cpu().numpy(), s.cpu().numpy(), x.cpu().numpy(), BC_T, BC_V)
+    del m
+    for S, i in live:
+        h = S.to_host()
+        for key in ("row", "col", "diag", "off", "b", "is_boundary"):
+            np.testing.assert_array_equal(h[key], seen[i][key])
+        np.testing.assert_array_equal(h["col"], ref["col"])
+    np.testing.assert_array_equal(seen[0]["off"], ref["off"])
+
+
 def test_amg_on_device_assembled_system_exact():
     import torch
     import fvm_amd
