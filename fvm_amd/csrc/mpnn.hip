@@ -162,7 +162,7 @@ __global__ void k_mp_h0(int n, const int *__restrict__ row, const int *__restric
             for (int u = 0; u < 8; u++) x[u] = j[u] >= 0 ? v[j[u]] : 0.f;
 #pragma unroll
             for (int u = 0; u < 8; u++)
-                if (p + u < re) a = fmaf(w[u], x[u], a);
+                if (p + u < re) a += w[u] * x[u];
         }
         h0[i] = make_uint2(pack2(v[i], a), pack2(l[i], 0.f));
     }
@@ -174,8 +174,8 @@ __device__ __forceinline__ float hi16(unsigned u) { return __uint_as_float(u & 0
 __device__ __forceinline__ void add8(float *acc, float w, u32x4 q) {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        acc[2 * k] = fmaf(w, lo16(q[k]), acc[2 * k]);
-        acc[2 * k + 1] = fmaf(w, hi16(q[k]), acc[2 * k + 1]);
+        acc[2 * k] += w * lo16(q[k]);
+        acc[2 * k + 1] += w * hi16(q[k]);
     }
 }
 __device__ __forceinline__ u32x4 pack8(const float *a) {
@@ -185,6 +185,33 @@ __device__ __forceinline__ u32x4 pack8(const float *a) {
     return q;
 }
 __device__ __forceinline__ bf16x8 frag(u32x4 q) { return __builtin_bit_cast(bf16x8, q); }
+
+// Aggregate of the input features, one node per thread (in the layer the four lanes of a node
+// would each gather all of it: 763,560 nodes 63 us, against 35 us and 17 us for this launch).
+__global__ void k_mp_a0(int n, const int *__restrict__ row, const int *__restrict__ col, const float *__restrict__ c,
+                        const uint2 *__restrict__ h0, uint2 *__restrict__ a0) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int rb = row[i], re = row[i + 1];
+        float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+        for (int p = rb; p < re; p += 4) {   // four entries in flight, added in order
+            uint2 g[4];
+            float w[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                g[u] = h0[p + u < re ? col[p + u] : i];
+                w[u] = p + u < re ? c[p + u] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (p + u < re) {
+                    s0 += w[u] * lo16(g[u].x);
+                    s1 += w[u] * hi16(g[u].x);
+                    s2 += w[u] * lo16(g[u].y);
+                }
+        }
+        a0[i] = make_uint2(pack2(s0, s1), pack2(s2, 0.f));
+    }
+}
 
 // Tiles of 16 nodes, one per wavefront and step. Blocks are handed to the 8 XCDs in turn,
 // so block b works on eighth b % 8 of the tiles, and its blocks walk through that eighth
@@ -204,7 +231,8 @@ struct MpTiles {
 
 // One layer:  a_i = sum_p c_p h_col(p)  (FP32 sums, then bf16; kept for the backward pass)
 //             h'_i = relu([h_i | a_i] W^T + b), W row o = [Ws(o,:) | Wn(o,:)] (bf16)
-// The products run as v_mfma_f32_16x16x32_bf16 with the weights as the first operand (lane l:
+// Every value that is rounded to bf16 is summed in this order, entries ascending and the bias
+// last: another order moves some over a rounding boundary (1e-5 of a loss). The products run as v_mfma_f32_16x16x32_bf16 with the weights as the first operand (lane l:
 // output l%16, k = 8(l/16)..+8) and the nodes as the second (node l%16, same k), so lane l
 // gathers for node l%16 exactly the features that it feeds to the matrix cores, and ends
 // with four consecutive outputs of its node per output block (rows 4(l/16)..+4). The
@@ -212,7 +240,8 @@ struct MpTiles {
 // wavefronts per SIMD. LAST: the readout e = s (wo . h' + bo) is taken from the registers;
 // h' is stored only for a backward pass. What bounds it: the gathers, 128 bytes per entry.
 // 763,560 nodes (7-point rows): layer 64 -> 64 165 -> 129 us, the last one with its readout
-// 260 -> 120 us (146 and 110 MB from memory, 10 and 7 million L2 accesses), layer 0 68 -> 41 us.
+// 260 -> 120 us (146 and 110 MB from memory, 10 and 7 million L2 accesses), layer 0 68 -> 35 us
+// (and k_mp_a0 17 us).
 // Weights in registers over several tiles: 142 us (3 wavefronts per SIMD). Stores and
 // column reads that bypass the caches, or 96 blocks instead of 192 per XCD: slower.
 template <int FIN, bool LAST>
@@ -241,31 +270,8 @@ k_mp_layer(int n, const int *__restrict__ row, const int *__restrict__ col, cons
         const int rb = row[ic], re = row[ic + 1];
         bf16x8 x[NK];
         if constexpr (FIN == MF0) {
-            // three features: k 0..7 (lanes q = 0) hold h, k 16..23 (q = 2) hold a; the four
-            // lanes of a node share its entries
-            const uint2 *H = (const uint2 *)Hv;
-            float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-            for (int p = rb + q; p < re; p += 8) {
-                const bool two = p + 4 < re;
-                const int j0 = col[p], j1 = two ? col[p + 4] : j0;
-                const float w0 = c[p], w1 = two ? c[p + 4] : 0.f;
-                const uint2 h0 = H[j0], h1 = H[j1];
-                a0 = fmaf(w0, lo16(h0.x), a0);
-                a1 = fmaf(w0, hi16(h0.x), a1);
-                a2 = fmaf(w0, lo16(h0.y), a2);
-                if (two) {
-                    a0 = fmaf(w1, lo16(h1.x), a0);
-                    a1 = fmaf(w1, hi16(h1.x), a1);
-                    a2 = fmaf(w1, lo16(h1.y), a2);
-                }
-            }
-            for (int o = 16; o < 64; o <<= 1) {
-                a0 += __shfl_xor(a0, o, 64);
-                a1 += __shfl_xor(a1, o, 64);
-                a2 += __shfl_xor(a2, o, 64);
-            }
-            const uint2 hi = H[ic], ai = make_uint2(pack2(a0, a1), pack2(a2, 0.f));
-            if (Aout && q == 2 && i < n) ((uint2 *)Aout)[i] = ai;
+            // three features: k 0..7 (lanes q = 0) hold h, k 16..23 (q = 2) hold a (k_mp_a0)
+            const uint2 hi = ((const uint2 *)Hv)[ic], ai = ((const uint2 *)Aout)[ic];
             const u32x4 z = {q == 0 ? hi.x : q == 2 ? ai.x : 0u, q == 0 ? hi.y : q == 2 ? ai.y : 0u, 0u, 0u};
             x[0] = frag(z);
         } else {
@@ -307,13 +313,17 @@ k_mp_layer(int n, const int *__restrict__ row, const int *__restrict__ col, cons
         float y = 0.f;
 #pragma unroll
         for (int ob = 0; ob < 4; ob++) {
-            f32x4 d = bs[ob * 4 + q];
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kk = 0; kk < NK; kk++)
                 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(ws[(ob * NK + kk) * 64 + lane]), x[kk], d, 0, 0, 0);
+            const f32x4 bias4 = bs[ob * 4 + q];
             float h[4];
 #pragma unroll
-            for (int t = 0; t < 4; t++) h[t] = d[t] > 0.f ? d[t] : 0.f;
+            for (int t = 0; t < 4; t++) {
+                const float z = d[t] + bias4[t];
+                h[t] = z > 0.f ? z : 0.f;
+            }
             const uint2 st = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
             if (Hn && i < n) *reinterpret_cast<uint2 *>(Hn + (size_t)i * MH + ob * 16 + 4 * q) = st;
             if (LAST) {
@@ -747,6 +757,7 @@ void mp_forward(fvm_mpnn *m, const double *r, double *e_out, int accumulate, boo
     k_mp_scale<<<1, BSZ, 0, st>>>(n, (int)nb, m->dpart.p, m->s.p);
     k_mp_v<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, r, m->diag, m->s.p, m->v.p);
     k_mp_h0<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->v.p, m->l.p, (uint2 *)m->H[0].p);
+    k_mp_a0<<<grid_for(n, BSZ), BSZ, 0, st>>>(n, m->row, m->col, m->c.p, (const uint2 *)m->H[0].p, (uint2 *)m->A[0].p);
     FVM_HIP(hipMemsetAsync(m->flag.p, 0, sizeof(int), st));
     const unsigned gl = mp_grid(n);
     for (int k = 0; k < MLAYERS; k++) {
@@ -754,7 +765,7 @@ void mp_forward(fvm_mpnn *m, const double *r, double *e_out, int accumulate, boo
         const bool last = k == MLAYERS - 1;
         auto launch = [&](auto kern) {
             kern<<<gl, BSZ, 0, st>>>(n, m->row, m->col, m->c.p, m->H[k].p, m->wbf[k].p, bias,
-                                     keep ? m->A[k].p : nullptr, (!last || keep) ? m->H[k + 1].p : nullptr,
+                                     k == 0 || keep ? m->A[k].p : nullptr, (!last || keep) ? m->H[k + 1].p : nullptr,
                                      m->theta.p + WO_OFF, m->s.p, e_out, accumulate, m->flag.p);
         };
         if (k == 0) launch(k_mp_layer<MF0, false>);
