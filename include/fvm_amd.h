@@ -195,9 +195,9 @@ int fvm_amg_kernel_timing(const fvm_amg *h, int kind, long long *launches, doubl
 int fvm_amg_kernel_bytes(const fvm_amg *h, int kind, double *total_bytes);
 /* Performance knobs that never change results (no reference counterpart; set
  * by the autotuner): "tail_max_rows" -- V-cycle levels with at most this many
- * rows run in one single-workgroup launch (0 disables); "tail_lds" -- 1
- * (default): there, a level whose matrix and vectors fit in the workgroup's LDS
- * is swept from LDS; "sell_block" -- threads
+ * rows run in one single-workgroup launch (default 6000; 0 disables);
+ * "tail_lds" -- 1 (default): there, levels are packed in the order of the sweeps
+ * and those that fit stay in the workgroup's LDS; "sell_block" -- threads
  * per block of the SELL-64 smoother kernels, "spmv_block" -- of the SELL-64
  * residual and SpMV kernels (64/128/256/512 each); "sell_xcd" / "spmv_xcd" --
  * 1: blocks of those kernels are renumbered so that each of the chip's 8 XCDs
