@@ -232,7 +232,8 @@ struct MpTiles {
 // One layer:  a_i = sum_p c_p h_col(p)  (FP32 sums, then bf16; kept for the backward pass)
 //             h'_i = relu([h_i | a_i] W^T + b), W row o = [Ws(o,:) | Wn(o,:)] (bf16)
 // Every value that is rounded to bf16 is summed in this order, entries ascending and the bias
-// last: another order moves some over a rounding boundary (1e-5 of a loss). The products run as v_mfma_f32_16x16x32_bf16 with the weights as the first operand (lane l:
+// last: another order moves some over a rounding boundary (1e-5 of a loss).
+// The products run as v_mfma_f32_16x16x32_bf16 with the weights as the first operand (lane l:
 // output l%16, k = 8(l/16)..+8) and the nodes as the second (node l%16, same k), so lane l
 // gathers for node l%16 exactly the features that it feeds to the matrix cores, and ends
 // with four consecutive outputs of its node per output block (rows 4(l/16)..+4). The
