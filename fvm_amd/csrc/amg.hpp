@@ -47,8 +47,8 @@ struct Level {
     struct SweepRun { int lvl0, nlev, width; bool wg; };
     std::vector<SweepRun> fwd_runs, bwd_runs;
     int runs_width = -1;
-    // packed schedules of the one-workgroup sweep, forward and backward, and the precision
-    // they were built for (-1: not used on this level)
+    // packed schedules of the one-workgroup sweep, forward and backward, the precision they
+    // were built for (-1: not used on this level) and the one last considered
     struct FlowPack {
         int nitem = 0;
         DArr<int> items, code;
@@ -56,7 +56,7 @@ struct Level {
     };
     FlowPack flow[2];
     DArr<unsigned char> flow_vec;   // b and two copies of x in schedule order
-    int flow_prec = -1, flow_groups = 0;   // (groups of four entries of its longest row)
+    int flow_prec = -1, flow_tried = -1, flow_groups = 0;   // (groups of four entries of its longest row)
     // coloured SELL layout
     bool fast_ready = false;
     int sell_u = 8;              // load depth of the SELL-64 row kernels (mean slice width, rounded up to 8/16/32)

@@ -611,6 +611,11 @@ int fvm_amg_get_tuning(const fvm_amg *h, const char *key, long long *value) {
     else if (k == "reuse_setup") *value = h->reuse_setup;
     else if (k == "setups_reused") *value = h->setup_reused;
     else if (k == "exact_flow_spin_limit") *value = h->flow_spin_limit;
+    else if (k == "exact_flow_wg_levels") {
+        *value = 0;
+        for (size_t l = 0; l < h->lev.size() && l < 63; l++)
+            if (h->exact_flow && h->lev[l].flow_prec == (h->prm.precision == FVM_PREC_MIXED ? 1 : 0)) *value |= 1LL << l;
+    }
     else return FVM_E_INVALID;
     return FVM_OK;
 }

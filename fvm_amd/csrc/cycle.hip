@@ -340,6 +340,11 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // is read after the wait, which costs the hop a round trip to memory.
 constexpr int FL_ITEMS = 12;        // items per dependency level, on average, up to which one workgroup is used
 constexpr int FL_ROWS = 150000;
+// An item is padded to its longest row: a level whose packs would hold more groups than it has
+// entries and rows together (7-point rows reach 0.3 of that, coarse levels 0.4; an item of one
+// hub and 63 short rows may need 64 times its entries) is left to the chip-wide sweep, which
+// reads the matrix as it lies.
+constexpr unsigned long long FL_GROUPS = 1ull << 28;   // and 32-bit positions of groups hold
 constexpr int FL_OWN_ROWS = 4096;   // up to here the kernel reorders x and b itself (8 rows per thread)
 constexpr int FL_NW = 8;   // wavefronts (twelve were slower: 44k rows, 620 against 510 us a sweep)
 template <class X> constexpr int fl_ring() { return sizeof(X) == 8 ? 4096 : 8192; }
@@ -355,7 +360,7 @@ constexpr int FL_NEW = (int)0x80000000, FL_FAR = 0x40000000, FL_IDX = 0x3fffffff
 template <class V, class X, bool FILL>
 __global__ void __launch_bounds__(64)
 k_flow_pack(int n, int dir, int4 *items, const int *lvl_end, const int *rows, const int *place, const int *row,
-            const int *col, const V *off, const X *diag, int *total, int4 *code, X *val, X *dg) {   // total: groups, longest item
+            const int *col, const V *off, const X *diag, unsigned long long *total, int4 *code, X *val, X *dg) {   // total: groups, longest item
     constexpr int R = fl_ring<X>();
     int4 t = items[blockIdx.x];
     const int np = t.y & 0xff, lane = threadIdx.x;
@@ -368,8 +373,8 @@ k_flow_pack(int n, int dir, int4 *items, const int *lvl_end, const int *rows, co
         if (lane == 0) {
             const int ng = max(1, (m + 3) / 4);   // (rows without entries: one group of padding)
             t.y = np | ng << 8;
-            t.w = atomicAdd(total, np * ng);
-            atomicMax(total + 1, ng);
+            t.w = (int)atomicAdd(total, (unsigned long long)np * ng);   // (a level past FL_GROUPS is not packed)
+            atomicMax(total + 1, (unsigned long long)ng);
             items[blockIdx.x] = t;
         }
         return;
@@ -2101,7 +2106,7 @@ void prepare_flow_packs(Run &R) {
     std::vector<DArr<int>> place(h->lev.size());
     for (int l = 0; l < (int)h->lev.size(); l++) {
         Level &L = h->lev[l];
-        if (L.flow_prec == prec) continue;
+        if (L.flow_tried == prec) continue;
         L.flow_prec = -1;
         // a value leaves the ring well after it was stored: more items later than there are wavefronts
         if (L.n == 0 || L.n > FL_ROWS || std::max(L.fwd_maxw, L.bwd_maxw) + 64 * (FL_NW + 1) > RING) continue;
@@ -2123,7 +2128,10 @@ void prepare_flow_packs(Run &R) {
             }
         }
     }
-    if (jobs.empty()) return;
+    auto finish = [&]() {
+        for (Level &L : h->lev) L.flow_tried = prec;
+    };
+    if (jobs.empty()) return finish();
     // the device's LDS for the kernel, granted once (outside any capture)
     FVM_HIP(hipFuncSetAttribute((const void *)k_gs_flow_wg<X, FL_NW, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)fl_lds<X, FL_NW, 2>()));
@@ -2131,7 +2139,7 @@ void prepare_flow_packs(Run &R) {
                                 (int)fl_lds<X, FL_NW, 4>()));
     FVM_HIP(hipFuncSetAttribute((const void *)k_gs_flow_wg<X, FL_NW, 6>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)fl_lds<X, FL_NW, 6>()));
-    DArr<int> total(2 * jobs.size());
+    DArr<unsigned long long> total(2 * jobs.size());
     FVM_HIP(hipMemsetAsync(total.p, 0, total.bytes(), s));
     auto launch = [&](Job &J, int k, bool fill) {
         Level &L = h->lev[J.l];
@@ -2165,29 +2173,37 @@ void prepare_flow_packs(Run &R) {
         J.d_lend.alloc(J.lend.size());
         if (J.dir == 0) {
             place[J.l].alloc(L.n);
-            L.flow_vec.alloc(3 * sizeof(X) * (size_t)L.n);
             k_flow_place<<<grid_for(L.n, BS, 4096), BS, 0, s>>>(L.n, L.fwd_rows.p, place[J.l].p);
         }
         FVM_HIP(hipMemcpyAsync(P.items.p, J.items.data(), sizeof(int4) * J.items.size(), hipMemcpyHostToDevice, s));
         FVM_HIP(hipMemcpyAsync(J.d_lend.p, J.lend.data(), sizeof(int) * J.lend.size(), hipMemcpyHostToDevice, s));
         launch(J, (int)k, false);
     }
-    std::vector<int> ht(2 * jobs.size());
+    std::vector<unsigned long long> ht(2 * jobs.size());
     FVM_HIP(hipMemcpyAsync(ht.data(), total.p, total.bytes(), hipMemcpyDeviceToHost, s));
     FVM_HIP(hipStreamSynchronize(s));
     for (size_t k = 0; k < jobs.size(); k++) {
-        Job &J = jobs[k];
-        Level::FlowPack &P = h->lev[J.l].flow[J.dir];
-        const size_t g = std::max(ht[2 * k], 1);
+        Job &J = jobs[k];   // (a level's forward job, then its backward one)
         Level &L = h->lev[J.l];
-        L.flow_groups = J.dir ? std::max(L.flow_groups, ht[2 * k + 1]) : ht[2 * k + 1];
+        Level::FlowPack &P = L.flow[J.dir];
+        const size_t kf = k - J.dir;
+        const unsigned long long most = std::max(ht[2 * kf], ht[2 * kf + 2]);
+        if (most > (unsigned long long)L.nnz + L.n || most > FL_GROUPS) {
+            P = Level::FlowPack{};
+            continue;
+        }
+        const size_t g = ht[2 * k];
+        if (J.dir == 0) L.flow_vec.alloc(3 * sizeof(X) * (size_t)L.n);
+        L.flow_groups = (int)std::max(ht[2 * kf + 1], ht[2 * kf + 3]);
         P.code.alloc(4 * g);
         P.val.alloc(4 * sizeof(X) * g);
         P.dg.alloc(sizeof(X) * (size_t)h->lev[J.l].n);
         launch(J, (int)k, true);
     }
     FVM_HIP(hipStreamSynchronize(s));
-    for (Job &J : jobs) h->lev[J.l].flow_prec = prec;
+    for (Job &J : jobs)
+        if (h->lev[J.l].flow[J.dir].nitem) h->lev[J.l].flow_prec = prec;
+    finish();
 }
 
 Run make_run(fvm_amg *h) {

@@ -71,6 +71,40 @@ def test_one_workgroup_reference_sweep_is_bit_identical(case, prec, npost):
     assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
 
 
+def bundle(n, hub, seed=0):
+    """Rows in bundles of 64, each linked to the same row of the bundle before (a dependency level per
+    bundle); the first row of every bundle reads ``hub`` rows of earlier bundles besides."""
+    rng = np.random.default_rng(seed)
+    rows = []
+    for i in range(n):
+        c = {j for j in (i - 64, i + 64) if 0 <= j < n}
+        if hub and i % 64 == 0 and i > 64:
+            c |= {int(j) for j in rng.integers(0, i - i % 64, hub)}
+        rows.append(sorted(c))
+    row = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    off = rng.uniform(0.1, 1.0, row[-1])
+    diag = np.array([-1.1 * off[row[i]:row[i + 1]].sum() - 0.1 for i in range(n)])
+    return dict(n_self=n, n_total=n, row=row, col=np.array([c for r in rows for c in r], np.int32), diag=diag,
+                off=off, b=rng.uniform(-1, 1, n))
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("hub,used", [(0, True), (300, False)])
+def test_level_with_hub_rows_is_not_padded_to_them(prec, hub, used):
+    """Items of one hub and 63 short rows: 64 rows padded to 300 entries each would be nine times the
+    entries and rows of the level (limit: once), so the chip-wide sweep keeps it. Same bits either way."""
+    m = bundle(2560, hub)
+    res = []
+    for flow in (0, 1):
+        a = gpu_amg(gsOrdering=0, precision=prec, nMaxIterations=6, relativeTolerance=1e-30)
+        a.set_tuning("exact_flow", flow)
+        ls = ls_from(m)
+        a.solve(ls)
+        res.append((ls.delta.copy(), a.history()))
+        assert a.get_tuning("exact_flow_wg_levels") & 1 == (flow and used)
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+
+
 @pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 127, 255, 256])
 def test_direct_level_inverse_at_panel_edges(n):
     """The blocked inverse of the direct level, at the edges of its panels and at its limit."""
