@@ -170,6 +170,7 @@ struct fvm_amg {
     long long setup_reused = 0;        // setups skipped that way
     bool parked = false;               // cleanup kept the hierarchy for such a setup
     int exact_flow = 1;                // reference-order sweeps as one dataflow launch per direction
+    int flow_wg_rows = 150000;         // levels up to this many rows may sweep in one workgroup (k_gs_flow_wg)
     fvm::DArr<int> flow_ctl;           // its block tickets, finished blocks and error flag
     bool flow_used = false;            // a dataflow sweep ran since the last check
     long long flow_ticks = 0;          // two seconds of the device's wall clock

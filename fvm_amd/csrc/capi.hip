@@ -559,7 +559,10 @@ int fvm_amg_set_tuning(fvm_amg *h, const char *key, long long value) {
     } else if (k == "exact_flow_spin_limit") {
         FVM_CHECK(value >= 0 && value <= INT_MAX, FVM_E_INVALID, "exact_flow_spin_limit must be in [0, INT_MAX]");
         h->flow_spin_limit = (int)value;
-
+    } else if (k == "exact_flow_wg_rows") {
+        FVM_CHECK(value >= 0 && value <= INT_MAX, FVM_E_INVALID, "exact_flow_wg_rows must be in [0, INT_MAX]");
+        h->flow_wg_rows = (int)value;
+        for (auto &L : h->lev) L.flow_tried = -1;   // decided anew by the next solve
     } else if (k == "bipartite_levels") {
         FVM_CHECK(value >= 0 && value <= 64, FVM_E_INVALID, "bipartite_levels must be in [0, 64]");
         h->bipartite_levels = (int)value;
@@ -611,6 +614,7 @@ int fvm_amg_get_tuning(const fvm_amg *h, const char *key, long long *value) {
     else if (k == "reuse_setup") *value = h->reuse_setup;
     else if (k == "setups_reused") *value = h->setup_reused;
     else if (k == "exact_flow_spin_limit") *value = h->flow_spin_limit;
+    else if (k == "exact_flow_wg_rows") *value = h->flow_wg_rows;
     else if (k == "exact_flow_wg_levels") {
         *value = 0;
         for (size_t l = 0; l < h->lev.size() && l < 63; l++)

@@ -329,8 +329,8 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // The price is one CU's throughput (about 20 GB/s of what its L2 does not hold), so b and
 // x are first brought into the order of the schedule: rows of one dependency level side
 // by side, sorted, their neighbours nearly so (44k rows: 510 -> 320 us a sweep). An item
-// takes 0.2 us, a hop across the chip about 2.9 us: past FL_ITEMS items per dependency level, and past FL_ROWS rows, whose entries
-// come from HBM, the whole chip is faster (210,000 rows, 7 items per level: 1.3 ms slower
+// takes 0.2 us, a hop across the chip about 2.9 us: past FL_ITEMS items per dependency level, and past
+// exact_flow_wg_rows (150,000) rows, whose entries come from HBM, the whole chip is faster (210,000 rows, 7 items per level: 1.3 ms slower
 // per sweep here). Milliseconds per V-cycle against chip-wide sweeps on every level:
 // 27,000 rows 1.31 / 5.08, 125,000 rows 3.7 / 11.1, 729,000 rows 15.6 / 26.2.
 // One schedule serves both directions: its reverse is a valid order of the backward sweep.
@@ -339,7 +339,6 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // (each costs registers and LDS words for the entries' old values). An entry past those
 // is read after the wait, which costs the hop a round trip to memory.
 constexpr int FL_ITEMS = 12;        // items per dependency level, on average, up to which one workgroup is used
-constexpr int FL_ROWS = 150000;
 // An item is padded to its longest row: a level whose packs would hold more groups than it has
 // entries and rows together (7-point rows reach 0.3 of that, coarse levels 0.4; an item of one
 // hub and 63 short rows may need 64 times its entries) is left to the chip-wide sweep, which
@@ -2108,8 +2107,10 @@ void prepare_flow_packs(Run &R) {
         Level &L = h->lev[l];
         if (L.flow_tried == prec) continue;
         L.flow_prec = -1;
+        for (Level::FlowPack &P : L.flow) P = Level::FlowPack{};
+        L.flow_vec.release();
         // a value leaves the ring well after it was stored: more items later than there are wavefronts
-        if (L.n == 0 || L.n > FL_ROWS || std::max(L.fwd_maxw, L.bwd_maxw) + 64 * (FL_NW + 1) > RING) continue;
+        if (L.n == 0 || L.n > h->flow_wg_rows || std::max(L.fwd_maxw, L.bwd_maxw) + 64 * (FL_NW + 1) > RING) continue;
         long long nitem = 0;
         for (int k = 0; k < L.fwd_nlev; k++) nitem += (L.h_fwd_ptr[k + 1] - L.h_fwd_ptr[k] + 63) / 64;
         if (nitem > (long long)FL_ITEMS * L.fwd_nlev) continue;

@@ -239,6 +239,9 @@ int fvm_amg_kernel_bytes(const fvm_amg *h, int kind, double *total_bytes);
  * "exact_flow_spin_limit" -- waits per wavefront after which such a sweep gives
  * up and the call fails with FVM_E_NUMERIC (default 0: no bound; a sweep that
  * sees no progress for two seconds gives up regardless);
+ * "exact_flow_wg_rows" -- such sweeps of levels of at most this many rows run
+ * inside one workgroup where their dependency levels are narrow enough (default
+ * 150000; 0: every level is swept by the whole chip);
  * "exact_flow_wg_levels" (read only) -- bit l: level l is swept by a single
  * workgroup (known once the handle has solved or smoothed in that order);
  * "exact_wg_width" -- in level-by-level reference-order sweeps, each run of

@@ -394,21 +394,27 @@ def test_autotune_keeps_results(prec):
 
 @pytest.mark.parametrize("cycle", [0, 1, 2])
 def test_reference_order_sweep_in_one_workgroup_is_bit_identical(cycle):
-    """The reference-order smoother runs as one dataflow launch per sweep
-    direction (exact_flow 1: each row updates once the rows it reads new values
-    of have published theirs), or level by level (exact_flow 0): each stretch of
-    narrow dependency levels (at most exact_wg_width rows) in one workgroup and
-    wider levels one launch each. Every variant gives the oracle's bits, so all
-    give the same delta and history (widths 8, 64, 200: sweeps that mix both
-    launch kinds)."""
+    """The reference-order smoother runs inside one workgroup (exact_flow 1, levels
+    of narrow dependency levels up to exact_flow_wg_rows rows), as one dataflow
+    launch per sweep direction over the chip (exact_flow 1, other levels: each row
+    updates once the rows it reads new values of have published theirs), or level
+    by level (exact_flow 0): each stretch of narrow dependency levels (at most
+    exact_wg_width rows) in one workgroup and wider levels one launch each. Every
+    variant gives the oracle's bits, so all give the same delta and history
+    (widths 8, 64, 200: sweeps that mix both launch kinds; 600 rows: coarse levels
+    in one workgroup below levels over the chip)."""
     m = matgen.grid3d(20, seed=29, contrast=1.5)
     out = []
-    for flow, width in ((1, 256), (0, 0), (0, 8), (0, 64), (0, 200), (0, 4096), (0, 1 << 30)):
+    for flow, width, wg_rows in ((1, 256, 150000), (1, 256, 0), (1, 256, 600), (0, 0, 0), (0, 8, 0), (0, 64, 0),
+                                 (0, 200, 0), (0, 4096, 0), (0, 1 << 30, 0)):
         ga = gpu_amg(gsOrdering=0, cycleType=cycle, nMaxIterations=12, relativeTolerance=1e-30)
         ga.set_tuning("exact_flow", flow)
         ga.set_tuning("exact_wg_width", width)
+        ga.set_tuning("exact_flow_wg_rows", wg_rows)
         ls = ls_from(m)
         ga.solve(ls)
+        swept = [l for l in range(ga.num_levels()) if flow and ga.level(l)["n"] <= wg_rows]
+        assert ga.get_tuning("exact_flow_wg_levels") == sum(1 << l for l in swept)
         out.append((ls.delta.copy(), ga.history()))
     want = oracle_for(m, n_max_iterations=12, relative_tolerance=1e-30, cycle_type=cycle).solve(m["b"])
     for d, hist in out:
@@ -508,14 +514,17 @@ def test_opt_in_setup_reuse_gives_the_rebuilt_results():
     assert ga.get_tuning("setups_reused") == 2 and ga.num_levels() == 4
 
 
-def test_dataflow_sweep_bounded_wait_fails_loudly_then_recovers():
-    """A reference-order dataflow sweep whose wavefronts may wait only once
+@pytest.mark.parametrize("wg_rows", [150000, 0])
+def test_dataflow_sweep_bounded_wait_fails_loudly_then_recovers(wg_rows):
+    """A reference-order dataflow sweep (in one workgroup, and over the chip:
+    exact_flow_wg_rows 0) whose wavefronts may wait only once
     (exact_flow_spin_limit 1) gives up through its own bounded wait: the call
     fails with the sweep's error, every kernel exits normally, and the next call
     without the bound gives the oracle's bits again."""
     from fvm_amd._lib import FVM_E_NUMERIC, FvmError
     m = matgen.grid3d(10, seed=30)
     ga = gpu_amg(gsOrdering=0, nMaxIterations=5, relativeTolerance=1e-30)
+    ga.set_tuning("exact_flow_wg_rows", wg_rows)
     ga.set_tuning("exact_flow_spin_limit", 1)
     for call in ("smooth", "solve"):
         with pytest.raises(FvmError, match="stopped waiting") as e:

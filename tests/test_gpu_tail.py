@@ -59,16 +59,22 @@ FLOW = {"chain300": lambda: matgen.chain(300, d=-2.1), "grid4": lambda: matgen.g
 @pytest.mark.parametrize("prec,npost", [(0, 1), (1, 1), (0, 2)])
 @pytest.mark.parametrize("case", sorted(FLOW))
 def test_one_workgroup_reference_sweep_is_bit_identical(case, prec, npost):
-    """Reference-order sweeps by one workgroup against the level-by-level launches."""
+    """Reference-order sweeps by one workgroup (every level of these is swept by it) and by the whole
+    chip (exact_flow_wg_rows 0) against the level-by-level launches."""
     m = FLOW[case]()
     res = []
-    for flow in (0, 1):
+    for flow, wg_rows in ((0, 0), (1, 150000), (1, 0)):
         a = gpu_amg(gsOrdering=0, precision=prec, nPostSweeps=npost, nMaxIterations=6, relativeTolerance=1e-30)
         a.set_tuning("exact_flow", flow)
+        a.set_tuning("exact_flow_wg_rows", wg_rows)
         ls = ls_from(m)
         a.solve(ls)
         res.append((ls.delta.copy(), a.history()))
-    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+        # an empty level is not swept at all
+        swept = [l for l in range(a.num_levels()) if flow and 0 < a.level(l)["n"] <= wg_rows]
+        assert a.get_tuning("exact_flow_wg_levels") == sum(1 << l for l in swept)
+    for d, h in res[1:]:
+        assert np.array_equal(res[0][0], d) and np.array_equal(res[0][1], h)
 
 
 def bundle(n, hub, seed=0):
