@@ -339,11 +339,16 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // (each costs registers and LDS words for the entries' old values). An entry past those
 // is read after the wait, which costs the hop a round trip to memory.
 constexpr int FL_ITEMS = 12;        // items per dependency level, on average, up to which one workgroup is used
-// An item is padded to its longest row: a level whose packs would hold more groups than it has
-// entries and rows together (7-point rows reach 0.3 of that, coarse levels 0.4; an item of one
-// hub and 63 short rows may need 64 times its entries) is left to the chip-wide sweep, which
-// reads the matrix as it lies.
-constexpr unsigned long long FL_GROUPS = 1ull << 28;   // and 32-bit positions of groups hold
+// Longer rows do not move that line, the chip-wide sweep slows down more (rows past its
+// registers are polled entry by entry): 25 entries, 140,608 rows, 6.7 items per level 3.3 ms
+// a sweep here against 9.9, 113 entries, 64,000 rows 25 against 89.
+// An item is padded to its longest row. A level whose packs would hold more than FL_PAD groups
+// per entry and row is left to the chip-wide sweep, which reads the matrix as it lies: 7-point
+// and coarse levels reach 0.3 to 0.5; one hub of 80 entries in every 64 short rows (4.9) takes
+// 0.70 of the chip-wide time at 25,600 rows and all of it at 140,800, one of 300 (9.8) 0.76 and
+// 1.14, at 0.9 KB per entry and row (FP64, both directions).
+constexpr int FL_PAD = 8;
+constexpr unsigned long long FL_GROUPS = 1ull << 26;   // 3.2 GB in FP64, and 32-bit positions
 constexpr int FL_OWN_ROWS = 4096;   // up to here the kernel reorders x and b itself (8 rows per thread)
 constexpr int FL_NW = 8;   // wavefronts (twelve were slower: 44k rows, 620 against 510 us a sweep)
 template <class X> constexpr int fl_ring() { return sizeof(X) == 8 ? 4096 : 8192; }
@@ -2189,7 +2194,7 @@ void prepare_flow_packs(Run &R) {
         Level::FlowPack &P = L.flow[J.dir];
         const size_t kf = k - J.dir;
         const unsigned long long most = std::max(ht[2 * kf], ht[2 * kf + 2]);
-        if (most > (unsigned long long)L.nnz + L.n || most > FL_GROUPS) {
+        if (most > FL_PAD * ((unsigned long long)L.nnz + L.n) || most > FL_GROUPS) {
             P = Level::FlowPack{};
             continue;
         }

@@ -95,10 +95,11 @@ def bundle(n, hub, seed=0):
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("hub,used", [(0, True), (300, False)])
+@pytest.mark.parametrize("hub,used", [(0, True), (80, True), (300, False)])
 def test_level_with_hub_rows_is_not_padded_to_them(prec, hub, used):
-    """Items of one hub and 63 short rows: 64 rows padded to 300 entries each would be nine times the
-    entries and rows of the level (limit: once), so the chip-wide sweep keeps it. Same bits either way."""
+    """Items of one hub and 63 short rows: 64 rows padded to 300 entries each take nine groups of four
+    per entry and row of the level (limit: eight; hubs of 80: 4.6), so the chip-wide sweep keeps it.
+    Same bits either way."""
     m = bundle(2560, hub)
     res = []
     for flow in (0, 1):
