@@ -173,7 +173,8 @@ struct fvm_amg {
     int flow_wg_rows = 150000;         // levels up to this many rows may sweep in one workgroup (k_gs_flow_wg)
     fvm::DArr<int> flow_ctl;           // its block tickets, finished blocks and error flag
     bool flow_used = false;            // a dataflow sweep ran since the last check
-    long long flow_ticks = 0;          // two seconds of the device's wall clock
+    int flow_khz = 100000;             // rate of the device's wall clock
+    int flow_give_up_ms = 2000;        // a wait without progress for this long ends the sweep
     int flow_spin_limit = 0;           // waits per wavefront before a sweep gives up (0: no bound)
     long long coarsen_small_rows = 2048;
     int coarsen_lanes = 0;             // lanes per row of the agglomeration rounds (0: by row width)

@@ -559,6 +559,9 @@ int fvm_amg_set_tuning(fvm_amg *h, const char *key, long long value) {
     } else if (k == "exact_flow_spin_limit") {
         FVM_CHECK(value >= 0 && value <= INT_MAX, FVM_E_INVALID, "exact_flow_spin_limit must be in [0, INT_MAX]");
         h->flow_spin_limit = (int)value;
+    } else if (k == "exact_flow_give_up_ms") {
+        FVM_CHECK(value >= 0 && value <= 3600000, FVM_E_INVALID, "exact_flow_give_up_ms must be in [0, 3600000]");
+        h->flow_give_up_ms = (int)value;
     } else if (k == "exact_flow_wg_rows") {
         FVM_CHECK(value >= 0 && value <= INT_MAX, FVM_E_INVALID, "exact_flow_wg_rows must be in [0, INT_MAX]");
         h->flow_wg_rows = (int)value;
@@ -614,6 +617,7 @@ int fvm_amg_get_tuning(const fvm_amg *h, const char *key, long long *value) {
     else if (k == "reuse_setup") *value = h->reuse_setup;
     else if (k == "setups_reused") *value = h->setup_reused;
     else if (k == "exact_flow_spin_limit") *value = h->flow_spin_limit;
+    else if (k == "exact_flow_give_up_ms") *value = h->flow_give_up_ms;
     else if (k == "exact_flow_wg_rows") *value = h->flow_wg_rows;
     else if (k == "exact_flow_wg_levels") {
         *value = 0;

@@ -194,6 +194,8 @@ constexpr int FLOW_RC = 16;   // entries of a row kept in registers while it wai
 // with up to 32 naps, 97.7 with 8, 103.4 without; polling every new value each
 // time: 107-110 (the polls' own traffic slows the rows that are ready).
 constexpr int FLOW_NAPS = 32;
+// unsuccessful polls between two looks at the clock (a bound of 0 ends the first wait)
+__device__ __forceinline__ int flow_look(long long give_up) { return give_up > 0 ? 4096 : 1; }
 template <class V, class D, class X>
 __global__ void __launch_bounds__(FLOW_BS)
 k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restrict__ row, const int *__restrict__ col,
@@ -248,6 +250,7 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
                 }
         }
     }
+    const int look = flow_look(give_up);
     int spins = 0, seen = -1, nap = 0, waits = 0;
     long long t_seen = 0;
     while (__ballot(todo)) {
@@ -291,7 +294,7 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
                 break;
             }
             for (int z = 0; z < nap; z++) __builtin_amdgcn_s_sleep(2);
-            if (++spins == 4096) {   // every few milliseconds: has any block finished since?
+            if (++spins == look) {   // every few milliseconds: has any block finished since?
                 spins = 0;
                 // one lane's view decides for the whole wavefront
                 const int pr = __builtin_amdgcn_readfirstlane(
@@ -300,10 +303,10 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
                     __hip_atomic_load(&ctl[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
                 const long long now = (long long)wall_clock64();
                 if (ab) break;   // another wavefront gave up
-                if (pr != seen) {
+                if (give_up > 0 && pr != seen) {
                     seen = pr;
                     t_seen = now;
-                } else if (now - t_seen > give_up) {
+                } else if (give_up == 0 || now - t_seen > give_up) {
                     if (__lane_id() == 0) atomicOr(&ctl[2], 1);
                     break;
                 }
@@ -322,7 +325,8 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // taken by the wavefronts in turn; a wavefront loads its item's rows, entries and old
 // values while the items before it are still running, then waits (an LDS counter of
 // finished items) until every item of the earlier dependency levels is done. Item i waits
-// only for items below it, so every wait ends. New values lie in an LDS ring, by their
+// only for items below it, so every wait ends (and one that sees no item finish for two seconds
+// is given up all the same, as in k_csr_gs_flow). New values lie in an LDS ring, by their
 // place in the schedule; a value that the ring has overwritten is read back from memory,
 // where it was stored many items ago by a wavefront of the same CU, whose vector memory
 // operations pass its L1 in order.
@@ -434,13 +438,15 @@ __global__ void k_flow_out(int n, const int *__restrict__ rows, const X *__restr
 template <class X, int NW, int Q>
 __global__ void __launch_bounds__(64 * NW)
 k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const int *__restrict__ rows, X *x_io,
-             const X *b_in, const uint8_t *__restrict__ mask, int *ctl, int spin_limit) {
+             const X *b_in, const uint8_t *__restrict__ mask, int *ctl, long long give_up, int spin_limit) {
     constexpr int R = fl_ring<X>(), FL_SCR = NW * Q * 4 * 64;
     extern __shared__ __align__(16) unsigned char s_fl[];
     X *sm = (X *)s_fl;            // [0, FL_SCR): old values; then the ring and its zero word
     int *done = (int *)(sm + FL_SCR + R + 1), *stop = done + 1;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int look = spin_limit > 0 ? min(flow_look(give_up), spin_limit) : flow_look(give_up);
     int waits = 0;
+    bool stopped = false;   // a wait was given up: the rest is not waited for
     if (x_io)   // a small level: x and b brought into schedule order here, without launches of their own
         for (int k = threadIdx.x; k < n; k += 64 * NW) {
             const int i = rows[k];
@@ -496,20 +502,30 @@ k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const in
             }
             const bool anyfar = __any(far);
             // every item of the earlier dependency levels done?
-            while (__builtin_amdgcn_readfirstlane(
-                       __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < need) {
-                if (spin_limit > 0) {   // a caller's bound on the waits (0: none)
-                    if (++waits >= spin_limit) {
-                        if (lane == 0) {
-                            atomicOr(&ctl[2], 1);
-                            __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        }
-                        break;
-                    }
-                    if (__builtin_amdgcn_readfirstlane(
-                            __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)))
-                        break;
+            auto finished = [&]() {
+                return __builtin_amdgcn_readfirstlane(
+                    __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+            };
+            int seen = -1;
+            long long t_seen = 0;
+            for (int d = finished(), left = look; d < need && !stopped; d = finished()) {
+                if (--left > 0) continue;
+                left = look;   // a look at the bounds: has any item finished since the last one?
+                const long long now = (long long)wall_clock64();
+                waits += look;
+                bool late = give_up == 0 || (spin_limit > 0 && waits >= spin_limit);
+                if (d != seen) {
+                    seen = d;
+                    t_seen = now;
+                } else {
+                    late = late || now - t_seen > give_up;
                 }
+                if (late && lane == 0) {
+                    atomicOr(&ctl[2], 1);
+                    __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+                stopped = late || __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                                      stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             if (anyfar) {
@@ -1620,6 +1636,9 @@ void residual(Run &R, int l, const X *x, const X *b, X *r) {
     if (t0) timing_end(R.h, KT_RESID64, t0, pass_bytes(V64, sizeof(X), 3, n, L.nnz));   // x, b read; r written
 }
 
+// bound on a wait without progress, in ticks of the device's wall clock
+long long flow_ticks(const fvm_amg *h) { return (long long)h->flow_give_up_ms * h->flow_khz; }
+
 template <class X>
 void gs_sweep(Run &R, int l, X *x, const X *b) {
     Level &L = R.h->lev[l];
@@ -1664,7 +1683,8 @@ void gs_sweep(Run &R, int l, X *x, const X *b) {
         if (!own) k_flow_in<X><<<grid_for(n, BS), BS, 0, s>>>(n, L.fwd_rows.p, x, b, xp, bp);
         auto launch = [&](auto kern, int nw, size_t lds) {
             kern<<<1, 64 * nw, lds, s>>>(n, dirp(L.flow[0]), dirp(L.flow[1]), xp, xq, bp, L.fwd_rows.p,
-                                         own ? x : nullptr, b, l == 0 ? R.mask0 : nullptr, h->flow_ctl.p, h->flow_spin_limit);
+                                         own ? x : nullptr, b, l == 0 ? R.mask0 : nullptr, h->flow_ctl.p, flow_ticks(h),
+                                         h->flow_spin_limit);
         };
         if (L.flow_groups <= 2) launch(k_gs_flow_wg<X, FL_NW, 2>, FL_NW, fl_lds<X, FL_NW, 2>());
         else if (L.flow_groups <= 4) launch(k_gs_flow_wg<X, FL_NW, 4>, FL_NW, fl_lds<X, FL_NW, 4>());
@@ -1684,7 +1704,7 @@ void gs_sweep(Run &R, int l, X *x, const X *b) {
             FVM_DISPATCH_VALS(R, l, L, X, (void)0,
                 (k_csr_gs_flow<<<(unsigned)((n + FLOW_BS - 1) / FLOW_BS), FLOW_BS, 0, s>>>(
                     n, dir, rows, L.row.p, L.col.p, val, dg, xa.p, ta.p, b, l == 0 ? R.mask0 : nullptr,
-                    h->flow_ctl.p, h->flow_ticks, h->flow_spin_limit)));
+                    h->flow_ctl.p, flow_ticks(h), h->flow_spin_limit)));
             std::swap(xa, ta);   // the new values become x (two swaps per sweep: the arrays end where they began)
         }
     } else {
@@ -2227,7 +2247,7 @@ Run make_run(fvm_amg *h) {
         FVM_HIP(hipMemsetAsync(h->flow_ctl.p, 0, h->flow_ctl.bytes(), h->stream));
         int khz = 0;
         FVM_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device));
-        h->flow_ticks = 2000LL * (khz > 0 ? khz : 100000);
+        h->flow_khz = khz > 0 ? khz : 100000;
     }
     if (R.mixed) {
         prepare_mixed(h, R.fast);

@@ -514,23 +514,26 @@ def test_opt_in_setup_reuse_gives_the_rebuilt_results():
     assert ga.get_tuning("setups_reused") == 2 and ga.num_levels() == 4
 
 
+@pytest.mark.parametrize("key,bound,unbound", [("exact_flow_spin_limit", 1, 0), ("exact_flow_give_up_ms", 0, 2000)])
 @pytest.mark.parametrize("wg_rows", [150000, 0])
-def test_dataflow_sweep_bounded_wait_fails_loudly_then_recovers(wg_rows):
+def test_dataflow_sweep_bounded_wait_fails_loudly_then_recovers(wg_rows, key, bound, unbound):
     """A reference-order dataflow sweep (in one workgroup, and over the chip:
     exact_flow_wg_rows 0) whose wavefronts may wait only once
-    (exact_flow_spin_limit 1) gives up through its own bounded wait: the call
+    (exact_flow_spin_limit 1) or for no time (exact_flow_give_up_ms 0: by the
+    clock, as after two seconds) gives up through its own bounded wait: the call
     fails with the sweep's error, every kernel exits normally, and the next call
     without the bound gives the oracle's bits again."""
     from fvm_amd._lib import FVM_E_NUMERIC, FvmError
     m = matgen.grid3d(10, seed=30)
     ga = gpu_amg(gsOrdering=0, nMaxIterations=5, relativeTolerance=1e-30)
     ga.set_tuning("exact_flow_wg_rows", wg_rows)
-    ga.set_tuning("exact_flow_spin_limit", 1)
+    assert ga.get_tuning(key) == unbound
+    ga.set_tuning(key, bound)
     for call in ("smooth", "solve"):
         with pytest.raises(FvmError, match="stopped waiting") as e:
             getattr(ga, call)(ls_from(m))
         assert e.value.code == FVM_E_NUMERIC
-    ga.set_tuning("exact_flow_spin_limit", 0)
+    ga.set_tuning(key, unbound)
     ls = ls_from(m)
     ga.solve(ls)
     want = oracle_for(m, n_max_iterations=5, relative_tolerance=1e-30).solve(m["b"])
