@@ -175,7 +175,7 @@ struct fvm_amg {
     bool flow_used = false;            // a dataflow sweep ran since the last check
     int flow_khz = 100000;             // rate of the device's wall clock
     int flow_give_up_ms = 2000;        // a wait without progress for this long ends the sweep
-    int flow_spin_limit = 0;           // waits per wavefront before a sweep gives up (0: no bound)
+    int flow_spin_limit = 0;           // polls of a waiting wavefront before a sweep gives up (0: no bound)
     long long coarsen_small_rows = 2048;
     int coarsen_lanes = 0;             // lanes per row of the agglomeration rounds (0: by row width)
     int coarsen_small_lanes = 16;      // the same for the single-workgroup rounds (0: as coarsen_lanes)

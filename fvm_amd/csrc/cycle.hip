@@ -445,7 +445,6 @@ k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const in
     int *done = (int *)(sm + FL_SCR + R + 1), *stop = done + 1;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int look = spin_limit > 0 ? min(flow_look(give_up), spin_limit) : flow_look(give_up);
-    int waits = 0;
     bool stopped = false;   // a wait was given up: the rest is not waited for
     if (x_io)   // a small level: x and b brought into schedule order here, without launches of their own
         for (int k = threadIdx.x; k < n; k += 64 * NW) {
@@ -506,7 +505,7 @@ k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const in
                 return __builtin_amdgcn_readfirstlane(
                     __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
             };
-            int seen = -1;
+            int seen = -1, waits = 0;
             long long t_seen = 0;
             for (int d = finished(), left = look; d < need && !stopped; d = finished()) {
                 if (--left > 0) continue;

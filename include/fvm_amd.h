@@ -236,8 +236,8 @@ int fvm_amg_kernel_bytes(const fvm_amg *h, int kind, double *total_bytes);
  * every setup rebuilds, as the reference does after cleanup); "setups_reused"
  * (read only) counts them; "exact_flow" -- reference-order sweeps as
  * one dataflow launch per direction (default 1; 0: level by level);
- * "exact_flow_spin_limit" -- waits per wavefront after which such a sweep gives
- * up and the call fails with FVM_E_NUMERIC (default 0: no bound);
+ * "exact_flow_spin_limit" -- polls of a wavefront that waits for its rows (up to
+ * 64) after which such a sweep gives up and the call fails with FVM_E_NUMERIC (default 0: no bound);
  * "exact_flow_give_up_ms" -- the same for a wait during which nothing was updated
  * for this long (default 2000; 0: the first wait gives up);
  * "exact_flow_wg_rows" -- such sweeps of levels of at most this many rows run

@@ -540,6 +540,21 @@ def test_dataflow_sweep_bounded_wait_fails_loudly_then_recovers(wg_rows, key, bo
     assert np.array_equal(ls.delta, want["x"])
 
 
+def test_bound_on_a_wait_is_not_a_bound_on_a_sweep():
+    """4,000 dependency levels of one row each, taken in turn by the wavefronts of one workgroup: each wait
+    is short (about fifty polls), so a bound of 2,000 polls lets the sweep pass, however many waits it has."""
+    m = matgen.chain(4000, d=-2.1)
+    out = []
+    for limit in (0, 2000):
+        ga = gpu_amg(gsOrdering=0, nMaxIterations=4, relativeTolerance=1e-30)
+        ga.set_tuning("exact_flow_spin_limit", limit)
+        ls = ls_from(m)
+        ga.solve(ls)
+        assert ga.get_tuning("exact_flow_wg_levels") & 1
+        out.append(ls.delta.copy())
+    assert np.array_equal(out[0], out[1])
+
+
 def _continuity():
     return O.load_mm(os.path.join(G, "cav32_continuity_matrix.mat"), os.path.join(G, "cav32_continuity_matrix.rhs"))
 
