@@ -144,6 +144,7 @@ struct fvm_amg {
     fvm::Workspace ws;
     fvm::Workspace ws2;          // of stream2
     bool ready = false;
+    unsigned long long hierarchy_id = 0;   // of the hierarchy in place: no two in the process share one
     int n_self = 0, n_total = 0;
     long long total_iterations = 0;
     std::vector<double> hist;
@@ -281,7 +282,9 @@ void kinetic_assemble_into(fvm_mesh *m, const double *c, const double *d_nue, co
                            double *F, uint8_t *inc);
 void system_post_solve_async(const fvm_system *S, double *d_delta, hipStream_t s);
 // learned correction (mpnn.hip)
-void mpnn_bind(fvm_mpnn *m, int n, const int *row, const int *col, const double *off, const double *diag);
+// makes the finest level of a hierarchy the network's graph, unless it is that already
+void mpnn_bind(fvm_mpnn *m, unsigned long long hierarchy_id, int n, const int *row, const int *col, const double *off,
+               const double *diag);
 void mpnn_correct(fvm_mpnn *m, hipStream_t st, const int *perm, const double *Az, const double *v, double *z,
                   int n, int *bad_out);
 struct LearnedHook {

@@ -3170,7 +3170,7 @@ void fgmres_solve(fvm_amg *h, KrylovWork &W, const fvm_fgmres_params &p, const d
     int total = 0;
     // learned correction of the preconditioner: on until the residual stalls
     bool nn_on = nn.m != nullptr && n > 0;
-    if (nn_on) mpnn_bind(nn.m, F.n, F.row.p, F.col.p, F.off.p, F.diag.p);
+    if (nn_on) mpnn_bind(nn.m, h->hierarchy_id, F.n, F.row.p, F.col.p, F.off.p, F.diag.p);
     if (nn.used) *nn.used = 0;
     if (nn.fallback_at) *nn.fallback_at = -1;
     std::vector<double> est_hist;

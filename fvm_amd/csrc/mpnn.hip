@@ -711,6 +711,7 @@ struct fvm_mpnn {
     int n = 0;
     const int *row = nullptr, *col = nullptr;
     const double *off = nullptr, *diag = nullptr;
+    unsigned long long bound = 0;   // hierarchy whose finest level it is (0: set by fvm_mpnn_set_graph)
     DArr<float> c, ct, l;
     // activations and work
     // layer inputs and aggregates; those of layer 0 hold its four packed features per node
@@ -841,10 +842,13 @@ void mpnn_correct(fvm_mpnn *m, hipStream_t st, const int *perm, const double *Az
     if (bad_out) *bad_out = read_scalar(m->flag.p, st);
 }
 
-void mpnn_bind(fvm_mpnn *m, int n, const int *row, const int *col, const double *off, const double *diag) {
-    if (m->n == n && m->row == row && m->col == col && m->off == off && m->diag == diag) return;
+// (the arrays' addresses do not tell: the next setup of a handle may get the same ones)
+void mpnn_bind(fvm_mpnn *m, unsigned long long hierarchy_id, int n, const int *row, const int *col, const double *off,
+               const double *diag) {
+    if (m->bound == hierarchy_id) return;
     const int rc = fvm_mpnn_set_graph(m, n, row, col, off, diag);
     if (rc) throw Error(rc, std::string("learned correction: ") + fvm_last_error());
+    m->bound = hierarchy_id;
 }
 
 }  // namespace fvm
@@ -958,6 +962,7 @@ int fvm_mpnn_set_graph(fvm_mpnn *m, int n, const int32_t *d_row, const int32_t *
     hipStream_t st = m->stream;
     const long long nnz = n > 0 ? fvm::read_scalar(d_row + n, st) : 0;
     FVM_CHECK(nnz == 0 || (d_col && d_off), FVM_E_INVALID, "null col/off arrays");
+    m->bound = 0;
     m->n = n; m->row = d_row; m->col = d_col; m->off = d_off; m->diag = d_diag;
     m->c.alloc(std::max<long long>(nnz, 1));
     m->ct.alloc(std::max<long long>(nnz, 1));

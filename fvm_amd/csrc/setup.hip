@@ -14,6 +14,7 @@
 #include "amg.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <condition_variable>
 #include <deque>
@@ -1747,6 +1748,11 @@ k_invert(int n, const int *row, const int *col, const double *diag, const double
     }
 }
 
+unsigned long long new_hierarchy_id() {
+    static std::atomic<unsigned long long> last{0};
+    return ++last;
+}
+
 double now_s() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
@@ -2159,6 +2165,7 @@ void build_hierarchy(fvm_amg *h, int n_self, int n_total, const int *d_row, cons
     h->parked = false;
     h->lev.clear();
     h->ready = false;
+    h->hierarchy_id = new_hierarchy_id();
     h->batch = nullptr;
     h->direct_level = -1;
     h->direct_tried = false;
@@ -2721,6 +2728,7 @@ void build_hierarchy_batched(fvm_amg *h, BatchInfo &B) {
     FVM_CHECK(h->prm.coarseGroupSize == 2, FVM_E_INVALID, "the GPU agglomeration supports coarseGroupSize == 2 only");
     h->lev.clear();
     h->ready = false;
+    h->hierarchy_id = new_hierarchy_id();
     h->batch = nullptr;
     h->direct_level = -1;
     h->direct_tried = false;

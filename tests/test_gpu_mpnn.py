@@ -251,6 +251,46 @@ def test_fgmres_with_learned_correction(prec):
     assert np.abs(x1.cpu().numpy() - ref).max() <= 1e-8 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("how", ["one handle", "a handle each", "graph set by hand"])
+def test_learned_correction_follows_the_hierarchy(how):
+    """One network in solves with two matrices of the same pattern in turn, set up in one handle or in a new
+    one each (whose arrays lie where those of the handle before lay): the correction takes the present
+    matrix's weights, so every solve has the bits that a fresh network gives."""
+    import gc
+    import torch
+    import fvm_amd
+    from fvm_amd import LearnedCorrection
+    ms = [matgen.grid3d(14, seed=s, ghosts=False, contrast=2.0) for s in (3, 8)]
+    gs = [_graph(m) for m in ms]
+    bs = [_dev(m["b"], torch.float64) for m in ms]
+
+    def solves(net, which, each):
+        amg, out = None, []
+        for k in which:
+            if amg is None or each:
+                amg = fg = None
+                gc.collect()
+                amg = fvm_amd.AMG()
+                amg.verbosity = 0
+                amg.gsOrdering = 1
+            g = gs[k]
+            amg.setup_device(ms[k]["n_self"], ms[k]["n_total"], g[1], g[2], g[4], g[3])
+            if how == "graph set by hand":
+                net.set_graph(*gs[1 - k])   # the solve takes its own
+            x = torch.zeros(ms[k]["n_self"], dtype=torch.float64, device="cuda:0")
+            fg = _fgmres(amg, net)
+            fg.nMaxIterations = 6
+            fg.solve_device(bs[k], x)
+            assert fg.learned_stats()["iterations_used"] > 0
+            out.append(x.cpu().numpy())
+        return out
+
+    want = [solves(LearnedCorrection(seed=2), (k,), False)[0] for k in (0, 1)]
+    seq = (0, 1, 0, 1, 0)
+    for k, x in zip(seq, solves(LearnedCorrection(seed=2), seq, how == "a handle each")):
+        assert np.array_equal(x, want[k])
+
+
 def test_bad_network_falls_back():
     import torch
     import fvm_amd
