@@ -746,7 +746,7 @@ def main():
                     help="no GPU: write profiles/hbm_traffic.json from the two counter passes of --profile")
     ap.add_argument("--sell-block", type=int, default=256, help="--profile: smoother threads per block")
     ap.add_argument("--spmv-block", type=int, default=256, help="--profile: residual/SpMV threads per block")
-    ap.add_argument("--tail-max-rows", type=int, default=40000, help="--profile: single-workgroup tail size")
+    ap.add_argument("--tail-max-rows", type=int, default=6000, help="--profile: single-workgroup tail size")
     ap.add_argument("--sell-xcd", type=int, default=1, help="--profile: XCD-contiguous smoother blocks")
     ap.add_argument("--spmv-xcd", type=int, default=0, help="--profile: XCD-contiguous residual/SpMV blocks")
     ap.add_argument("--cycle-graph", type=int, default=1, help="--profile: replay levels >= 1 of the cycle from a graph")

@@ -2438,7 +2438,8 @@ std::string autotune(fvm_amg *h, int reps) {
     h->ktime = false;
     std::vector<int> blocks = {128, 256, 512};
     const int keep_sx = h->sell_xcd, keep_px = h->spmv_xcd, keep_cg = h->cycle_graph;
-    std::vector<long long> tails = {0, 1000, 2500, 10000, 40000};
+    // the default among them; past TAIL_ROWS_CAP no level can be packed (40,000: 3.0 against 1.8 ms a cycle)
+    std::vector<long long> tails = {0, 1000, 2500, 6000, 10000};
     hipEvent_t e0, e1;
     FVM_HIP(hipEventCreate(&e0));
     FVM_HIP(hipEventCreate(&e1));

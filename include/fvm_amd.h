@@ -262,7 +262,7 @@ int fvm_amg_get_tuning(const fvm_amg *h, const char *key, long long *value);
 /* Autotuner (no counterpart in the reference): times every candidate launch
  * shape that cannot change a result -- "sell_block" (threads per block of the
  * coloured SELL-64 smoother kernels: 128/256/512) x "tail_max_rows"
- * (0/1000/2500/1e4/4e4) x "sell_xcd" (0/1) x "cycle_graph" (0/1) -- with one warm-up and `reps` timed
+ * (0/1000/2500/6000/10000) x "sell_xcd" (0/1) x "cycle_graph" (0/1) -- with one warm-up and `reps` timed
  * cycles each on the handle's current hierarchy and parameters, keeps the
  * fastest, then "nt_levels" (0..3) with those shapes, then times the
  * finest-level residual alone for "spmv_block"

@@ -369,7 +369,10 @@ def test_autotune_keeps_results(prec):
     ga = gpu_amg(gsOrdering=1, precision=prec, nMaxIterations=15, relativeTolerance=1e-30)
     ls1 = ls_from(m)
     ga.setup(ls1)
+    default = {k: ga.get_tuning(k) for k in ("sell_block", "tail_max_rows", "sell_xcd", "cycle_graph")}
     rep = ga.autotune(reps=2)
+    # the shapes in place are among those timed: a tuned handle is not slower for want of them
+    assert any(all(c[k] == v for k, v in default.items()) for c in rep["candidates"])
     assert len(rep["candidates"]) == 60 and len(rep["spmv_candidates"]) == 6
     ch = rep["chosen"]
     assert any(c["sell_block"] == ch["sell_block"] and c["tail_max_rows"] == ch["tail_max_rows"]
