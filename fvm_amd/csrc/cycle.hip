@@ -327,9 +327,9 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // finished items) until every item of the earlier dependency levels is done. Item i waits
 // only for items below it, so every wait ends (and one that sees no item finish for two seconds
 // is given up all the same, as in k_csr_gs_flow). New values lie in an LDS ring, by their
-// place in the schedule; a value that the ring has overwritten is read back from memory,
-// where it was stored many items ago by a wavefront of the same CU, whose vector memory
-// operations pass its L1 in order.
+// place in the schedule; a value that the ring has overwritten is read back from memory.
+// The counter orders both: an item's values are stored before its count (release), and read
+// after the wait (acquire), at workgroup scope, whose wavefronts share the CU's L1.
 // The price is one CU's throughput (about 20 GB/s of what its L2 does not hold), so b and
 // x are first brought into the order of the schedule: rows of one dependency level side
 // by side, sorted, their neighbours nearly so (44k rows: 510 -> 320 us a sweep). An item
@@ -526,7 +526,7 @@ k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const in
                 stopped = late || __builtin_amdgcn_readfirstlane(__hip_atomic_load(
                                       stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             if (anyfar) {
 #pragma unroll
                 for (int u = 0; u < 4 * Q; u++)
@@ -567,8 +567,7 @@ k_gs_flow_wg(int n, FlowDir<X> fwd, FlowDir<X> bwd, X *xa, X *xb, X *b, const in
                 sm[FL_SCR + (pos & (R - 1))] = x;
                 __hip_atomic_store(xn + i, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-            // LDS operations of a wavefront are performed in order: the values before the count
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             if (lane == 0) __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         __syncthreads();

@@ -112,6 +112,75 @@ def test_level_with_hub_rows_is_not_padded_to_them(prec, hub, used):
     assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
 
 
+def layered(n, dists, hub=0, seed=0):
+    """Bundles of 64 rows as in ``bundle``; row i is linked to i - d and i + d for every distance d (64 among
+    them, so that a bundle is a dependency level), one row in 64 reads ``hub`` earlier and as many later rows
+    besides; columns in any order."""
+    rng = np.random.default_rng(seed)
+    col, row = [], [0]
+    for i in range(n):
+        c = {j for d in dists for j in (i - d, i + d) if 0 <= j < n}
+        if hub and i % 64 == 7 and i > 64:
+            c |= {int(j) for j in rng.integers(0, i - i % 64, hub)}
+            c |= {int(j) for j in rng.integers(min(i - i % 64 + 64, n - 1), n, hub) if j > i}
+        col += list(rng.permutation(sorted(c)))
+        row.append(len(col))
+    row = np.array(row, np.int32)
+    off = rng.uniform(0.1, 1.0, len(col))
+    diag = -1.1 * np.add.reduceat(off, row[:-1]) - 0.1
+    return dict(n_self=n, n_total=n, row=row, col=np.array(col, np.int32), diag=diag, off=off,
+                b=rng.uniform(-1, 1, n))
+
+
+def ring_distances(m, back):
+    """For every entry that reads a value updated in the same sweep: the rows of the schedule between that
+    value and the end of the reader's dependency level, and the entry's place in its row."""
+    n, row, col = m["n_self"], m["row"], m["col"]
+    level = np.zeros(n, int)
+    for i in range(n):   # (the backward sweep takes the forward schedule from its end)
+        c = col[row[i]:row[i + 1]]
+        level[i] = level[c[c < i]].max(initial=-1) + 1
+    order = np.lexsort((np.arange(n), level))
+    place = np.empty(n, int)
+    place[order] = np.arange(n)
+    if back:
+        place, level = n - 1 - place, level.max() - level
+    end = np.cumsum(np.bincount(level))
+    i = np.repeat(np.arange(n), np.diff(row))
+    new = col > i if back else col < i
+    return (end[level[i]] - place[col])[new], (np.arange(len(col)) - row[i])[new]
+
+
+NEAR = tuple(range(64, 640, 64))
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("dists,hub,longest", [((64, 4064, 8160), 0, 8), ((64, 128, 4064, 8160, 9600), 0, 8),
+                                               (NEAR[:5] + (4064, 8160, 9600, 9664), 0, 16),
+                                               (NEAR + (4064, 8160), 0, 24), ((64, 4064, 8160), 30, 70)])
+def test_values_that_left_the_ring(dists, hub, longest, prec):
+    """The ring in LDS holds the last 4,096 new values in FP64, 8,192 in FP32: links that reach just inside
+    it, just past it and far past it, in rows of each shape of the kernel (8, 16 and 24 entries loaded
+    ahead, and entries past those). Against the level-by-level launches: same bits."""
+    m = layered(12800, dists, hub)
+    ring = 8192 if prec else 4096
+    assert longest - 8 < np.diff(m["row"]).max() <= longest
+    for back in (False, True):
+        dist, k = ring_distances(m, back)
+        assert (dist > ring).sum() > 1000 and (dist <= ring).sum() > 1000
+        assert {ring, ring + 1} <= set(dist)
+        assert not hub or ((dist > ring) & (k >= 24)).sum() > 100
+    res = []
+    for flow in (0, 1):
+        a = gpu_amg(gsOrdering=0, precision=prec, nMaxIterations=5, relativeTolerance=1e-30)
+        a.set_tuning("exact_flow", flow)
+        ls = ls_from(m)
+        a.solve(ls)
+        res.append((ls.delta.copy(), a.history()))
+        assert a.get_tuning("exact_flow_wg_levels") & 1 == flow
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+
+
 @pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 127, 255, 256])
 def test_direct_level_inverse_at_panel_edges(n):
     """The blocked inverse of the direct level, at the edges of its panels and at its limit."""
