@@ -204,6 +204,7 @@ struct fvm_amg {
     // single-workgroup tail of the V-cycle: levels >= tail_level run in one launch
     int tail_level = -1;
     int tail_prec = -1;                // precision the descriptors were built for
+    int tail_form = 0;                 // kernel of the last cycle's tail: 0 none, 1 k_tail, 2 k_tail_gs
     int tail_lds = 1;                  // tail levels that fit sweep from LDS
     int tail_lds_lim = -1;             // LDS bytes per workgroup of the device (-1: not queried)
     std::vector<int> tail_lds_bytes[2];   // LDS bytes per level (FP64 / mixed descriptors)
@@ -231,6 +232,7 @@ struct fvm_amg {
 
 namespace fvm {
 inline void invalidate_cycle_graphs(fvm_amg *h) {
+    h->tail_form = 0;
     for (auto &g : h->cg_exec)
         if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
 }

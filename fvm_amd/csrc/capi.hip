@@ -610,6 +610,9 @@ int fvm_amg_get_tuning(const fvm_amg *h, const char *key, long long *value) {
     else if (k == "coarsen_wait_lists") *value = h->coarsen_wait_lists;
     else if (k == "coarsen_block") *value = h->coarsen_block;
     else if (k == "tail_lds") *value = h->tail_lds;
+    else if (k == "tail_form") *value = h->tail_form;
+    else if (k == "tail_level") *value = h->tail_form ? h->tail_level : -1;
+    else if (k == "tail_resident_level") *value = h->tail_form == 2 ? h->tail_lr : -1;
     else if (k == "gal_lanes") *value = h->gal_lanes;
     else if (k == "colour_grid") *value = h->colour_grid;
     else if (k == "coarsen_batch") *value = h->coarsen_batch;

@@ -2045,6 +2045,7 @@ void cycle(Run &R, int type, int l, bool x_zero) {
                 };
                 if (R.mixed) launch(k_tail_gs<uint16_t, float, float>);
                 else launch(k_tail_gs<double, double, double>);
+                h->tail_form = 2;
                 FVM_HIP(hipGetLastError());
                 return;
             }
@@ -2062,6 +2063,7 @@ void cycle(Run &R, int type, int l, bool x_zero) {
         };
         if (R.mixed) launch(k_tail<uint16_t, float, float>);
         else launch(k_tail<double, double, double>);
+        h->tail_form = 1;
         FVM_HIP(hipGetLastError());
         return;
     }

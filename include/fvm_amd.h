@@ -197,7 +197,11 @@ int fvm_amg_kernel_bytes(const fvm_amg *h, int kind, double *total_bytes);
  * by the autotuner): "tail_max_rows" -- V-cycle levels with at most this many
  * rows run in one single-workgroup launch (default 6000; 0 disables);
  * "tail_lds" -- 1 (default): there, levels are packed in the order of the sweeps
- * and those that fit stay in the workgroup's LDS; "sell_block" -- threads
+ * and those that fit stay in the workgroup's LDS; "tail_form" (read only) -- 2
+ * if the last cycle's tail ran in that packed form, 1 in the general one (Jacobi,
+ * pre-sweeps, levels too large to pack), 0 without a tail, "tail_level" and
+ * "tail_resident_level" its first level and the first one that stays in LDS
+ * (-1: none); "sell_block" -- threads
  * per block of the SELL-64 smoother kernels, "spmv_block" -- of the SELL-64
  * residual and SpMV kernels (64/128/256/512 each); "sell_xcd" / "spmv_xcd" --
  * 1: blocks of those kernels are renumbered so that each of the chip's 8 XCDs

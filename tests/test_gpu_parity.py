@@ -350,6 +350,8 @@ def test_tail_kernel_is_bit_identical(prec, smoother, npre):
         ls = ls_from(m)
         ga.solve(ls)
         res.append((ls.delta.copy(), ga.history()))
+        # packed where it can be: Gauss-Seidel without pre-sweeps
+        assert ga.get_tuning("tail_form") == (0 if tail == 0 else 1 if smoother or npre or not lds else 2)
         # a second solve on the same handle replays the captured graph
         ls = ls_from(m)
         ga.solve(ls)

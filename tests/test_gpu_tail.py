@@ -43,6 +43,12 @@ def test_packed_tail_is_bit_identical(case, prec, npost):
         ls = ls_from(m)
         a.solve(ls)
         res.append((ls.delta.copy(), a.history()))
+        # the packed form ran, from the first level that fits the limit, with levels streamed and resident
+        form, first, resident = (a.get_tuning("tail_" + k) for k in ("form", "level", "resident_level"))
+        n = [a.level(l)["n"] for l in range(a.num_levels())]
+        assert form == (2 if tail else 0)
+        assert first == (next(l for l in range(1, len(n)) if n[l] <= tail) if tail else -1)
+        assert not tail or (resident > first if n[first] > 1000 else resident >= first)
     for d, h in res[1:]:
         assert np.array_equal(res[0][0], d) and np.array_equal(res[0][1], h)
 
