@@ -129,9 +129,10 @@ def _ring(n, rng):
     return dict(n_self=n, row=row, col=c[o].astype(np.int32), off=v[o], diag=diag)
 
 
-def _rounded(theta, G, r, et):
+def _rounded(theta, G, r, et, without=()):
     """The restatement with the activations rounded to bf16 where the kernels round them; FP64 otherwise.
-    et None: the residual loss. Returns (e, loss, gradient, amplification of an error of e into the loss)."""
+    et None: the residual loss; without: nodes left out of the gradient's sums (a planted mistake). Returns
+    (e, loss, gradient, amplification of an error of e into the loss)."""
     P = M.unpack(theta)
     u = -r / G.diag
     s = np.sqrt(np.mean(u * u)) + 1e-300
@@ -155,24 +156,60 @@ def _rounded(theta, G, r, et):
         Mt = -G.matvec(t)
         ge, loss, amp = 2.0 * Mt / den, t @ Mt / den, np.linalg.norm(e) / np.linalg.norm(t)
     dy = s * ge
-    D = {"wo": h.T @ dy, "bo": np.array([dy.sum()])}
+    summed = np.ones(G.n)
+    summed[list(without)] = 0
+    D = {"wo": h.T @ (dy * summed), "bo": np.array([(dy * summed).sum()])}
     dh = np.outer(dy, P["wo"])
     for k in reversed(range(M.LAYERS)):
         h, a, hn = cache[k]
         delta = dh * (hn > 0)
-        D["Ws%d" % k], D["Wn%d" % k], D["b%d" % k] = delta.T @ h, delta.T @ a, delta.sum(0)
+        ds = delta * summed[:, None]
+        D["Ws%d" % k], D["Wn%d" % k], D["b%d" % k] = ds.T @ h, ds.T @ a, ds.sum(0)
         if k > 0:
             dh = delta @ P["Ws%d" % k] + G.agg_t(delta @ P["Wn%d" % k])
     return e, loss, M.pack(D), max(1.0, amp)
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 65, 127, 129, 511, 513, 32769, 98321])
+def _edge_nodes(n):
+    """Sets of nodes at the edges of the kernels' loops: the remainder (last node, last tile of 16), both sides
+    of a run of the weight gradients (128 nodes, n / 256 from 32,768 on, in steps of 4) and of an eighth of
+    the tiles, and the last tile of an eighth with one tile more than a step of the widest grid (192 x 4)."""
+    tiles, runs, steps = (n + 15) // 16, min((n + 127) // 128, 256), (n + 3) // 4
+    eighth = [tiles * x // 8 for x in range(9)]
+    sets = {"last": [n - 1], "last tile": range(16 * (tiles - 1), n)}
+    if runs > 1:
+        s = 4 * (steps * (runs // 2) // runs)
+        sets["run"] = range(s - 2, s + 2)
+    if tiles >= 8:
+        sets["eighth"] = range(16 * eighth[3] - 2, 16 * eighth[3] + 2)
+    second = [x for x in range(8) if eighth[x + 1] - eighth[x] > 768]
+    if second:
+        sets["second step"] = range(16 * (eighth[second[0] + 1] - 1), 16 * eighth[second[0] + 1])
+    return {k: np.array([i for i in v if i < n]) for k, v in sets.items()}
+
+
+def _worst_block(g, ref):
+    """Largest relative error of a parameter array's gradient."""
+    G, R = M.unpack(g), M.unpack(ref)
+    return max(np.linalg.norm(G[k] - R[k]) / max(np.linalg.norm(R[k]), 1e-300) for k in R)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 65, 127, 129, 511, 513, 4099, 32769, 98321])
 def test_tile_edges(n):
     """Sizes at the edges of a tile (16 nodes), a block (64), a run of the weight gradients (128; 256 runs
     from 32,768 nodes on) and of one step of the widest grid (98,304), against the restatement with the
-    kernels' roundings. What is left are FP32 sums of at most 128 terms (1e-5) and the activations that
-    these move over a rounding boundary: fewer than 1 % of them, by one bf16 step (2^-8) each, so less
-    than 2^-8 of a norm even if all lay in one direction; the losses magnify an error of e by amp."""
+    kernels' roundings.
+
+    The output, node by node: FP32 sums differ by 1e-6 of the output's rms, unless an activation that a node
+    depends on lies so close to a rounding boundary (2^-8 apart) that these sums move it over; that is one
+    activation in some 10^4, so up to 2 % of the nodes may differ by more than 1e-4, by single flips: no node
+    by more than 2^-5 (seen: 0.5 %, 1.3e-2; a node that is left out or taken twice: about 1).
+
+    The gradient, array by array, with inputs whose gradient comes from the nodes of one edge (and their
+    neighbours) almost alone, for the residual loss (r large there) and the energy loss (e* far off there):
+    FP32 sums of at most 388 nodes and their total in FP64, 1e-5, and flips of single activations of those
+    few nodes, at most 2^-7 together (seen: 4e-4, with other seeds 1.3e-3). The restatement with those nodes
+    left out of the sums is at least eight times that far off. The losses magnify an error of e by amp."""
     import torch
     from fvm_amd import LearnedCorrection
     rng = np.random.default_rng(n)
@@ -183,21 +220,33 @@ def test_tile_edges(n):
     net = LearnedCorrection(seed=3)
     net.set_params(th)
     net.set_graph(*_graph(m))
+
+    def check(label, r, et, without=None):
+        _, Lr, gr, amp = _rounded(thq, G, r, et)
+        L = net.loss_grad(_dev(r, torch.float64)) if et is None else \
+            net.loss_grad_pair(_dev(r, torch.float64), _dev(et, torch.float64))
+        ge = _worst_block(net.grad(reset=True).astype(np.float64), gr)
+        print("n", n, label, "loss", abs(L - Lr) / Lr, "grad", ge, "amp", amp, flush=True)
+        assert abs(L - Lr) < 2 * 2.0 ** -8 * amp * Lr
+        assert ge < 2.0 ** -7 * amp
+        if without is not None:
+            assert _worst_block(_rounded(thq, G, r, et, without)[2], gr) > 8 * 2.0 ** -7 * amp
+
     r, et = rng.normal(size=G.n), rng.normal(size=G.n)
     out = torch.zeros(G.n, dtype=torch.float64, device="cuda:0")
     net.forward(_dev(r, torch.float64), out)
-    tol = 2.0 ** -8
-    for pair in (None, et):
-        e, Lr, gr, amp = _rounded(thq, G, r, pair)
-        err = np.linalg.norm(out.cpu().numpy() - e) / np.linalg.norm(e)
-        L = net.loss_grad(_dev(r, torch.float64)) if pair is None else \
-            net.loss_grad_pair(_dev(r, torch.float64), _dev(et, torch.float64))
-        g = net.grad(reset=True).astype(np.float64)
-        ge = np.linalg.norm(g - gr) / np.linalg.norm(gr)
-        print("n", n, "e", err, "loss", abs(L - Lr) / Lr, "grad", ge, "amp", amp, flush=True)
-        assert err < tol
-        assert abs(L - Lr) < 2 * tol * amp * Lr
-        assert ge < 2 * tol * amp
+    e = _rounded(thq, G, r, None)[0]
+    rms = np.sqrt(np.mean(e * e))
+    d = np.abs(out.cpu().numpy() - e) / rms
+    print("n", n, "e: largest", d.max(), "share over 1e-4", (d > 1e-4).mean(), flush=True)
+    assert (d > 1e-4).sum() <= max(4, 0.02 * n) and d.max() < 2.0 ** -5
+    check("all", r, None)
+    check("all, pair", r, et)
+    for name, nodes in _edge_nodes(n).items():
+        big = np.zeros(n)
+        big[nodes] = rng.choice([-1.0, 1.0], len(nodes)) * rng.uniform(0.5, 1.0, len(nodes)) * np.sqrt(n)
+        check(name, 1e-2 * r + big, None, nodes)
+        check(name + ", pair", r, e + (100 * rms) * big, nodes)
 
 
 def test_training_lowers_the_loss():
