@@ -21,6 +21,8 @@
 
 namespace fvm {
 
+constexpr int TAIL_ROWS_CAP = 16384;   // largest level that the packed tail may hold
+
 struct Level {
     int n = 0;
     long long nnz = 0;
@@ -39,7 +41,7 @@ struct Level {
     // exact Gauss-Seidel schedule (device level pointers; host knows the count)
     bool sched_ready = false;
     DArr<int> fwd_ptr, fwd_rows, bwd_ptr, bwd_rows;
-    int fwd_nlev = 0, bwd_nlev = 0, fwd_maxw = 0, bwd_maxw = 0;
+    int sched_nlev = 0, sched_maxw = 0;   // of both directions: the backward schedule is the forward one reversed
     std::vector<int> h_fwd_ptr, h_bwd_ptr;
     // launch plan of a sweep: maximal runs of consecutive dependency levels of at most
     // exact_wg_width rows share one single-workgroup launch, wider levels get a launch
@@ -159,9 +161,11 @@ struct fvm_amg {
     fvm::DArr<double> dense_inv;
     // tuning knobs (fvm_amg_set_tuning): rows below which a level runs in the
     // single-workgroup tail of the V-cycle / is coarsened by one workgroup
-    // one workgroup beats the launches of a level up to here (ms per solve at 1,500 / 6,000 / 12,000 rows:
+    // the packed form beats the launches of a level up to here (ms per solve at 1,500 / 6,000 / 12,000 rows:
     // 402k rows FP64 40.6 / 37.0 / 38.0, 8M rows mixed 239.7 / 237.1 / 233.3, 32 systems of ~30k rows
-    // 116.2 / 110.5 / 129.7)
+    // 116.2 / 110.5 / 129.7). The general form (Jacobi, pre-sweeps) pays up to about 1,000 rows at most, ms
+    // per cycle at 6,000 / 1,000 / 0, 216,000 rows: Jacobi FP64 0.351 / 0.237 / 0.255, mixed 0.356 / 0.234
+    // / 0.198; one pre-sweep FP64 1.593 / 1.522 / 1.918, mixed 1.616 / 1.383 / 1.456
     long long tail_max_rows = 6000;
     int exact_wg_width = 256;          // runs of consecutive dependency levels of at most this many rows
                                        // sweep in one workgroup launch (no result changes)

@@ -321,8 +321,10 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // A reference-order sweep (both directions) of a level by one workgroup. Spread over the
 // chip (k_csr_gs_flow) a hop from one dependency level to the next costs 2 to 6 us: the
 // new value goes through the memory side of the caches. Inside one workgroup it goes
-// through LDS: 0.35 us a hop for rows of 4 entries, 0.6 us for 10. Items of up to 64 rows of one dependency level are
-// taken by the wavefronts in turn; a wavefront loads its item's rows, entries and old
+// through LDS: 0.36 us a hop for rows of 2 entries, 0.5 for 6, 1.1 for 23. That is not the LDS's
+// latency (65 clocks) but what lies between two items in a row: poll, the operands' LDS reads,
+// the whole sum, an FP64 division, store and count. Items of up to 64 rows of one dependency level
+// are taken by the wavefronts in turn; a wavefront loads its item's rows, entries and old
 // values while the items before it are still running, then waits (an LDS counter of
 // finished items) until every item of the earlier dependency levels is done. Item i waits
 // only for items below it, so every wait ends (and one that sees no item finish for two seconds
@@ -333,10 +335,12 @@ k_csr_gs_flow(int n, int dir, const int *__restrict__ rows, const int *__restric
 // The price is one CU's throughput (about 20 GB/s of what its L2 does not hold), so b and
 // x are first brought into the order of the schedule: rows of one dependency level side
 // by side, sorted, their neighbours nearly so (44k rows: 510 -> 320 us a sweep). An item
-// takes 0.2 us, a hop across the chip about 2.9 us: past FL_ITEMS items per dependency level, and past
-// exact_flow_wg_rows (150,000) rows, whose entries come from HBM, the whole chip is faster (210,000 rows, 7 items per level: 1.3 ms slower
-// per sweep here). Milliseconds per V-cycle against chip-wide sweeps on every level:
-// 27,000 rows 1.31 / 5.08, 125,000 rows 3.7 / 11.1, 729,000 rows 15.6 / 26.2.
+// takes 0.2 us, and that bounds levels with several (64,000 7-point rows, 9 items per dependency
+// level: 446 us for 2,100 items, 118 us of hops); a hop across the chip takes about 2.9 us: past
+// FL_ITEMS items per dependency level, and past exact_flow_wg_rows (150,000) rows, whose entries
+// come from HBM, the whole chip is faster (210,000 rows, 7 items per level: 1.3 ms slower per
+// sweep here). Milliseconds per V-cycle against chip-wide sweeps on every level: 27,000 rows
+// 1.31 / 5.08, 125,000 rows 3.7 / 11.1, 729,000 rows 15.6 / 26.2.
 // One schedule serves both directions: its reverse is a valid order of the backward sweep.
 // Arithmetic and order per row: those of k_csr_gs_flow.
 // Shapes by the level's longest row: two, four or six groups of four entries loaded ahead
@@ -368,7 +372,8 @@ constexpr int FL_NEW = (int)0x80000000, FL_FAR = 0x40000000, FL_IDX = 0x3fffffff
 template <class V, class X, bool FILL>
 __global__ void __launch_bounds__(64)
 k_flow_pack(int n, int dir, int4 *items, const int *lvl_end, const int *rows, const int *place, const int *row,
-            const int *col, const V *off, const X *diag, unsigned long long *total, int4 *code, X *val, X *dg) {   // total: groups, longest item
+            const int *col, const V *off, const X *diag, unsigned long long *total, int4 *code, X *val, X *dg) {
+    // total: groups, longest item
     constexpr int R = fl_ring<X>();
     int4 t = items[blockIdx.x];
     const int np = t.y & 0xff, lane = threadIdx.x;
@@ -1109,7 +1114,6 @@ k_tail(const TailLv *lv, int l0, int last, int npre, int npost, int jacobi, cons
 // 400 us. A step of a resident level costs 0.4 to 0.8 us, about 130 to 250 instructions
 // of one wavefront plus five LDS round trips.
 constexpr int TAIL_NT = 512;                // eight wavefronts (a barrier of 4 / 8 / 16 costs 11 / 87 / 336 clocks)
-constexpr int TAIL_ROWS_CAP = 16384;        // largest level packed
 constexpr int TAIL_RES_BYTES = 104 * 1024;  // LDS of the item tables and the resident levels
 constexpr int TAIL_Q = 4;                   // groups of four entries loaded ahead
 
@@ -1707,8 +1711,8 @@ void gs_sweep(Run &R, int l, X *x, const X *b) {
         }
     } else {
         if (L.runs_width != R.h->exact_wg_width) {
-            sweep_runs(L.h_fwd_ptr, L.fwd_nlev, R.h->exact_wg_width, L.fwd_runs);
-            sweep_runs(L.h_bwd_ptr, L.bwd_nlev, R.h->exact_wg_width, L.bwd_runs);
+            sweep_runs(L.h_fwd_ptr, L.sched_nlev, R.h->exact_wg_width, L.fwd_runs);
+            sweep_runs(L.h_bwd_ptr, L.sched_nlev, R.h->exact_wg_width, L.bwd_runs);
             L.runs_width = R.h->exact_wg_width;
         }
         for (int dir = 0; dir < 2; dir++) {
@@ -2135,10 +2139,10 @@ void prepare_flow_packs(Run &R) {
         for (Level::FlowPack &P : L.flow) P = Level::FlowPack{};
         L.flow_vec.release();
         // a value leaves the ring well after it was stored: more items later than there are wavefronts
-        if (L.n == 0 || L.n > h->flow_wg_rows || std::max(L.fwd_maxw, L.bwd_maxw) + 64 * (FL_NW + 1) > RING) continue;
+        if (L.n == 0 || L.n > h->flow_wg_rows || L.sched_maxw + 64 * (FL_NW + 1) > RING) continue;
         long long nitem = 0;
-        for (int k = 0; k < L.fwd_nlev; k++) nitem += (L.h_fwd_ptr[k + 1] - L.h_fwd_ptr[k] + 63) / 64;
-        if (nitem > (long long)FL_ITEMS * L.fwd_nlev) continue;
+        for (int k = 0; k < L.sched_nlev; k++) nitem += (L.h_fwd_ptr[k + 1] - L.h_fwd_ptr[k] + 63) / 64;
+        if (nitem > (long long)FL_ITEMS * L.sched_nlev) continue;
         for (int dir = 0; dir < 2; dir++) {
             jobs.emplace_back();
             Job &J = jobs.back();

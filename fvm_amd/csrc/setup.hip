@@ -1252,34 +1252,33 @@ __global__ void k_gal_compact(int nc, const int *toff, const int *crow, const in
 // higher index; reverse sweep (dir 1): from higher to lower. With a
 // non-symmetric pattern both row and rowT are walked (an edge present in both
 // is counted twice on both sides, which keeps the in-degree bookkeeping exact).
-__global__ void k_sched_init(int n, int dir, const int *row, const int *col, const int *rowT,
-                             const int *colT, int *indeg, int *rows, int *tail) {
+__global__ void k_sched_init(int n, const int *row, const int *col, const int *rowT, const int *colT,
+                             int *indeg, int *rows, int *tail) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         int k = 0;
-        for (int p = row[i]; p < row[i + 1]; p++) k += dir ? (col[p] > i) : (col[p] < i);
+        for (int p = row[i]; p < row[i + 1]; p++) k += col[p] < i;
         if (rowT)
-            for (int p = rowT[i]; p < rowT[i + 1]; p++) k += dir ? (colT[p] > i) : (colT[p] < i);
+            for (int p = rowT[i]; p < rowT[i + 1]; p++) k += colT[p] < i;
         indeg[i] = k;
         if (k == 0) rows[atomicAdd(tail, 1)] = i;
     }
 }
 
-__global__ void k_sched_round(int lvl, int dir, const int *row, const int *col, const int *rowT,
-                              const int *colT, int *indeg, int *rows, int *ptr, int *tail,
-                              unsigned *done_blocks) {
+__global__ void k_sched_round(int lvl, const int *row, const int *col, const int *rowT, const int *colT,
+                              int *indeg, int *rows, int *ptr, int *tail, unsigned *done_blocks) {
     const int b = ptr[lvl], e = ptr[lvl + 1];
     for (int idx = b + blockIdx.x * blockDim.x + threadIdx.x; idx < e;
          idx += gridDim.x * blockDim.x) {
         const int i = rows[idx];
         for (int p = row[i]; p < row[i + 1]; p++) {
             const int c = col[p];
-            if (dir ? (c < i) : (c > i))
+            if (c > i)
                 if (atomicSub(&indeg[c], 1) == 1) rows[atomicAdd(tail, 1)] = c;
         }
         if (rowT)
             for (int p = rowT[i]; p < rowT[i + 1]; p++) {
                 const int c = colT[p];
-                if (dir ? (c < i) : (c > i))
+                if (c > i)
                     if (atomicSub(&indeg[c], 1) == 1) rows[atomicAdd(tail, 1)] = c;
             }
     }
@@ -2300,7 +2299,7 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
         unsigned *done_blocks = (unsigned *)(ctr.p + 1);
         const int *rT = L.sym ? nullptr : L.rowT.p;
         const int *cT = L.sym ? nullptr : L.colT.p;
-        k_sched_init<<<grid_for(n, BS, 4096), BS, 0, s>>>(n, 0, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, tail);
+        k_sched_init<<<grid_for(n, BS, 4096), BS, 0, s>>>(n, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, tail);
         k_set_ptr01<<<1, 1, 0, s>>>(ptr.p, tail);
         FVM_HIP(hipGetLastError());
         int lvl = 0;
@@ -2308,8 +2307,7 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
         for (;;) {
             for (int k = 0; k < batch; k++, lvl++) {
                 FVM_CHECK((size_t)lvl + 2 < ptr.n, FVM_E_NUMERIC, "GS schedule overflow");
-                k_sched_round<<<g, BS, 0, s>>>(lvl, 0, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, ptr.p, tail,
-                                               done_blocks);
+                k_sched_round<<<g, BS, 0, s>>>(lvl, L.row.p, L.col.p, rT, cT, indeg.p, rows.p, ptr.p, tail, done_blocks);
             }
             FVM_HIP(hipGetLastError());
             if (read_scalar(tail, s) >= n) break;
@@ -2327,8 +2325,8 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
         int nl = 0, maxw = 0;
         while (nl + 1 < (int)hp.size() && hp[nl] < n) { maxw = std::max(maxw, hp[nl + 1] - hp[nl]); nl++; }
         hp.resize(nl + 1);
-        L.fwd_nlev = L.bwd_nlev = nl;
-        L.fwd_maxw = L.bwd_maxw = maxw;
+        L.sched_nlev = nl;
+        L.sched_maxw = maxw;
         // rows ascending inside each dependency level (the rounds append them in any order)
         DArr<int> key(n), key_out(n), idx(n);
         L.fwd_rows.alloc(n);
@@ -2345,7 +2343,7 @@ void prepare_exact_schedule(fvm_amg *h, Level &L) {
     // backward: the same schedule from its end. A row reads new values of linked rows of
     // higher index, all of them in later forward levels.
     {
-        const int nl = L.fwd_nlev;
+        const int nl = L.sched_nlev;
         L.h_bwd_ptr.resize(nl + 1);
         for (int k = 0; k <= nl; k++) L.h_bwd_ptr[k] = n - hp[nl - k];
         L.bwd_rows.alloc(n);
@@ -2478,7 +2476,7 @@ void prepare_fast_level(fvm_amg *h, Level &L, int l, hipStream_t s, Workspace &w
     L.sell_off.alloc((size_t)nslice + 1);
     ws.scan.exclusive(w64.p, L.sell_off.p, nslice + 1, s);
     int total;
-    if (n <= 16384) {   // levels that the single-workgroup tail may pack: it needs every slice's width
+    if (n <= TAIL_ROWS_CAP) {   // levels that the single-workgroup tail may pack: it needs every slice's width
         L.h_sell_off.resize((size_t)nslice + 1);
         FVM_HIP(hipMemcpyAsync(L.h_sell_off.data(), L.sell_off.p, L.sell_off.bytes(), hipMemcpyDeviceToHost, s));
         FVM_HIP(hipStreamSynchronize(s));
