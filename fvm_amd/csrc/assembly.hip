@@ -521,9 +521,10 @@ __global__ void k_grad_ghost(int n_cells, int nct, const int *cf_row, const int 
 // both of its rows, from the same operands in the same order: that costs four divisions per
 // entry and saves the face arrays and the passes that clear rows and look for boundary faces.
 // Values are kept by component and not by cell or face: with 24 bytes between lanes each
-// load touched three times as many cache lines, and the address unit was busy 3/4 of the time.
+// load touched three times as many cache lines.
 // A block's coefficients go through LDS, for whole lines (by row they were written 3.2 times
-// over). Bound by its loads, 80 bytes per entry, 48 of them gathered. 1,397,760
+// over). Bound by its loads, 80 bytes per entry, 48 of them gathered (the address units are
+// busy 0.7 of the time, 0.64 GB from and to memory). 1,397,760
 // cells: 114 us, 236 us with values by cell and face; bcells 24, ghosts 4 us (six passes, 375 us, before).
 struct Thermal {
     int n_cells, nct, nf, central;
@@ -1042,7 +1043,8 @@ struct Dev {
 //    (a copy each was 73 MB and 310 us at 1,397,760 cells);
 //  - at most one spare block each for a system's values and for an assembly's scratch, so that
 //    a loop that assembles and drops systems does not map and unmap memory every time
-//    (932 -> 232 us per assembly there, copies included; 75 -> 65 us at 9,450 cells).
+//    (932 -> 232 us per assembly there, copies included; 75 -> 65 us at 9,450 cells). Kept until
+//    the mesh and its last system are gone: together as much as one more system and its scratch.
 // A system's block comes back only when the device has finished with it, as with hipFree;
 // scratch is used on the mesh's stream alone. Both from any thread.
 struct MeshStore {

@@ -241,7 +241,7 @@ struct MpTiles {
 // wavefronts per SIMD. LAST: the readout e = s (wo . h' + bo) is taken from the registers;
 // h' is stored only for a backward pass. What bounds it: the gathers, 128 bytes per entry.
 // 763,560 nodes (7-point rows): layer 64 -> 64 165 -> 129 us, the last one with its readout
-// 260 -> 120 us (146 and 110 MB from memory, 10 and 7 million L2 accesses), layer 0 68 -> 35 us
+// 260 -> 120 us (296 and 218 MB from memory, 10 and 7 million L2 accesses), layer 0 68 -> 35 us
 // (and k_mp_a0 17 us).
 // Weights in registers over several tiles: 142 us (3 wavefronts per SIMD). Stores and
 // column reads that bypass the caches, or 96 blocks instead of 192 per XCD: slower.
