@@ -457,6 +457,12 @@ int fvm_mesh_create(fvm_mesh **out, int device, int n_nodes, const double *nodes
 int fvm_mesh_create_general(fvm_mesh **out, int device, int dim, int n_nodes, const double *nodes, int n_faces,
                             const int32_t *face_nptr, const int32_t *face_nodes, const int32_t *face_cells,
                             int n_cells, int n_ghost, int n_groups, const int32_t *group_ptr);
+/* A mesh keeps what its assemblies share on the device: the sparsity pattern of
+ * its systems, and from the first thermal assembly or gradient on row slices with
+ * gradient coefficients (32 bytes per matrix entry) and face geometry (32 bytes
+ * per face). A dropped system's values and an assembly's scratch stay as one
+ * spare block each for the next ones. All of it is freed with the mesh and the
+ * last of its systems. */
 int fvm_mesh_destroy(fvm_mesh *m);
 /* dimension, total face-node count and (may be NULL) a host copy of face_nptr */
 int fvm_mesh_topology(const fvm_mesh *m, int *dim, long long *n_face_nodes, int32_t *face_nptr);
@@ -498,10 +504,10 @@ int fvm_convdiff_assemble(fvm_mesh *m, const double *d_k, const double *d_source
  * memory (code under HIP graph capture, tight time-stepping or serving loops).
  * fvm_convdiff_assemble's linearization (same kernels, same results) into an
  * existing system S that fvm_convdiff_assemble / fvm_thermal_assemble built from
- * this mesh, with no allocation: its scratch (per-face coefficients and fluxes,
- * cell gradients) is a per-device static array of 4,194,304 doubles (32 MiB, held
- * until the process ends), so 2 n_faces + 3 (n_cells + n_ghost) must not exceed
- * that (FVM_E_INVALID otherwise), and the mesh must have been assembled once
+ * this mesh, with no allocation: its scratch (the cell gradients) lies in a
+ * per-device static array of 4,194,304 doubles (32 MiB, held until the process
+ * ends), and 2 n_faces + 3 (n_cells + n_ghost) must not exceed
+ * that (FVM_E_INVALID otherwise); the mesh must have been assembled once
  * (its metrics and gradient coefficients exist). Every call on a device shares
  * that device's scratch: calls that overlap on one device (other threads) race. */
 int fvm_convdiff_reassemble_noalloc(fvm_mesh *m, const double *d_k, const double *d_source, const double *d_x,
